@@ -256,85 +256,128 @@ __device__ __forceinline__ double hat_w(int span, int ly, int lx, int lz, int a,
   return wy * wx * wz;
 }
 
-// Accumulates R += Q^T Kc Q for one child held in shK (24x24 full, row-major)
-// using the Kronecker structure Q = N (x) I3.
-__device__ __forceinline__ void galerkin_child(int span, int ly, int lx, int lz, const double (*shK)[24],
-                                               double (*shT)[24], double* acc, int nThreads) {
-  // shT[a'][(3J+c')] = sum_b K[a'][3b+c'] N[b][J]
-  for (int t = threadIdx.x; t < 576; t += nThreads) {
-    const int row = t / 24, col = t % 24, J = col / 3, cp = col % 3;
-    double s = 0.0;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) s += shK[row][3 * b + cp] * hat_w(span, ly, lx, lz, b, J);
-    shT[row][col] = s;
-  }
-  __syncthreads();
-  int i = 0;
-  for (int t = threadIdx.x; t < kTri; t += nThreads, ++i) {
-    int q = 0;
-    while ((q + 1) * (q + 2) / 2 <= t) ++q;
-    const int p = t - q * (q + 1) / 2;  // p <= q
-    const int I = p / 3, c = p % 3;
-    double s = 0.0;
-#pragma unroll
-    for (int a = 0; a < 8; ++a) s += hat_w(span, ly, lx, lz, a, I) * shT[3 * a + c][q];
-    acc[i] += s;
-  }
-  __syncthreads();
-}
-
 // Level 2 cells with a child that touches a fixed node (961-971): children get
-// E * P_free Ke P_free + diag(1/nAdj) on their fixed DOFs.
-__global__ __launch_bounds__(kBlock) void k_galerkin_l2_bc(Geo gf, Geo gc, int span, const int* __restrict__ bcCells,
-                                                           const double* __restrict__ Ke, const double* __restrict__ E,
-                                                           const uint8_t* __restrict__ emaskF,
-                                                           const uint8_t* __restrict__ fix, double* __restrict__ Ks) {
-  __shared__ double shK[24][24];
-  __shared__ double shT[24][24];
-  __shared__ uint8_t shF[24];
-  __shared__ double shAdj[8];
+// E * P_free Ke P_free + diag(1/nAdj) on their fixed DOFs, then R += Q^T Kc Q
+// with the Kronecker structure Q = N (x) I3.  One work-group per cell takes
+// kBcKids children at a time, 72 threads each: thread (row, c') forms the 8
+// entries T[row][3J + c'] = sum_b Kc[row][3b + c'] N[b][J], thread (q, c) the 8
+// entries sum_a N[a][I] T[3a + c][q], from 8 values and with the hat weights in
+// registers; then the children's entries are added in the
+// children's order.  The cell's moduli, masks, node fixations and adjacency
+// counts are staged once, in one memory round trip.
+// Bound: a cell's latency chain (38 us: staging, then 8 rounds of 8 children).
+// 277 -> 38 us at 50x100x50 (225 cells), 1.00 -> 0.58 ms at 256x512x256 (4,225
+// cells, one group per CU by its 126 VGPRs; bounded to two it spills, 0.78 ms)
+// against the whole group on one child at a time, one entry per thread and
+// its loads behind four barriers.
+constexpr int kBcKids = 8;
+constexpr int kBcThreads = 72 * kBcKids;
+__global__ __launch_bounds__(kBcThreads) void k_galerkin_l2_bc(Geo gf, Geo gc, int span,
+                                                               const int* __restrict__ bcCells,
+                                                               const double* __restrict__ Ke,
+                                                               const double* __restrict__ E,
+                                                               const uint8_t* __restrict__ emaskF,
+                                                               const uint8_t* __restrict__ fix,
+                                                               double* __restrict__ Ks) {
+  __shared__ double shS[kBcKids][24][25];  // the children's entries [q][p]
+  __shared__ double shT[kBcKids][24][25];
+  __shared__ double shE[64];
+  __shared__ uint8_t shM[64];
+  __shared__ uint8_t shFix[125];
+  __shared__ double shAdj[125];
+  const int tid = threadIdx.x;
   const long long cc = bcCells[blockIdx.x];
   int cy, cx, cz;
   node_yxz(cc, gc, cy, cx, cz);
-  double acc[2] = {0.0, 0.0};
-  const int s3 = span * span * span;
-  for (int ss = 0; ss < s3; ++ss) {
-    const int ly = ss % span, lx = (ss / span) % span, lz = ss / (span * span);
-    const int fy = span * cy + ly, fx = span * cx + lx, fz = span * cz + lz;
-    const long long fe = nidx(gf, fy, fx, fz);
-    const double Ee = E[fe];
-    if (!emaskF[fe]) continue;  // void child contributes nothing
-    if (threadIdx.x < 8) {
-      const int j = threadIdx.x;
-      const int ny_ = fy + kLocDy[j], nx_ = fx + kLocDx[j], nz_ = fz + kLocDz[j];
-      const uint8_t f = fix[nidx(gf, ny_, nx_, nz_)];
-      for (int k = 0; k < 3; ++k) shF[3 * j + k] = (f >> k) & 1;
-      int cnt = 0;
-      for (int c = 0; c < 8; ++c) {
-        const int qy = ny_ - (c & 1), qx = nx_ - ((c >> 1) & 1), qz = nz_ - (c >> 2);
-        if (cell_in(gf, qy, qx, qz) && emaskF[nidx(gf, qy, qx, qz)]) ++cnt;
-      }
-      shAdj[j] = (double)cnt;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < 576; t += kBlock) {
-      const int p = t / 24, q = t % 24;
-      double v = (shF[p] || shF[q]) ? 0.0 : Ke[p * 24 + q] * Ee;
-      if (p == q && shF[p]) v = v + 1.0 / shAdj[p / 3];
-      shK[p][q] = v;
-    }
-    __syncthreads();
-    galerkin_child(span, ly, lx, lz, shK, shT, acc, kBlock);
+  const int s3 = span * span * span, sn = span + 1;
+  const int kid = tid / 72, e = tid % 72, row = e / 3, cp = e % 3;
+  double ke[8];  // this thread's row entries of Ke
+#pragma unroll
+  for (int b = 0; b < 8; ++b) ke[b] = Ke[row * 24 + 3 * b + cp];
+  if (tid < s3) {
+    const long long fe = nidx(gf, span * cy + tid % span, span * cx + (tid / span) % span, span * cz + tid / (span * span));
+    shE[tid] = E[fe];
+    shM[tid] = emaskF[fe];
   }
-  int i = 0;
-  for (int t = threadIdx.x; t < kTri; t += kBlock, ++i) Ks[(size_t)t * gc.NN + cc] = acc[i];
+  if (tid < sn * sn * sn) {
+    const int ny_ = span * cy + tid % sn, nx_ = span * cx + (tid / sn) % sn, nz_ = span * cz + tid / (sn * sn);
+    shFix[tid] = fix[nidx(gf, ny_, nx_, nz_)];
+    int cnt = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int qy = ny_ - (c & 1), qx = nx_ - ((c >> 1) & 1), qz = nz_ - (c >> 2);
+      if (cell_in(gf, qy, qx, qz) && emaskF[nidx(gf, qy, qx, qz)]) ++cnt;
+    }
+    shAdj[tid] = (double)cnt;
+  }
+  __syncthreads();
+  // entry tid of the upper triangle, t = tri_index(tp, tq)
+  int tq = (int)((sqrtf(8.f * tid + 1.f) - 1.f) * 0.5f);
+  tq += (tq + 1) * (tq + 2) / 2 <= tid;
+  tq -= tq * (tq + 1) / 2 > tid;
+  const int tp = tid - tq * (tq + 1) / 2;
+  double acc = 0.0;
+  const double inv = 1.0 / span;
+  for (int s0 = 0; s0 < s3; s0 += kBcKids) {  // span^3 is a multiple of kBcKids
+    const int ss = s0 + kid;
+    const bool on = shM[ss];  // a void child contributes nothing
+    const int ly = ss % span, lx = (ss / span) % span, lz = ss / (span * span);
+    // hat weights per axis, [child node offset][coarse node offset]
+    double wy[2][2], wx[2][2], wz[2][2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      wy[d][1] = (ly + d) * inv, wy[d][0] = (span - (ly + d)) * inv;
+      wx[d][1] = (lx + d) * inv, wx[d][0] = (span - (lx + d)) * inv;
+      wz[d][1] = (lz + d) * inv, wz[d][0] = (span - (lz + d)) * inv;
+    }
+    auto N = [&](int a, int J) {
+      return wy[kLocDy[a]][kLocDy[J]] * wx[kLocDx[a]][kLocDx[J]] * wz[kLocDz[a]][kLocDz[J]];
+    };
+    if (on) {
+      auto node = [&](int j) { return ly + kLocDy[j] + sn * (lx + kLocDx[j] + sn * (lz + kLocDz[j])); };
+      // thread (row, cp): Kc's entries (row, 3b + cp) and from them its 8 entries of T
+      const int nr = node(row / 3), cr = row % 3;
+      const bool fr = (shFix[nr] >> cr) & 1;
+      double s[8] = {};
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const bool fq = (shFix[node(b)] >> cp) & 1;
+        double v = (fr || fq) ? 0.0 : ke[b] * shE[ss];
+        if (row == 3 * b + cp && fr) v = v + 1.0 / shAdj[nr];
+#pragma unroll
+        for (int J = 0; J < 8; ++J) s[J] += v * N(b, J);
+      }
+#pragma unroll
+      for (int J = 0; J < 8; ++J) shT[kid][row][3 * J + cp] = s[J];
+    }
+    __syncthreads();
+    if (on) {  // thread (q = row, c = cp): the entries (3I + c, q)
+      double s[8] = {};
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        const double t = shT[kid][3 * a + cp][row];
+#pragma unroll
+        for (int I = 0; I < 8; ++I) s[I] += N(a, I) * t;
+      }
+#pragma unroll
+      for (int I = 0; I < 8; ++I) shS[kid][row][3 * I + cp] = s[I];
+    }
+    __syncthreads();
+    if (tid < kTri) {
+#pragma unroll
+      for (int k = 0; k < kBcKids; ++k)
+        if (shM[s0 + k]) acc += shS[k][tq][tp];
+    }
+    __syncthreads();
+  }
+  if (tid < kTri) Ks[(size_t)tid * gc.NN + cc] = acc;
 }
 
 void launch_galerkin_l2_bc(hipStream_t s, const Geo& gf, const Geo& gc, int span, int nBc, const int* bcCells,
                            const double* Ke, const double* E, const uint8_t* emaskF, const uint8_t* fix,
                            double* Ks) {
   if (nBc <= 0) return;
-  hipLaunchKernelGGL(k_galerkin_l2_bc, dim3(nBc), dim3(kBlock), 0, s, gf, gc, span, bcCells, Ke, E, emaskF, fix, Ks);
+  hipLaunchKernelGGL(k_galerkin_l2_bc, dim3(nBc), dim3(kBcThreads), 0, s, gf, gc, span, bcCells, Ke, E, emaskF, fix, Ks);
 }
 
 // Level >= 3 (span 2): Ks_c = sum over 8 children of Q^T Ks_child Q (980-995).
@@ -450,39 +493,59 @@ void launch_coarse_scatter(hipStream_t s, int n, const long long* map, const dou
   hipLaunchKernelGGL(k_coarse_scatter<float>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, map, v, x, fl);
 }
 
-// Node-centric assembly of the lower band: the thread of coarsest node n owns
-// rows 3*pos(n)+c, so no two threads write the same entry.
-__global__ void k_band_assemble(Geo g, const double* __restrict__ Ks, const uint8_t* __restrict__ emask,
-                                const int* __restrict__ nodePos, int bw, double* __restrict__ band) {
-  const long long n = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (n >= g.NN) return;
-  const int pn = nodePos[n];
-  if (pn < 0) return;
-  const int W = bw + 1;
+// Assembly of the lower band: one thread per (coarsest node a, node b of its
+// 3x3x3 neighbourhood) sums the 3x3 entries of rows a, columns b over the
+// cells that hold both, in the cells' order, and writes them once.  Bound: one
+// memory round trip per shared cell.  (One thread per node adding its 8 cells'
+// 576 products into the band one after the other: 105 -> 8 us at 12x24x12, 250
+// -> 19 us at 128x256x128.)
+__global__ __launch_bounds__(kBlock) void k_band_assemble(Geo g, const double* __restrict__ Ks,
+                                                          const uint8_t* __restrict__ emask,
+                                                          const int* __restrict__ nodePos, int bw,
+                                                          double* __restrict__ band) {
+  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (t >= 27 * g.NN) return;
+  const int o = (int)(t / g.NN);  // the neighbours of one offset adjacent: coalesced Ks reads
+  const long long n = t - o * g.NN;
+  const int pa = nodePos[n];
+  if (pa < 0) return;
   int iy, ix, iz;
   node_yxz(n, g, iy, ix, iz);
+  const int by = iy + o % 3 - 1, bx = ix + (o / 3) % 3 - 1, bz = iz + o / 9 - 1;
+  if (by < 0 || bx < 0 || bz < 0 || by >= g.NY || bx >= g.NX || bz >= g.NZ) return;
+  const int pb = nodePos[nidx(g, by, bx, bz)];
+  if (pb < 0 || pb > pa) return;  // lower triangle
+  double acc[3][3] = {};
+  bool any = false;
+#pragma unroll
   for (int c = 0; c < 8; ++c) {
-    const int dy = c & 1, dx = (c >> 1) & 1, dz = c >> 2;
-    const int cy = iy - dy, cx = ix - dx, cz = iz - dz;
+    const int cy = iy - (c & 1), cx = ix - ((c >> 1) & 1), cz = iz - (c >> 2);
+    const int dy = by - cy, dx = bx - cx, dz = bz - cz;
+    if ((unsigned)dy > 1u || (unsigned)dx > 1u || (unsigned)dz > 1u) continue;  // b is no corner of this cell
     if (!cell_in(g, cy, cx, cz)) continue;
     const long long ce = nidx(g, cy, cx, cz);
     if (!emask[ce]) continue;
-    const int jn = loc_index(dy, dx, dz);
-    for (int b = 0; b < 8; ++b) {
-      const int pb = nodePos[nidx(g, cy + kLocDy[b], cx + kLocDx[b], cz + kLocDz[b])];
-      for (int k = 0; k < 3; ++k)
-        for (int kk = 0; kk < 3; ++kk) {
-          const long long row = 3LL * pn + k, col = 3LL * pb + kk;
-          if (col > row) continue;
-          band[row * W + (row - col)] += Ks[(size_t)tri_index(3 * jn + k, 3 * b + kk) * g.NN + ce];
-        }
-    }
+    any = true;
+    const int ja = loc_index(c & 1, (c >> 1) & 1, c >> 2), jb = loc_index(dy, dx, dz);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int kk = 0; kk < 3; ++kk) acc[k][kk] += Ks[(size_t)tri_index(3 * ja + k, 3 * jb + kk) * g.NN + ce];
   }
+  if (!any) return;
+  const long long W = bw + 1;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk) {
+      const long long row = 3LL * pa + k, col = 3LL * pb + kk;
+      if (col <= row) band[row * W + (row - col)] = acc[k][kk];
+    }
 }
 void launch_band_assemble(hipStream_t s, const Geo& g, const double* Ks, const uint8_t* emask, const int* nodePos,
                           int bw, double* band, long long nBand) {
   launch_fill(s, band, 0.0, nBand);
-  hipLaunchKernelGGL(k_band_assemble, dim3(grid_for(g.NN)), dim3(kBlock), 0, s, g, Ks, emask, nodePos, bw, band);
+  hipLaunchKernelGGL(k_band_assemble, dim3(grid_for(27 * g.NN)), dim3(kBlock), 0, s, g, Ks, emask, nodePos, bw, band);
 }
 
 // Right-looking banded Cholesky in one work-group.

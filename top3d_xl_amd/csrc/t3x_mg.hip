@@ -129,7 +129,8 @@ __global__ __launch_bounds__(kBlock) void k_restrict_y_lds(Geo gf, int NYc, int 
   }
 }
 
-// x-z pass: rc[c](J) = mask(J) * sum_dz w(dz) sum_dx w(dx) tmp[c](Jy, S*Jx+dx, S*Jz+dz)
+// x-z pass: rc[c](J) = mask(J) * sum_dz w(dz) sum_dx w(dx) tmp[c](Jy, S*Jx+dx, S*Jz+dz),
+// one thread per output (many outputs: see restrict_impl)
 template <int S, typename TM, typename TO>
 __global__ __launch_bounds__(kBlock) void k_restrict_xz(Geo gf, Geo gc, const TM* __restrict__ tmp,
                                                         const uint8_t* __restrict__ nmaskC, TO* __restrict__ rc,
@@ -169,6 +170,54 @@ __global__ __launch_bounds__(kBlock) void k_restrict_xz(Geo gf, Geo gc, const TM
   rc[n] = (TO)a0;
   rc[gc.NN + n] = (TO)a1;
   rc[2 * gc.NN + n] = (TO)a2;
+}
+
+// The x-z pass with the (2S - 1) fine planes side by side: a block takes 64 outputs of one coarse plane; wave dz + S - 1 forms the x sums
+// of its fine plane (3 (2S - 1) independent loads per thread), which one wave
+// per component then adds up over z in order (the sums above, term by term).
+// Bound: load latency, a coarse grid has few outputs.
+constexpr int kXzOut = 64;
+template <int S, typename TM, typename TO>
+__global__ __launch_bounds__(kXzOut * (2 * S - 1)) void k_restrict_xz_w(Geo gf, Geo gc, const TM* __restrict__ tmp,
+                                                                      const uint8_t* __restrict__ nmaskC,
+                                                                      TO* __restrict__ rc, const int* fl) {
+  if (fl && fl[FL_DONE]) return;
+  __shared__ double sz[2 * S - 1][3][kXzOut];
+  const int planeC = gc.NY * gc.NX;
+  const int lane = threadIdx.x % kXzOut, w = threadIdx.x / kXzOut;
+  const int idx = blockIdx.x * kXzOut + lane;
+  const int Jz = blockIdx.y;
+  const long long n = idx + (long long)planeC * Jz;
+  const bool solid = idx < planeC && nmaskC[n];
+  const int plane = gc.NY * gf.NX;  // intermediate plane: NYc x NXf
+  const long long TN = (long long)plane * gf.NZ;
+  auto in_z = [&](int dz) { return S * Jz + dz >= 0 && S * Jz + dz < gf.NZ; };
+  if (solid && in_z(w - (S - 1))) {
+    const int Jx = idx / gc.NY, Jy = idx - Jx * gc.NY;
+    const long long m0 = Jy + (long long)plane * (S * Jz + w - (S - 1));
+    double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int dx = -(S - 1); dx <= S - 1; ++dx) {
+      const int x = S * Jx + dx;
+      if (x < 0 || x >= gf.NX) continue;
+      const double wx = hat_w<S>(dx);
+      const long long m = m0 + (long long)gc.NY * x;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) s[c] += wx * (double)tmp[c * TN + m];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sz[w][c][lane] = s[c];
+  }
+  __syncthreads();
+  if (w < 3 && idx < planeC) {  // 2 S - 1 >= 3 waves
+    double a = 0.0;
+    if (solid) {
+#pragma unroll
+      for (int dz = -(S - 1); dz <= S - 1; ++dz)
+        if (in_z(dz)) a += hat_w<S>(dz) * sz[dz + S - 1][w][lane];
+    }
+    rc[w * gc.NN + n] = (TO)a;
+  }
 }
 
 // out = omega*(r/d) + P xc + (omega*r)/d on solid nodes, 0 elsewhere (758,
@@ -335,6 +384,7 @@ void k_prolong_add(Geo gf, Geo gc, int zc, const TX* __restrict__ xc,
   }
 }
 
+constexpr long long kXzWideOut = 131072;     // coarse nodes up to which the x-z pass runs its planes side by side
 constexpr size_t kRestrictLds = 48 * 1024;  // LDS bytes of the y pass's rows at most
 
 template <typename TI, typename TM, typename TO>
@@ -342,7 +392,6 @@ void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const 
                    const uint8_t* nmaskC, TO* rc, const int* fl, Act actF) {
   const int plane = gc.NY * gf.NX;
   const dim3 g1((plane + kBlock - 1) / kBlock, gf.NZ);
-  const dim3 g2((gc.NY * gc.NX + kBlock - 1) / kBlock, gc.NZ);
   // the LDS y pass: about one intermediate value per thread (R rows a block)
   // while the rows fit kRestrictLds bytes
   const int R = std::max(1, (kBlock + gc.NY / 2) / gc.NY);
@@ -355,13 +404,23 @@ void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const 
       hipLaunchKernelGGL((k_restrict_y_lds<4, TI, TM>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl, actF);
     else
       hipLaunchKernelGGL((k_restrict_y<4, TI, TM>), g1, dim3(kBlock), 0, s, gf, gc.NY, rf, tmp, fl, actF);
-    hipLaunchKernelGGL((k_restrict_xz<4, TM, TO>), g2, dim3(kBlock), 0, s, gf, gc, tmp, nmaskC, rc, fl);
   } else {
     if (viaLds)
       hipLaunchKernelGGL((k_restrict_y_lds<2, TI, TM>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl, actF);
     else
       hipLaunchKernelGGL((k_restrict_y<2, TI, TM>), g1, dim3(kBlock), 0, s, gf, gc.NY, rf, tmp, fl, actF);
-    hipLaunchKernelGGL((k_restrict_xz<2, TM, TO>), g2, dim3(kBlock), 0, s, gf, gc, tmp, nmaskC, rc, fl);
+  }
+  // the x-z pass: planes side by side while one thread per output would leave
+  // the chip idle.  FP64, span 4: 18.4 -> 5.2 us at 6,075 outputs, 19.4 -> 17.3
+  // at 70,785; FP32 at 545,025 outputs 55 -> 62 us
+  if (gc.NN <= kXzWideOut) {
+    const dim3 g2((gc.NY * gc.NX + kXzOut - 1) / kXzOut, gc.NZ), b2(kXzOut * (2 * span - 1));
+    if (span == 4) hipLaunchKernelGGL((k_restrict_xz_w<4, TM, TO>), g2, b2, 0, s, gf, gc, tmp, nmaskC, rc, fl);
+    else hipLaunchKernelGGL((k_restrict_xz_w<2, TM, TO>), g2, b2, 0, s, gf, gc, tmp, nmaskC, rc, fl);
+  } else {
+    const dim3 g2((gc.NY * gc.NX + kBlock - 1) / kBlock, gc.NZ);
+    if (span == 4) hipLaunchKernelGGL((k_restrict_xz<4, TM, TO>), g2, dim3(kBlock), 0, s, gf, gc, tmp, nmaskC, rc, fl);
+    else hipLaunchKernelGGL((k_restrict_xz<2, TM, TO>), g2, dim3(kBlock), 0, s, gf, gc, tmp, nmaskC, rc, fl);
   }
 }
 
@@ -382,7 +441,11 @@ void prolong_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, double 
   int mode = 0;
   if (ws) mode = (fl && sc) ? 2 : 1;
   int zc = 0;
-  const dim3 g = prolong_grid(gf, &zc);
+  dim3 g = prolong_grid(gf, &zc);
+  if (!mode && (long long)g.x * g.y <= 512) {  // no partials to keep: a coarse grid's planes all side by side
+    zc = 1;                                    // (span 2, 14x26x14 cells: 7.5 -> 5.9 us)
+    g.y = gf.NZ;
+  }
   double* part = mode ? ws->partials : nullptr;
   if (span == 4)
     hipLaunchKernelGGL((k_prolong_jacobi<4, TX, TR, TD, TO>), g, dim3(kBlock), 0, s, gf, gc, omega, zc, xc, rf, diag,
