@@ -7,12 +7,12 @@
 
 namespace t3x {
 
-// Device words of the one-launch recurrences (k_solve_chain), zeroed at set-up:
-// per work-group the tag its next launch starts from (equal across the
-// groups between launches), and a failure word set when a wait expired
-// (cleared by the host).
-constexpr int kChainMaxSB = 2048;            // largest solve block of the one-launch recurrences
-constexpr int kChainMaxWG = kChainMaxSB / 4;  // their work-groups (one row per wave, 4 waves)
+// Device words of the one-launch recurrences (k_solve_chain, k_solve_fused),
+// zeroed at set-up: per work-group the tag its next launch starts from (equal
+// across the groups between launches), and a failure word set when a wait
+// expired (cleared by the host).
+constexpr int kChainMaxSB = 2048;             // largest solve block of the one-launch recurrences
+constexpr int kChainMaxWG = kChainMaxSB / 4;  // their work-groups at most
 struct ChainState {
   unsigned tag[kChainMaxWG];
   int fail;

@@ -20,11 +20,11 @@
 //        backward  x_b = Dinv_b^T y_b - H_b x_{b+1}, H_b = Dinv_b^T L_{b+1,b}^T
 //     Dinv_b, G_b come from one batched blocked TRSM on [I | L_{b,b-1}],
 //     H_b from a batched GEMM.
-//  3. the two recurrences as a chain of 2*nblk+1 small launches instead of
-//     one dependent step per 64 rows.
+//  3. the two recurrences in one or two launches whose work-groups hand the
+//     blocks on through tagged words, or as a chain of 2*nblk+1 small launches,
+//     instead of one dependent step per 64 rows.
 //
-// Kernel boundaries are the only cross-work-group synchronisation: on MI355X
-// a device-wide barrier inside a kernel (cooperative grid sync, or fences that
+// Everything else synchronises at kernel boundaries: on MI355X a device-wide barrier inside a kernel (cooperative grid sync, or fences that
 // write back the per-XCD L2) costs more than a dependent launch (~3 us).
 //
 // All arithmetic is FP64.  Rows beyond the true size are identity rows.
@@ -522,42 +522,82 @@ __global__ __launch_bounds__(CT) void k_h_blocks(BandView V, int SB, int nblk, c
 }
 
 // ---- 3. the solve --------------------------------------------------------
-// One wave per row dot product: out[row] = base - sum_j M[row][j] v[j].
+// One wave per row dot product: out[row] = base - sum_j M[row][j] v[j].  Products
+// are fused explicitly: the forms of the solve agree bit for bit, and where two
+// branches share a product the compiler would round it on its own.
 __device__ __forceinline__ double wave_dot(const double* __restrict__ m, const double* __restrict__ v, int len) {
   const int lane = threadIdx.x & 63;
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
   int j = lane;
   for (; j + 192 < len; j += 256) {  // four independent loads in flight per lane
-    s0 += m[j] * v[j];
-    s1 += m[j + 64] * v[j + 64];
-    s2 += m[j + 128] * v[j + 128];
-    s3 += m[j + 192] * v[j + 192];
+    s0 = fma(m[j], v[j], s0);
+    s1 = fma(m[j + 64], v[j + 64], s1);
+    s2 = fma(m[j + 128], v[j + 128], s2);
+    s3 = fma(m[j + 192], v[j + 192], s3);
   }
-  for (; j < len; j += 64) s0 += m[j] * v[j];
+  for (; j < len; j += 64) s0 = fma(m[j], v[j], s0);
   double s = (s0 + s1) + (s2 + s3);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   return s;
 }
 
-// forward phase 0: gather the permuted right-hand side and va_b = Dinv_b v_b
+// forward phase 0: gather the permuted right-hand side and va_b = Dinv_b v_b,
+// a lane's columns lane + 64 c summed in order.  A work-group takes kOwnRows
+// rows of one block, kOwnRows / 4 per wave, against the block's vector in LDS:
+// 16 loads in flight per lane, and the vector is gathered once per group.
+// HBM-bound: 110 MB at 256x512x256 in 32 us, against 42 us with a wave per row
+// that gathered its own vector.
+constexpr int kOwnRows = 16;  // divides TB, so a group's rows share a diagonal tile
+constexpr int kOwnPerWave = kOwnRows / (CT / 64);
 template <typename TR>
 __global__ __launch_bounds__(CT) void k_solve_f0(int n, int np, int SB, const long long* __restrict__ map,
                                                  const TR* __restrict__ rdense, const double* __restrict__ Dinv,
                                                  double* __restrict__ va, const int* fl) {
   if (fl && fl[FL_DONE]) return;
-  const int row = blockIdx.x * (CT / 64) + (threadIdx.x >> 6);
-  if (row >= np) return;
-  const int b = row / SB, i = row % SB, lane = threadIdx.x & 63;
-  const double* m = Dinv + (size_t)b * SB * SB + (size_t)i * SB;
-  double s = 0.0;
-  for (int j = lane; j <= i; j += 64) {
-    const int g = b * SB + j;
-    s += m[j] * (g < n ? (double)rdense[map[g]] : 0.0);
+  constexpr int SEG = 64;  // 64-column chunks of the vector in LDS at a time
+  __shared__ double sv[SEG * TB];
+  const int row0 = blockIdx.x * kOwnRows;  // SB is a multiple of kOwnRows
+  const int b = row0 / SB, i0 = row0 % SB, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = i0 + kOwnPerWave * w;  // this wave's rows i .. i + kOwnPerWave - 1
+  const double* m = Dinv + ((size_t)b * SB + i) * SB;
+  const int c1 = i0 / TB + 1;  // chunks up to the diagonal's; Dinv is 0 right of the diagonal
+  double s[kOwnPerWave] = {};
+  for (int cs = 0; cs < c1; cs += SEG) {
+    const int ce = min(c1, cs + SEG);
+    __syncthreads();
+    for (int j = cs * TB + threadIdx.x; j < ce * TB; j += CT) {
+      const int g = b * SB + j;
+      sv[j - cs * TB] = g < n ? (double)rdense[map[g]] : 0.0;
+    }
+    __syncthreads();
+    int c = cs;
+    for (; c + 4 <= ce; c += 4) {
+      double t[kOwnPerWave][4];
+#pragma unroll
+      for (int r = 0; r < kOwnPerWave; ++r)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[r][u] = m[(size_t)r * SB + lane + TB * (c + u)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double v = sv[lane + TB * (c + u - cs)];
+#pragma unroll
+        for (int r = 0; r < kOwnPerWave; ++r) s[r] = fma(t[r][u], v, s[r]);
+      }
+    }
+    for (; c < ce; ++c) {
+      const double v = sv[lane + TB * (c - cs)];
+#pragma unroll
+      for (int r = 0; r < kOwnPerWave; ++r) s[r] = fma(m[(size_t)r * SB + lane + TB * c], v, s[r]);
+    }
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if (lane == 0) va[row] = s;
+  for (int r = 0; r < kOwnPerWave; ++r) {
+    double t = s[r];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+    if (lane == 0) va[row0 + kOwnPerWave * w + r] = t;
+  }
 }
 // v[b] -= M_b v[b + d] for the SB rows of block b (d = -1 forward, +1 backward)
 __global__ __launch_bounds__(CT) void k_solve_step(int SB, int b, int d, const double* __restrict__ M,
@@ -716,14 +756,14 @@ __global__ __launch_bounds__(CT) void k_solve_chain(int n, int SB, int nblk, con
         const int j = lane + 256 * q;
         quad = quad && j + 192 < SB;
         if (quad) {
-          s0 += rg[4 * q] * chainNbr[j];
-          s1 += rg[4 * q + 1] * chainNbr[j + 64];
-          s2 += rg[4 * q + 2] * chainNbr[j + 128];
-          s3 += rg[4 * q + 3] * chainNbr[j + 192];
+          s0 = fma(rg[4 * q], chainNbr[j], s0);
+          s1 = fma(rg[4 * q + 1], chainNbr[j + 64], s1);
+          s2 = fma(rg[4 * q + 2], chainNbr[j + 128], s2);
+          s3 = fma(rg[4 * q + 3], chainNbr[j + 192], s3);
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (j + 64 * r < SB) s0 += rg[4 * q + r] * chainNbr[j + 64 * r];
+            if (j + 64 * r < SB) s0 = fma(rg[4 * q + r], chainNbr[j + 64 * r], s0);
         }
       }
       const double s = ab - chain_wave_sum((s0 + s1) + (s2 + s3));
@@ -735,19 +775,195 @@ __global__ __launch_bounds__(CT) void k_solve_chain(int n, int SB, int nblk, con
   if (!FWD && threadIdx.x == 0) st->tag[blockIdx.x] = tag0 + nblk;
 }
 
+// SB <= kFusedMaxSB: the own terms and both recurrences in one launch.  The
+// operators of a block are small there (2 MB at SB 512), so a step is its
+// hand-over whatever else it loads: own terms formed while waiting, the way
+// back's (DT y) when the block before arrives.  Against k_solve_f0, two
+// k_solve_chain and k_solve_b0 that is three launches and two passes over the
+// vectors less, with the same sums in the same order.  Words and polls as in
+// k_solve_chain, but y and x have words of their own, so a word is written
+// once per solve and one tag per solve serves every block.  Rows: one per wave;
+// NW waves per group, few, so that a block's loads spread over many CUs.
+// Bound: the hand-over, 1.9 us a step.  50x100x50 (SB 256, 11 blocks): 42 us
+// against 51 us and three launches; 2 waves per group against 4: 42.4 / 42.9
+// us, at SB 384 70 / 76 us.  Groups with waves that only poll, beside the row
+// waves, were slower (62 us; at SB 960 163 against 92 us a direction: polls
+// that do not wait for the operator rows compete with them for memory).
+constexpr int kFusedMaxSB = 512;
+struct FusedArgs {
+  int n, SB, nblk;
+  const long long* map;
+  const double *Dinv, *DT, *Gm, *H;
+  double* vb;                 // own terms of the way back
+  unsigned long long *W, *X;  // tagged y and x
+  ChainState* st;
+};
+// NCH: 64-column chunks of a row (SB <= 64 NCH), PT = NCH / NW entries polled per thread
+template <typename TV, int NW, int NCH>
+__global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* __restrict__ rdense,
+                                                         TV* __restrict__ xdense, const int* fl) {
+  if (fl && fl[FL_DONE]) return;
+  constexpr int PT = NCH / NW, NT = 64 * NW;
+  extern __shared__ double chainNbr[];  // two neighbour blocks, in turn
+  const int SB = A.SB, nblk = A.nblk;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * NW + (threadIdx.x >> 6);  // SB is a multiple of NW: row < SB
+  const unsigned tag = A.st->tag[blockIdx.x] + 1;  // one above this group's last solve
+  int step = 0;
+  // block b of Wd into the next buffer once every entry carries the tag
+  auto poll = [&](const unsigned long long* Wd, int b) -> const double* {
+    double* sY = chainNbr + (step++ & 1) * SB;
+    unsigned pending = 0;
+#pragma unroll
+    for (int k = 0; k < PT; ++k)
+      if ((int)threadIdx.x + k * NT < SB) pending |= 1u << k;
+    unsigned polls = 0;
+    while (pending) {
+      unsigned long long hi[PT], lo[PT];
+#pragma unroll
+      for (int k = 0; k < PT; ++k)
+        if (pending & (1u << k)) {
+          const int i = b * SB + threadIdx.x + k * NT;
+          hi[k] = __hip_atomic_load(Wd + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          lo[k] = __hip_atomic_load(Wd + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+      for (int k = 0; k < PT; ++k)
+        if ((pending & (1u << k)) && (unsigned)hi[k] == tag && (unsigned)lo[k] == tag) {
+          sY[threadIdx.x + k * NT] = __longlong_as_double((long long)((hi[k] & 0xFFFFFFFF00000000ull) | (lo[k] >> 32)));
+          pending &= ~(1u << k);
+        }
+      if (!pending) break;
+      bool give = __hip_atomic_load(&A.st->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+      if (!give && ++polls > kChainSpin) {
+        __hip_atomic_store(&A.st->fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        give = true;
+      }
+      if (give) {
+#pragma unroll
+        for (int k = 0; k < PT; ++k)
+          if (pending & (1u << k)) sY[threadIdx.x + k * NT] = 0.0;
+        break;
+      }
+    }
+    __syncthreads();  // (the buffer's readers of two steps ago have passed the barrier since)
+    return sY;
+  };
+  // entries e >= len repeat the last one and enter no sum
+  auto load = [&](const double* m, int len, double (&r)[NCH]) {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) r[c] = m[min(lane + 64 * c, len - 1)];
+  };
+  // wave_dot's order over a row in registers
+  auto dot = [&](const double (&r)[NCH], const double* v, int len) {
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    bool quad = true;
+#pragma unroll
+    for (int q = 0; q < NCH / 4; ++q) {
+      const int j = lane + 256 * q;
+      quad = quad && j + 192 < len;
+      if (quad) {
+        s0 = fma(r[4 * q], v[j], s0);
+        s1 = fma(r[4 * q + 1], v[j + 64], s1);
+        s2 = fma(r[4 * q + 2], v[j + 128], s2);
+        s3 = fma(r[4 * q + 3], v[j + 192], s3);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (j + 64 * u < len) s0 = fma(r[4 * q + u], v[j + 64 * u], s0);
+      }
+    }
+    return chain_wave_sum((s0 + s1) + (s2 + s3));
+  };
+  auto op_row = [&](const double* M, int b) { return M + ((size_t)b * SB + row) * SB; };
+  double rg[NCH], rt[NCH], rd[NCH], rv[NCH];  // rows of G or H, of DT from the diagonal on, of Dinv; the right-hand side
+  auto load_own = [&](int b) {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int g = b * SB + min(lane + 64 * c, SB - 1);
+      const double v = (double)rdense[A.map[min(g, A.n - 1)]];
+      rv[c] = g < A.n ? v : 0.0;
+    }
+    load(op_row(A.Dinv, b), SB, rd);
+  };
+  auto emit_x = [&](int b, double v) {
+    const int g = b * SB + row;
+    chain_put(A.X, g, v, tag);
+    if (g < A.n) xdense[A.map[g]] = (TV)v;
+  };
+  load_own(0);
+  for (int b = 0; b < nblk; ++b) {  // forwards
+    double y = 0.0;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c)  // k_solve_f0's order
+      if (lane + 64 * c <= row) y = fma(rd[c], rv[c], y);
+    y = chain_wave_sum(y);
+    const double* sY = nullptr;
+    if (b > 0) {
+      sY = poll(A.W, b - 1);
+      y -= dot(rg, sY, SB);
+    }
+    if (lane == 0) chain_put(A.W, b * SB + row, y, tag);
+    if (b + 1 < nblk) {
+      load(op_row(A.Gm, b + 1), SB, rg);
+      load_own(b + 1);
+    }
+    if (b > 0) {
+      const double t = dot(rt, sY + row, SB - row);
+      if (lane == 0) A.vb[(size_t)(b - 1) * SB + row] = t;
+    }
+    load(op_row(A.DT, b) + row, SB - row, rt);
+  }
+  {  // x of the last block is its own term
+    const double* sY = poll(A.W, nblk - 1);
+    const double x = dot(rt, sY + row, SB - row);
+    if (lane == 0) emit_x(nblk - 1, x);
+  }
+  for (int b = nblk - 2; b >= 0; --b) {  // backwards
+    load(op_row(A.H, b), SB, rg);
+    double own = 0.0;
+    if (lane == 0) own = A.vb[(size_t)b * SB + row];  // this lane's own store
+    const double* sY = poll(A.X, b + 1);
+    const double x = own - dot(rg, sY, SB);
+    if (lane == 0) emit_x(b, x);
+  }
+  if (threadIdx.x == 0) A.st->tag[blockIdx.x] = tag;
+}
+
 // ---- host side -----------------------------------------------------------
+template <typename TV>
+struct FusedForm {
+  int waves;  // per group
+  void (*fn)(FusedArgs, const TV*, TV*, const int*);
+};
+template <typename TV>
+static FusedForm<TV> fused_form(int SB) {
+  if (SB <= 256) return {2, k_solve_fused<TV, 2, 4>};
+  return {2, k_solve_fused<TV, 2, 8>};
+}
+static size_t fused_lds(int SB) { return 2 * (size_t)SB * sizeof(double); }
+
 long long CoarseSolver::chain_share() const {
   constexpr long long kNever = 2000000;
   if (SB > kChainMaxSB) return kNever;
-  const int G = (SB + 3) / 4;
-  const size_t lds = (size_t)SB * sizeof(double);
   int dev = 0, cus = 0, perCU = 0, perCU2 = 0;
   if (hipGetDevice(&dev) != hipSuccess) return kNever;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return kNever;
-  auto fwd = SB <= 4 * CT ? k_solve_chain<double, 4, true> : k_solve_chain<double, kChainMaxSB / CT, true>;
-  auto bwd = SB <= 4 * CT ? k_solve_chain<float, 4, false> : k_solve_chain<float, kChainMaxSB / CT, false>;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fwd, CT, lds) != hipSuccess) return kNever;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, bwd, CT, lds) != hipSuccess) return kNever;
+  int G = (SB + 3) / 4;
+  if (SB <= kFusedMaxSB) {
+    const FusedForm<double> fd = fused_form<double>(SB);
+    const FusedForm<float> ff = fused_form<float>(SB);
+    G = SB / fd.waves;
+    const size_t lds = fused_lds(SB);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fd.fn, 64 * fd.waves, lds) != hipSuccess) return kNever;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, ff.fn, 64 * ff.waves, lds) != hipSuccess) return kNever;
+  } else {
+    const size_t lds = (size_t)SB * sizeof(double);
+    auto fwd = SB <= 4 * CT ? k_solve_chain<double, 4, true> : k_solve_chain<double, kChainMaxSB / CT, true>;
+    auto bwd = SB <= 4 * CT ? k_solve_chain<float, 4, false> : k_solve_chain<float, kChainMaxSB / CT, false>;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fwd, CT, lds) != hipSuccess) return kNever;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, bwd, CT, lds) != hipSuccess) return kNever;
+  }
   const long long slots = (long long)std::min(perCU, perCU2) * cus;
   if (slots <= 0) return kNever;
   return (1000000LL * G + slots - 1) / slots;
@@ -795,11 +1011,19 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
                        double* vb, const int* fl) {
   const int wpb = CT / 64;
   const int n = C.n, np = C.np, SB = C.SB, nblk = C.nblk;
+  if (C.one_launch() && SB <= kFusedMaxSB) {
+    const FusedForm<TV> f = fused_form<TV>(SB);
+    const FusedArgs A{n, SB, nblk, map, Dinv, DT, Gm, H, vb, (unsigned long long*)(va + np),
+                      (unsigned long long*)(vb + np), C.chain};
+    hipLaunchKernelGGL(f.fn, dim3(SB / f.waves), dim3(64 * f.waves), fused_lds(SB), s, A, rdense, xdense, fl);
+    return;
+  }
+  const dim3 ownGrid(np / kOwnRows);
   if (C.one_launch()) {  // va, vb: np plain doubles, then 2 np tagged words each
     auto fwd = SB <= 4 * CT ? k_solve_chain<TV, 4, true> : k_solve_chain<TV, kChainMaxSB / CT, true>;
     auto bwd = SB <= 4 * CT ? k_solve_chain<TV, 4, false> : k_solve_chain<TV, kChainMaxSB / CT, false>;
     const dim3 grid((SB + wpb - 1) / wpb);
-    hipLaunchKernelGGL(k_solve_f0<TV>, dim3((np + wpb - 1) / wpb), dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
+    hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
                        fl);
     hipLaunchKernelGGL(fwd, grid, dim3(CT), SB * sizeof(double), s, n, SB, nblk, map, xdense, Gm, va,
                        (unsigned long long*)(va + np), C.chain, fl);
@@ -808,7 +1032,7 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
                        (unsigned long long*)(vb + np), C.chain, fl);
     return;
   }
-  hipLaunchKernelGGL(k_solve_f0<TV>, dim3((np + wpb - 1) / wpb), dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
+  hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
                      fl);
   for (int b = 1; b < nblk; ++b)
     hipLaunchKernelGGL(k_solve_step, dim3((SB + wpb - 1) / wpb), dim3(CT), 0, s, SB, b, -1, Gm, va, fl);
