@@ -34,7 +34,8 @@ struct CoarseSolver {
   void plan(int n, int bw);
   size_t band_len() const;
   size_t tinv_len() const { return (size_t)np * 64; }
-  // two panels of row tiles (64x64) below a diagonal tile: the factorization's scratch
+  // two panels of row tiles (64x64) below a diagonal tile, each with a tile for
+  // the inverses of the diagonal tile's 16x16 blocks: the factorization's scratch
   size_t panel_len() const { return 2 * (size_t)((bw + 63) / 64 + 1) * 64 * 64; }
   size_t blk_len() const { return (size_t)nblk * SB * SB; }
   void pad_identity(hipStream_t s, double* band);

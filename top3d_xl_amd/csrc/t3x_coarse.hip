@@ -78,61 +78,140 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 
 typedef double cd4 __attribute__((ext_vector_type(4)));
 
-// In-place Cholesky of the lower triangle of sA, blocked in 4 panels of 16
-// columns.  The block's first wave factors a 64x16 panel in registers (lane i
-// owns row i): per column the pivot and the column entries are broadcast with
-// readlane (compile-time lanes), the pivot's reciprocal square root scales
-// the column, and the rank-1 update stays in registers.  Every lane applies
-// the same operations branch-free: a lane's entries right of its diagonal
-// only ever hold values that are neither broadcast nor stored.  Then the
-// panel's rank-16 update of the trailing triangle runs on the matrix cores,
-// its 16x16 tiles round-robin over the 4 waves (the upper halves of the
-// diagonal tiles are updated too and never read).  One 64x64 tile: 8.3 us
-// against 12.8 us with the library rsqrt and 2x2 register-blocked updates.
-__device__ __forceinline__ void tile_potrf(double (*sA)[TB + 1], int* status) {
+// LDS traffic between the lanes of one wave: the hardware keeps a wave's LDS
+// operations in order; this keeps the compiler from moving a lane's load over
+// another lane's store (by its own addresses alone the two may be disjoint).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int PW = 8;          // waves of a factorisation work-group
+constexpr int FT = 64 * PW;    // its threads
+
+// Inverse of the 16x16 diagonal block b of the lower-triangular sL into
+// sD[b], by one wave: lane c (< 16) one column, forward substitution with
+// independent updates after each step; the reciprocal diagonal is formed
+// first (lane k), off the dependency chain.
+__device__ __forceinline__ void diag16_inverse(const double (*sL)[TB + 1], int b, double (*sD)[16][17]) {
+  const int lane = threadIdx.x & 63, o = 16 * b;
+  const double rdl = lane < 16 ? 1.0 / sL[o + lane][o + lane] : 0.0;
+  if (lane < 16) {
+    const int c = lane;
+    double bvec[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) bvec[i] = (i == c) ? 1.0 : 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const double xk = bvec[k] * readlane_d(rdl, k);  // zero above the column's diagonal
+      bvec[k] = xk;
+#pragma unroll
+      for (int i = k + 1; i < 16; ++i) bvec[i] = fma(-sL[o + i][o + k], xk, bvec[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sD[b][i][c] = bvec[i];
+  }
+}
+
+// sC(I, J) -= X_I X_J^T for the 16x16 tile (I, J), X = sX (64x64), by one wave
+__device__ __forceinline__ void tile16_syrk(double (*sC)[TB + 1], const double (*sX)[TB + 1], int I, int J) {
+  const int lane = threadIdx.x & 63, i = lane & 15, kq = lane >> 4;
+  cd4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int kb = 0; kb < TB / 4; ++kb)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sX[16 * I + i][4 * kb + kq], sX[16 * J + i][4 * kb + kq], acc, 0, 0, 0);
+#pragma unroll
+  for (int r4 = 0; r4 < 4; ++r4) sC[16 * I + kq + 4 * r4][16 * J + i] -= acc[r4];
+}
+
+// In-place Cholesky of the lower triangle of sA, and the inverses of its first
+// three 16x16 diagonal blocks (sD), blocked in 4 panels of 16 columns, by PW
+// waves.
+// Wave 0 factors a 64x16 panel in registers (lane i owns row i): the pivot and
+// the column entries are broadcast with readlane (compile-time lanes), the
+// pivot's reciprocal square root scales the column, and the rank-1 update
+// stays in registers.  Every lane applies the same operations branch-free: a
+// lane's entries right of its diagonal only ever hold values that are neither
+// broadcast nor stored.  The panel's rank-16 update of the trailing triangle
+// runs on the matrix cores, the next panel's 16 columns first (one tile per
+// wave); the other tiles, the inverse of the block just factored and the
+// caller's side work (side(w, b) on waves w = 1 .. PW - 1 while panel b is
+// factored; the columns before it are final) run while wave 0 factors on.  The
+// upper halves of the diagonal tiles are updated too and never read.
+// Bound: the latency chain of 64 pivots (broadcast, reciprocal square root,
+// scale, update of the next column); the updates of the columns after that fill
+// its waits, their factors broadcast through LDS (7.2 us a tile; all of them by
+// readlane 8.0).
+template <class Side>
+__device__ __forceinline__ void tile_potrf(double (*sA)[TB + 1], double (*sD)[16][17], int* status, Side side) {
   constexpr int PB = 16;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, kq = lane >> 4;
+  __shared__ double sC[2][TB];  // wave 0's columns, for broadcasts
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kq = lane >> 4;
+  // the rank-16 update of panel b on 16x16 tile (I, J)
+  auto update = [&](int b, int I, int J) {
+    cd4 acc;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) acc[r4] = sA[16 * I + kq + 4 * r4][16 * J + li];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-sA[16 * I + li][PB * b + 4 * kb + kq],
+                                                 sA[16 * J + li][PB * b + 4 * kb + kq], acc, 0, 0, 0);
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) sA[16 * I + kq + 4 * r4][16 * J + li] = acc[r4];
+  };
 #pragma unroll
   for (int b = 0; b < TB / PB; ++b) {
     const int b0 = b * PB;
-    if (threadIdx.x < 64) {
+    if (w == 0) {
       double p[PB];
 #pragma unroll
       for (int k = 0; k < PB; ++k) p[k] = sA[lane][b0 + k];
       bool bad = false;
+      double piv = readlane_d(p[0], b0);
+      double rs = rsqrt_nr(piv);
+      double c[PB] = {};  // column k - 1's entries (b0 + kk, k - 1), kk >= k + 2
 #pragma unroll
       for (int k = 0; k < PB; ++k) {
-        const double piv = readlane_d(p[k], b0 + k);
         bad |= !(piv > 0.0);
-        p[k] *= rsqrt_nr(piv);  // the pivot's lane gets sqrt(piv), lanes below L(i, c)
+        p[k] *= rs;  // the pivot's lane gets sqrt(piv), lanes below L(i, c)
+        sC[k & 1][lane] = p[k];
+        wave_lds_fence();
+        auto rank1 = [&](int kk) { p[kk] = fma(-p[k], readlane_d(p[k], b0 + kk), p[kk]); };
+        if (k + 1 < PB) {
+          rank1(k + 1);
+          piv = readlane_d(p[k + 1], b0 + k + 1);
+          const double y = __builtin_amdgcn_rsq(piv);  // rsqrt_nr(piv) for the next column
+          if (k > 0) {
 #pragma unroll
-        for (int kk = k + 1; kk < PB; ++kk) p[kk] -= p[k] * readlane_d(p[k], b0 + kk);
+            for (int kk = k + 2; kk < PB; ++kk) p[kk] = fma(-p[k - 1], c[kk], p[kk]);
+          }
+          if (k + 2 < PB) rank1(k + 2);
+#pragma unroll
+          for (int kk = k + 3; kk < PB; ++kk) c[kk] = sC[k & 1][b0 + kk];
+          const double h = fma(-piv * y, y, 1.0);
+          rs = fma(y * h, 0.5, y);
+        }
       }
-      if (lane >= b0) {
+      if (lane >= b0) {  // (entries right of the diagonal are never read)
 #pragma unroll
-        for (int k = 0; k < PB; ++k)
-          if (b0 + k <= lane) sA[lane][b0 + k] = p[k];
+        for (int k = 0; k < PB; ++k) sA[lane][b0 + k] = p[k];
       }
       if (bad && lane == 0) *status = 1;
+    } else {
+      if (b > 0) {  // the rest of panel b - 1's update: tiles right of this panel
+        int t = 1;
+#pragma unroll
+        for (int J = b + 1; J < TB / PB; ++J)
+#pragma unroll
+          for (int I = J; I < TB / PB; ++I, ++t)
+            if (w == t) update(b - 1, I, J);
+        if (w == PW - 1) diag16_inverse(sA, b - 1, sD);
+      }
+      side(w, b);
     }
     __syncthreads();
-    if (b0 + PB < TB) {  // trailing triangle: 16x16 tiles (I, J), J <= I, at rows/columns >= b0 + PB
-      const int t0 = b0 + PB, m = (TB - t0) / 16;
-      for (int t = w; t < m * (m + 1) / 2; t += CT / 64) {
-        int I = 0;
-        while ((I + 1) * (I + 2) / 2 <= t) ++I;
-        const int J = t - I * (I + 1) / 2;
-        const int R0 = t0 + 16 * I, C0 = t0 + 16 * J;
-        cd4 acc;
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) acc[r4] = sA[R0 + kq + 4 * r4][C0 + li];
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-sA[R0 + li][b0 + 4 * kb + kq], sA[C0 + li][b0 + 4 * kb + kq],
-                                                     acc, 0, 0, 0);
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) sA[R0 + kq + 4 * r4][C0 + li] = acc[r4];
-      }
+    if (b + 1 < TB / PB) {
+      if (w < TB / PB - 1 - b) update(b, b + 1 + w, b + 1);
       __syncthreads();
     }
   }
@@ -220,40 +299,18 @@ __device__ __forceinline__ void tile_gemm_nn_mfma(const double (*sA)[TB + 1], co
   }
 }
 
-// Inverses of the four 16x16 diagonal blocks of the lower-triangular sL into
-// sD[4][16][16]: wave w inverts block w, lane c (< 16) one column, by
-// forward substitution with independent updates after each step; the
-// reciprocal diagonal is formed first (lane k), off the dependency chain.
-__device__ __forceinline__ void diag16_inverses(const double (*sL)[TB + 1], double (*sD)[16][17]) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, o = 16 * w;
-  const double rdl = lane < 16 ? 1.0 / sL[o + lane][o + lane] : 0.0;
-  if (lane < 16) {
-    const int c = lane;
-    double bvec[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) bvec[i] = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const double xk = bvec[k] * readlane_d(rdl, k);  // zero above the column's diagonal
-      bvec[k] = xk;
-#pragma unroll
-      for (int i = k + 1; i < 16; ++i) bvec[i] -= sL[o + i][o + k] * xk;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sD[w][i][c] = bvec[i];
-  }
-}
-
 // X = A L^{-T} in place (sX: A on entry, X on exit), blocked by 16 columns on
 // the matrix cores:  R_b = A_b - X_{<b} L_{b,<b}^T,  X_b = R_b Dinv_b^T,
-// Dinv_b the inverses of L's diagonal blocks.  Wave w owns rows 16w..16w+15
-// throughout, so the waves need no barrier between the steps.
+// Dinv_b the inverses of L's diagonal blocks; column blocks [b0, b1).  Wave w of
+// four owns rows 16w..16w+15 throughout, so the waves need no barrier between
+// the steps.
+template <int b0, int b1>
 __device__ __forceinline__ void tile_trsm_rt(double (*sX)[TB + 1], const double (*sL)[TB + 1],
-                                             const double (*sD)[16][17]) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, kq = lane >> 4;
+                                             const double (*sD)[16][17], int w) {
+  const int lane = threadIdx.x & 63, i = lane & 15, kq = lane >> 4;
   const int r0 = 16 * w;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+  for (int b = b0; b < b1; ++b) {
     cd4 acc;
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) acc[r4] = sX[r0 + kq + 4 * r4][16 * b + i];  // D layout: row kq + 4 r4, col i
@@ -262,12 +319,14 @@ __device__ __forceinline__ void tile_trsm_rt(double (*sX)[TB + 1], const double 
       acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-sX[r0 + i][4 * kb + kq], sL[16 * b + i][4 * kb + kq], acc, 0, 0, 0);
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) sX[r0 + kq + 4 * r4][16 * b + i] = acc[r4];  // R_b
+    wave_lds_fence();
     cd4 x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)  // X_b = R_b Dinv_b^T
       x = __builtin_amdgcn_mfma_f64_16x16x4f64(sX[r0 + i][16 * b + 4 * kb + kq], sD[b][i][4 * kb + kq], x, 0, 0, 0);
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) sX[r0 + kq + 4 * r4][16 * b + i] = x[r4];
+    wave_lds_fence();
   }
 }
 
@@ -286,25 +345,25 @@ __device__ __forceinline__ void stage_tile(BandView V, int i0, int k0, double (*
     sT[t / TB][t % TB] = v[u];
   }
 }
-// Two or three tiles at once (one memory round trip): (i0, k0) -> s0,
-// (i1, k1) -> s1 and, with THREE, (i2, k2) -> s2.  THREE is a compile-time
+// Two or three tiles at once (one memory round trip), by FT threads: (i0, k0) ->
+// s0, (i1, k1) -> s1 and, with THREE, (i2, k2) -> s2.  THREE is a compile-time
 // choice: a load under a run-time condition makes the compiler wait for the
 // loads before it at every branch.
 template <bool THREE>
 __device__ __forceinline__ void stage_tiles(BandView V, int i0, int k0, double (*s0)[TB + 1], int i1, int k1,
                                             double (*s1)[TB + 1], int i2, int k2, double (*s2)[TB + 1]) {
-  constexpr int U = TB * TB / CT;
+  constexpr int U = TB * TB / FT;
   double v0[U], v1[U], v2[THREE ? U : 1];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int t = threadIdx.x + u * CT, r = t / TB, c = t % TB;
+    const int t = threadIdx.x + u * FT, r = t / TB, c = t % TB;
     v0[u] = V.get(i0 + r, k0 + c);
     v1[u] = V.get(i1 + r, k1 + c);
     if constexpr (THREE) v2[u] = V.get(i2 + r, k2 + c);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int t = threadIdx.x + u * CT, r = t / TB, c = t % TB;
+    const int t = threadIdx.x + u * FT, r = t / TB, c = t % TB;
     s0[r][c] = v0[u];
     s1[r][c] = v1[u];
     if constexpr (THREE) s2[r][c] = v2[u];
@@ -312,41 +371,78 @@ __device__ __forceinline__ void stage_tiles(BandView V, int i0, int k0, double (
 }
 
 // ---- 1. banded Cholesky ---------------------------------------------------
-__global__ __launch_bounds__(CT) void k_chol_diag(BandView V, int d0, int* status) {
-  __shared__ double sA[TB][TB + 1];
-  for (int t = threadIdx.x; t < TB * TB; t += CT) sA[t / TB][t % TB] = V.get(d0 + t / TB, d0 + t % TB);
-  __syncthreads();
-  tile_potrf(sA, status);
-  for (int t = threadIdx.x; t < TB * TB; t += CT) {
-    const int i = t / TB, k = t % TB;
+// Columns [16 c, 16 c + 16) of the factored tile, and the inverse of its
+// diagonal block (c < 3), from LDS to the band and to dinv [3][16][16]; t: this
+// thread's place among nt
+__device__ __forceinline__ void store_cols(BandView V, int d0, const double (*sA)[TB + 1], int c, int t, int nt) {
+  for (int e = t; e < TB * 16; e += nt) {
+    const int i = e >> 4, k = 16 * c + (e & 15);
     if (k <= i) V.set(d0 + i, d0 + k, sA[i][k]);
   }
+}
+__device__ __forceinline__ void store_inverse(const double (*sD)[16][17], double* __restrict__ dinv, int c, int t,
+                                              int nt) {
+  for (int e = t; e < 256; e += nt) dinv[256 * c + e] = sD[c][e >> 4][e & 15];
+}
+// what is left to store once tile_potrf has returned, if its side work called
+// store_early: the last columns and the third inverse
+constexpr int kStoreWaves = 2;  // waves 5 and 6
+__device__ __forceinline__ void store_early(BandView V, int d0, const double (*sA)[TB + 1], const double (*sD)[16][17],
+                                            double* __restrict__ dinv, int sw, int b) {
+  const int t = (sw - 5) * 64 + (threadIdx.x & 63);
+  if (b == 0 || t < 0 || t >= 64 * kStoreWaves) return;
+  store_cols(V, d0, sA, b - 1, t, 64 * kStoreWaves);
+  if (b >= 2) store_inverse(sD, dinv, b - 2, t, 64 * kStoreWaves);
+}
+__device__ __forceinline__ void store_rest(BandView V, int d0, const double (*sA)[TB + 1], const double (*sD)[16][17],
+                                           double* __restrict__ dinv) {
+  store_cols(V, d0, sA, 3, threadIdx.x, FT);
+  store_inverse(sD, dinv, 2, threadIdx.x, FT);
+}
+
+__global__ __launch_bounds__(FT) void k_chol_diag(BandView V, int d0, double* __restrict__ dinv, int* status) {
+  __shared__ double sA[TB][TB + 1];
+  __shared__ double sD[4][16][17];
+  for (int t = threadIdx.x; t < TB * TB; t += FT) sA[t / TB][t % TB] = V.get(d0 + t / TB, d0 + t % TB);
+  __syncthreads();
+  tile_potrf(sA, sD, status, [&](int sw, int b) { store_early(V, d0, sA, sD, dinv, sw, b); });
+  store_rest(V, d0, sA, sD, dinv);
 }
 
 // One launch per 64-column panel J (right-looking, the panel solve folded into
 // the trailing update).  Work-group (I, K), K <= I, over the row tiles below
 // diagonal tile J that the band reaches:
-//   X_I = A(I, J) L_JJ^{-T}, X_K = A(K, J) L_JJ^{-T}   (substitution in LDS)
+//   X_I = A(I, J) L_JJ^{-T}, X_K = A(K, J) L_JJ^{-T}   (four waves each)
 //   A(I, K) -= X_I X_K^T                               (matrix cores)
 // The (I, I) groups keep L(I, J) = X_I in a scratch panel (the band's copy of
 // A(I, J) is still being read by the other groups); the next launch's extra
-// groups copy it into the band.  Group (0, 0) updates the next diagonal tile
-// and factors it.
-__global__ __launch_bounds__(CT) void k_chol_panel(BandView V, int J, int nrt, int nrtPrev,
-                                                   double* __restrict__ pan, int panStride, int* status) {
+// groups copy it into the band.  Group (0, 0) updates the next diagonal tile,
+// factors it and leaves the inverses of its first three 16x16 diagonal blocks
+// behind the scratch panel for the next launch's substitutions (the last one,
+// which would prolong its chain, is formed there beside their first steps).
+// Bound: group (0, 0)'s latency chain; all it does but that chain (the tiles
+// of X X^T past the first 16 columns, L(I, J) to the scratch panel, the
+// inverses, the stores of finished columns) runs beside the pivots.  20.9 ->
+// 15.9 us a launch at 128x256x128 and 256x512x256 (20.3 -> 14.4 at 50x100x50);
+// its parts there, with four waves and in sequence / now: staging 3.6 / 2.3,
+// inverses and substitution 3.3 / 2.7, product 3.0 / 0.75, pivots 8.0 / 7.4,
+// store 1.6 / 0.4 us.
+__global__ __launch_bounds__(FT) void k_chol_panel(BandView V, int J, int nrt, int nrtPrev, double* __restrict__ pan,
+                                                   int panStride, int* status) {
   __shared__ double sL[TB][TB + 1];  // L_JJ (zeros above the diagonal)
   __shared__ double sA[TB][TB + 1];  // A(I, J) -> X_I
   __shared__ double sB[TB][TB + 1];  // A(K, J) -> X_K, or the next diagonal tile
-  __shared__ double sD[4][16][17];   // inverses of L_JJ's 16x16 diagonal blocks
+  __shared__ double sD[4][16][17];   // inverses of L_JJ's 16x16 diagonal blocks, then of the next tile's
   const int bw = V.bw, n = V.n;
   const int j0 = J * TB, r0 = j0 + TB;
   const int npairs = nrt * (nrt + 1) / 2;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if ((int)blockIdx.x >= npairs) {  // copy row tile t of panel J - 1 into the band
     const int t = blockIdx.x - npairs;
     if (t >= nrtPrev) return;
     const double* src = pan + (size_t)((J - 1) & 1) * panStride + (size_t)t * TB * TB;
     const int i0 = j0 + t * TB, k0 = j0 - TB;
-    for (int e = threadIdx.x; e < TB * TB; e += CT) V.set(i0 + e / TB, k0 + e % TB, src[e]);
+    for (int e = threadIdx.x; e < TB * TB; e += FT) V.set(i0 + e / TB, k0 + e % TB, src[e]);
     return;
   }
   const int t0 = blockIdx.x;
@@ -355,6 +451,10 @@ __global__ __launch_bounds__(CT) void k_chol_panel(BandView V, int J, int nrt, i
   const int K = t0 - I * (I + 1) / 2;
   const int i0 = r0 + I * TB, k0 = r0 + K * TB;
   if (i0 - (k0 + TB - 1) > bw) return;  // tile outside the band
+  double* panJ = pan + (size_t)(J & 1) * panStride;
+  // the inverses lie behind the panel's last row tile
+  const double* dinv = panJ + panStride - TB * TB;
+  const double dv0 = dinv[threadIdx.x], dv1 = dinv[FT + (threadIdx.x & 255)];  // 768 entries
   // L_JJ (zeros above the diagonal), A(I, J), and A(K, J) or, for group
   // (0, 0), the next diagonal tile (no other group of this launch writes it)
   if (K != I)
@@ -363,42 +463,55 @@ __global__ __launch_bounds__(CT) void k_chol_panel(BandView V, int J, int nrt, i
     stage_tiles<true>(V, j0, j0, sL, i0, j0, sA, r0, r0, sB);
   else
     stage_tiles<false>(V, j0, j0, sL, i0, j0, sA, 0, 0, nullptr);
+  sD[threadIdx.x >> 8][(threadIdx.x >> 4) & 15][threadIdx.x & 15] = dv0;
+  if (threadIdx.x < 256) sD[2][threadIdx.x >> 4][threadIdx.x & 15] = dv1;
   __syncthreads();
-  diag16_inverses(sL, sD);
+  if (w == PW - 1) diag16_inverse(sL, 3, sD);
+  if (w < 4) tile_trsm_rt<0, 3>(sA, sL, sD, w);
+  else if (K != I) tile_trsm_rt<0, 3>(sB, sL, sD, w - 4);
   __syncthreads();
-  tile_trsm_rt(sA, sL, sD);
-  if (K != I) tile_trsm_rt(sB, sL, sD);
+  if (w < 4) tile_trsm_rt<3, 4>(sA, sL, sD, w);
+  else if (K != I) tile_trsm_rt<3, 4>(sB, sL, sD, w - 4);
   __syncthreads();
-  if (K == I) {  // L(I, J) to the scratch panel
-    double* dst = pan + (size_t)(J & 1) * panStride + (size_t)I * TB * TB;
-    for (int t = threadIdx.x; t < TB * TB; t += CT) dst[t] = sA[t / TB][t % TB];
-  }
-  cd4 acc[2][2] = {};
-  tile_gemm_nt_mfma(sA, K == I ? sA : sB, acc);  // X_I X_K^T
   if (I == 0) {  // the next diagonal tile (staged in sB): update in LDS, then factor
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) sB[nt_row(a, r4)][nt_col(b)] -= acc[a][b][r4];
+    if (w < 4) tile16_syrk(sB, sA, w, 0);
     __syncthreads();
-    tile_potrf(sB, status);
-    for (int t = threadIdx.x; t < TB * TB; t += CT) {
-      const int i = t / TB, k = t % TB;
-      if (k <= i) V.set(r0 + i, r0 + k, sB[i][k]);
-    }
+    double* dinvNext = pan + (size_t)((J + 1) & 1) * panStride + panStride - TB * TB;
+    tile_potrf(sB, sD, status, [&](int sw, int b) {
+      if (b == 0) {
+        if (sw <= 6) {  // the other lower tiles of X X^T
+          const int tI = sw <= 3 ? sw : (sw <= 5 ? sw - 2 : 3), tJ = sw <= 3 ? 1 : (sw <= 5 ? 2 : 3);
+          tile16_syrk(sB, sA, tI, tJ);
+        }
+        for (int t = (sw - 1) * 64 + lane; t < TB * TB; t += 64 * (PW - 1)) panJ[t] = sA[t / TB][t % TB];  // L(I, J)
+      }
+      store_early(V, r0, sB, sD, dinvNext, sw, b);
+    });
+    store_rest(V, r0, sB, sD, dinvNext);
     return;
   }
+  if (K == I) {  // L(I, J) to the scratch panel
+    double* dst = panJ + (size_t)I * TB * TB;
+    for (int t = threadIdx.x; t < TB * TB; t += FT) dst[t] = sA[t / TB][t % TB];
+  }
+  // A(I, K) -= X_I X_K^T: wave w the 16x16 tiles (w / 2, 2 (w % 2)) and the one beside it
+  const double(*sK)[TB + 1] = K == I ? sA : sB;
+  const int i = lane & 15, kq = lane >> 4, R = 16 * (w >> 1), C = 32 * (w & 1);
+  cd4 acc[2] = {};
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int kb = 0; kb < TB / 4; ++kb) {
+    const double a = sA[R + i][4 * kb + kq];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int c = 0; c < 2; ++c)
+      acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, sK[C + 16 * c + i][4 * kb + kq], acc[c], 0, 0, 0);
+  }
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int i = i0 + nt_row(a, r4), k = k0 + nt_col(b);
-        if (k <= i && i - k <= bw && i < n) V.B[(size_t)i * V.W() + (i - k)] -= acc[a][b][r4];
-      }
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const int row = i0 + R + kq + 4 * r4, col = k0 + C + 16 * c + i;
+      if (col <= row && row - col <= bw && row < n) V.B[(size_t)row * V.W() + (row - col)] -= acc[c][r4];
+    }
 }
 
 // Inverses of all 64x64 diagonal tiles (after the factorization, in parallel).
@@ -985,7 +1098,9 @@ void CoarseSolver::factor(hipStream_t s, double* band, double* tinv, double* pan
   BandView V{band, np, bw};
   const int nt = np / TB;
   const int panStride = (int)(panel_len() / 2);
-  hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(CT), 0, s, V, 0, status);
+  // tile J's inverses lie behind scratch panel J mod 2 (its row tiles: (bw + 63) / 64)
+  auto dinv = [&](int J) { return pan + (size_t)(J & 1) * panStride + panStride - TB * TB; };
+  hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(FT), 0, s, V, 0, dinv(0), status);
   int nrtPrev = 0;
   for (int J = 0; J < nt; ++J) {
     const int j0 = J * TB, r0 = j0 + TB;
@@ -993,12 +1108,12 @@ void CoarseSolver::factor(hipStream_t s, double* band, double* tinv, double* pan
     const int nrt = rlast >= r0 ? (rlast - r0) / TB + 1 : 0;
     const int grid = nrt * (nrt + 1) / 2 + nrtPrev;
     if (nrt > 0 || nrtPrev > 0)
-      hipLaunchKernelGGL(k_chol_panel, dim3(grid), dim3(CT), 0, s, V, J, nrt, nrtPrev, pan, panStride, status);
-    if (nrt == 0 && J + 1 < nt) hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(CT), 0, s, V, r0, status);
+      hipLaunchKernelGGL(k_chol_panel, dim3(grid), dim3(FT), 0, s, V, J, nrt, nrtPrev, pan, panStride, status);
+    if (nrt == 0 && J + 1 < nt) hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(FT), 0, s, V, r0, dinv(J + 1), status);
     nrtPrev = nrt;
   }
   if (nrtPrev > 0)  // copy the last panel
-    hipLaunchKernelGGL(k_chol_panel, dim3(nrtPrev), dim3(CT), 0, s, V, nt, 0, nrtPrev, pan, panStride, status);
+    hipLaunchKernelGGL(k_chol_panel, dim3(nrtPrev), dim3(FT), 0, s, V, nt, 0, nrtPrev, pan, panStride, status);
   hipLaunchKernelGGL(k_tile_inverses, dim3(nt), dim3(CT), 0, s, V, tinv);
   const int st = SB / TB;
   hipLaunchKernelGGL(k_trsm_blocks, dim3(nblk * 2 * st), dim3(CT), 0, s, V, SB, tinv, Dinv, DT, Gm);
