@@ -1193,12 +1193,11 @@ double masked_sum(t3x_problem& P, const double* a, const double* b, int mode) {
 // ------------------------------------------------------------- OC (145-155)
 double oc_update(t3x_problem& P, double* x, const double* xPhys, const double* dc, double V0, int* nBis) {
   hipStream_t s = P.stream;
-  const double fval = masked_sum(P, xPhys, nullptr, 0) / (double)P.nCells - V0;  // 145
-  const double init[8] = {0.0, 1e9, fval, 0.0, 0.0, 0.0, 0.0, 0.0};            // 146
-  launch_set_vals(s, P.oc, 8, init);
-  for (int pass = 0; pass < 64; ++pass) {
-    launch_oc_pass(s, P.NN(), P.lv[0].emask, P.passive, x, dc, P.ws, P.oc, 3);
-    if (pass % 8 == 7) {
+  launch_masked_sum(s, P.NN(), P.lv[0].emask, xPhys, nullptr, 0, P.ws, P.sc + 32);
+  launch_oc_begin(s, P.sc + 32, (double)P.nCells, V0, P.ws, P.oc);  // 145-146
+  for (int pass = 0; pass < kOcMaxPasses; ++pass) {
+    launch_oc_pass(s, P.NN(), P.lv[0].emask, P.passive, x, dc, P.ws, P.oc);
+    if (oc_check_after(pass)) {
       T3X_HIP(hipMemcpyAsync(P.hbuf, P.oc, 8 * sizeof(double), hipMemcpyDeviceToHost, s));
       P.sync();
       if (P.hbuf[3] != 0.0) break;

@@ -236,8 +236,14 @@ void launch_masked_sum(hipStream_t s, long long n, const uint8_t* emask, const d
                        int mode, const RedWs& ws, double* out);
 void launch_masked_maxdiff(hipStream_t s, long long n, const uint8_t* emask, const double* a, const double* b,
                            const RedWs& ws, double* out);
+// OC (145-155): begin (vsum: the sum of xPhys over the n cells), passes until
+// oc[3] is set, final.  oc_check_after: whether to look at oc[3] after pass i
+// (most searches end with the fifth or sixth pass).
+void launch_oc_begin(hipStream_t s, const double* vsum, double n, double V0, const RedWs& ws, double* oc);
 void launch_oc_pass(hipStream_t s, long long n, const uint8_t* emask, const uint8_t* passive, const double* x,
-                    const double* dc, const RedWs& ws, double* oc, int depth);
+                    const double* dc, const RedWs& ws, double* oc);
+constexpr int kOcMaxPasses = 64;
+inline bool oc_check_after(int pass) { return pass >= 4 && pass % 2 == 0; }
 void launch_oc_final(hipStream_t s, long long n, const uint8_t* emask, const uint8_t* passive, double* x,
                      const double* dc, const RedWs& ws, double* oc);
 void launch_set_where(hipStream_t s, long long n, const uint8_t* mask, double* a, double v);

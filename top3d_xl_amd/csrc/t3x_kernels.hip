@@ -1130,13 +1130,35 @@ void launch_masked_sum(hipStream_t s, long long n, const uint8_t* emask, const d
   fin1(s, FIN_SUM, red_blocks(n), ws, nullptr, nullptr, out);
 }
 
-// ---- OC bisection (145-153), k-ary: one pass evaluates the 2^depth-1
-// midpoints of the next `depth` bisection levels; the last block replays the
-// sequential decisions with identical arithmetic.  emask == nullptr: every
-// cell is a design cell (compact cell arrays).
-// oc[]: 0 l1, 1 l2, 2 fval, 3 done, 4 lastLmid, 5 nBisect, 6 change
+// ---- OC bisection (145-153) by brackets: a pass evaluates gt at 15 multipliers
+// (candidates) in one sweep over the cells; the finaliser keeps the largest with
+// gt > 0 and the smallest with gt <= 0 and replays the sequential bisection as
+// far as these decide it.  gt(l) never rises with l: every term max(lo, min(hi,
+// t / sqrt(l))) - x is monotone in l, rounded operations are, and so is a sum in
+// a fixed order.  So a midpoint at or below a candidate with gt > 0 has gt > 0
+// itself, bit for bit, and likewise above one with gt <= 0; the decisions, the
+// final multiplier and the bisection count are the sequential loop's.  Candidates
+// close in on the root: powers of 16, then quarter octaves, then clusters
+// around the bracket's secant (the 2^4 - 1 midpoints the loop would visit next,
+// once the bracket is as fine as they are).  Bound: a pass's FP64 issue (115
+// instructions a cell) and its 16 bytes a cell about alike, so passes count: 5
+// instead of the 13 that 4 levels of midpoints at a time need (33.5M cells, the
+// whole update 2.74 -> 1.16 ms; 50x100x50 0.55 -> 0.2 ms).
+// emask == nullptr: every cell is a design cell (compact cell arrays).
+// oc[]: 0 l1, 1 l2, 2 fval, 3 done, 4 lastLmid, 5 nBisect, 6 change; the
+// candidates and the bracket lie behind the pass's partials (OcSearch).
 constexpr int kOcDepth = 4;
 constexpr int kOcCand = (1 << kOcDepth) - 1;
+constexpr int kOcMaxLevels = 256;  // bisection levels at most (no root above 1e9 2^-256)
+struct OcSearch {
+  double l[kOcCand + 1], rl[kOcCand + 1];  // candidates and 1 / sqrt of them
+  double A, gA, B, gB;                     // bracket: gt(A) = gA > 0 (A = 0: none yet), gt(B) = gB <= 0 (B = inf: none)
+};
+static_assert(kOcCand * kMaxRedBlocks + sizeof(OcSearch) / 8 <= 16 * kMaxRedBlocks,
+              "the search state fits behind the partials of the widest pass");
+__host__ __device__ inline OcSearch* oc_search(double* partials) {
+  return (OcSearch*)(partials + kOcCand * kMaxRedBlocks);
+}
 
 // x .* sqrt(-dc ./ lmid) (149) as t * rl with t = x sqrt(-dc) formed once per
 // cell and rl = 1/sqrt(lmid) once per candidate, then the move limits (150).
@@ -1148,30 +1170,42 @@ __device__ __forceinline__ double oc_clamp(double x, double v) {
   return fmax(0.0, v);
 }
 
+// fval = mean(xPhys) - V0 (145), l1 = 0, l2 = 1e9 (146), the first candidates
+__global__ __launch_bounds__(64) void k_oc_begin(const double* __restrict__ vsum, double n, double V0, double* oc,
+                                                 double* partials) {
+  OcSearch* S = oc_search(partials);
+  const int k = threadIdx.x;
+  if (k == 0) {
+    oc[0] = 0.0;
+    oc[1] = 1e9;
+    oc[2] = *vsum / n - V0;
+    oc[3] = oc[4] = oc[5] = oc[6] = 0.0;
+    S->A = 0.0;
+    S->gA = 0.0;
+    S->B = INFINITY;
+    S->gB = 0.0;
+  }
+  if (k < kOcCand) {
+    const double l = ldexp(1.0, 4 * k - 30);  // 9e-10 .. 6.7e7
+    S->l[k] = l;
+    S->rl[k] = 1.0 / sqrt(l);
+  }
+}
+void launch_oc_begin(hipStream_t s, const double* vsum, double n, double V0, const RedWs& ws, double* oc) {
+  hipLaunchKernelGGL(k_oc_begin, dim3(1), dim3(64), 0, s, vsum, n, V0, oc, ws.partials);
+}
+
 __global__ __launch_bounds__(kBlock) void k_oc_pass(long long n, const uint8_t* __restrict__ emask,
                                                     const uint8_t* __restrict__ passive,
                                                     const double* __restrict__ x, const double* __restrict__ dc,
-                                                    RedWs ws, double* oc) {
+                                                    RedWs ws, const double* oc) {
   if (oc[3] != 0.0) return;
-  const double l1 = oc[0], l2 = oc[1];
-  // heap-ordered candidate intervals: node k -> (a,b); children 2k (gt<=0), 2k+1 (gt>0)
-  double lm[kOcCand + 1], A[2 * kOcCand + 2], Bv[2 * kOcCand + 2];
-  A[1] = l1;
-  Bv[1] = l2;
-  for (int k = 1; k <= kOcCand; ++k) {
-    lm[k] = 0.5 * (Bv[k] + A[k]);
-    if (2 * k + 1 <= 2 * kOcCand + 1) {
-      A[2 * k] = A[k];
-      Bv[2 * k] = lm[k];
-      A[2 * k + 1] = lm[k];
-      Bv[2 * k + 1] = Bv[k];
-    }
-  }
+  const OcSearch* S = oc_search(ws.partials);
   double s[kOcCand], rl[kOcCand];
 #pragma unroll
   for (int k = 0; k < kOcCand; ++k) {
     s[k] = 0.0;
-    rl[k] = 1.0 / sqrt(lm[k + 1]);
+    rl[k] = S->rl[k];
   }
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) {
     if (emask && !emask[i]) continue;
@@ -1192,35 +1226,126 @@ __global__ __launch_bounds__(kBlock) void k_oc_pass(long long n, const uint8_t* 
   write_partials<kOcCand>(s, ws.partials);
 }
 
-__global__ __launch_bounds__(kFinBlock) void k_oc_fin(int nb, const double* __restrict__ partials, double* oc) {
+// One wave per candidate folds its partials (as 1024 threads would: each its
+// partials b, b + 1024, .., then 16 wave sums in order), then the first thread
+// replays the bisection and the candidates' threads place the next ones.
+__global__ __launch_bounds__(kFinBlock) void k_oc_fin(int nb, double* partials, double* oc) {
   if (oc[3] != 0.0) return;
-  double s[kOcCand];
-  fold_partials<kOcCand, kFinBlock>(partials, nb, s);
-  if (threadIdx.x != 0) return;
-  const double l1 = oc[0], l2 = oc[1];
-  double a = l1, b = l2;
-  int node = 1;
-  const double fval = oc[2];
-  int nbis = (int)oc[5];
-  double last = oc[4];
-  bool done = false;
-  for (int d = 0; d < kOcDepth; ++d) {
-    if (!((b - a) / (a + b) > 1e-6)) { done = true; break; }  // 147
-    const double lmid = 0.5 * (b + a);                         // 148
-    const double gt = fval + s[node - 1];                      // 151
-    if (gt > 0) { a = lmid; node = 2 * node + 1; } else { b = lmid; node = 2 * node; }  // 152
-    last = lmid;
-    ++nbis;
+  __shared__ double sg[kOcCand + 1], sl[kOcCand + 1], sq[8], so[8];  // gt, candidates, bracket, oc
+  __shared__ double sA, sB, sL1, sL2, sEst, sE;
+  __shared__ int sMode;  // 0 done; 1 powers of 16 below B; 2 quarter octaves; 3 secant cluster; 4 midpoints
+  OcSearch* S = oc_search(partials);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  static_assert(kFinBlock == 1024 && kOcCand <= 15, "a wave per candidate, 16 groups of 64 partials");
+  if (w == 15) {  // what the first thread reads one after the other, in one round trip
+    if (lane < kOcCand) sl[lane] = S->l[lane];
+    else if (lane >= 16 && lane < 20) sq[lane - 16] = (&S->A)[lane - 16];
+    else if (lane >= 24 && lane < 32) so[lane - 24] = oc[lane - 24];
   }
-  if (!((b - a) / (a + b) > 1e-6)) done = true;
-  oc[0] = a;
-  oc[1] = b;
-  oc[4] = last;
-  oc[5] = (double)nbis;
-  if (done) oc[3] = 1.0;
+  if (w < kOcCand) {
+    const double fval = oc[2];
+    const double* p = partials + (size_t)w * nb;
+    static_assert(kMaxRedBlocks <= 2 * kFinBlock, "at most two partials per thread of the fold");
+    double s = 0.0;
+    for (int g0 = 0; g0 < 16; g0 += 8) {
+      double a[8];
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const int b = 64 * (g0 + g) + lane;
+        const double p0 = p[min(b, nb - 1)], p1 = p[min(b + 1024, nb - 1)];
+        a[g] = b < nb ? p0 : 0.0;
+        if (b + 1024 < nb) a[g] += p1;
+      }
+      for (int g = 0; g < 8; ++g) s += wave_sum(a[g]);
+    }
+    if (lane == 0) sg[w] = fval + s;  // gt (151)
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double A = sq[0], gA = sq[1], B = sq[2], gB = sq[3];
+#pragma unroll
+    for (int k = 0; k < kOcCand; ++k) {
+      const double l = sl[k], g = sg[k];
+      if (g > 0) {
+        if (l > A) A = l, gA = g;
+      } else if (l < B) {
+        B = l, gB = g;
+      }
+    }
+    double l1 = so[0], l2 = so[1], last = so[4];
+    int nbis = (int)so[5];
+    bool done = false;
+    for (;;) {
+      // 147; with l1 = 0 the quotient is 1
+      if (nbis >= kOcMaxLevels || (l1 != 0.0 && !((l2 - l1) / (l1 + l2) > 1e-6))) { done = true; break; }
+      const double lmid = 0.5 * (l2 + l1);  // 148
+      if (lmid <= A) l1 = lmid;             // 152: gt > 0
+      else if (lmid >= B) l2 = lmid;
+      else break;
+      last = lmid;
+      ++nbis;
+    }
+    oc[0] = l1;
+    oc[1] = l2;
+    oc[4] = last;
+    oc[5] = (double)nbis;
+    if (done) oc[3] = 1.0;
+    S->A = A;
+    S->gA = gA;
+    S->B = B;
+    S->gB = gB;
+    sA = A;
+    sB = B;
+    sL1 = l1;
+    sL2 = l2;
+    int mode = 4;
+    if (done) {
+      mode = 0;
+    } else if (A == 0.0 && B < INFINITY) {
+      mode = 1;
+    } else if (A > 0.0 && B < INFINITY) {
+      const double h = (B - A) / A;
+      if (h > 0.5) {
+        mode = 2;
+      } else if (h > 2e-6 && gA - gB > 0.0) {
+        // root of the secant; its error is about h^2 / 16 of l
+        mode = 3;
+        sEst = A + (B - A) * (gA / (gA - gB));
+        sE = fmax(h * h * 0.0625, 1e-8);
+      }
+    }
+    sMode = mode;
+  }
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (sMode == 0 || k >= kOcCand) return;
+  const double A = sA, B = sB;
+  double l;
+  if (sMode == 1) {
+    l = ldexp(B, 4 * (k - kOcCand));
+  } else if (sMode == 2) {  // quarter octaves from A (the first passes step by 16)
+    const double q = (k & 1) ? ((k & 2) ? 1.0 : 1.4142135623730951) : ((k & 2) ? 1.681792830507429 : 1.189207115002721);
+    l = A * ldexp(q, (k + 1) >> 2);
+  } else if (sMode == 3 && k >= 9) {  // even fractions of the bracket
+    l = A + (B - A) * ((k - 8) * (1.0 / 7));
+  } else if (sMode == 3) {  // est and est (1 +- e 4^j), j = -2 .. 1
+    const double d = k == 0 ? 0.0 : sE * ldexp(1.0, 2 * ((k - 1) >> 1) - 4);
+    l = sEst * (1.0 + ((k & 1) ? d : -d));
+  } else {  // the next midpoints: heap order, node 1 the root, children 2n (l2 = mid), 2n + 1 (l1 = mid)
+    double a = sL1, b = sL2;
+    const int node = k + 1;
+    l = 0.5 * (b + a);
+    for (int lev = 30 - __clz(node); lev >= 0; --lev) {
+      if ((node >> lev) & 1) a = l;
+      else b = l;
+      l = 0.5 * (b + a);
+    }
+  }
+  S->l[k] = l;
+  S->rl[k] = 1.0 / sqrt(l);
 }
 void launch_oc_pass(hipStream_t s, long long n, const uint8_t* emask, const uint8_t* passive, const double* x,
-                    const double* dc, const RedWs& ws, double* oc, int) {
+                    const double* dc, const RedWs& ws, double* oc) {
   hipLaunchKernelGGL(k_oc_pass, dim3(red_blocks(n)), dim3(kBlock), 0, s, n, emask, passive, x, dc, ws, oc);
   hipLaunchKernelGGL(k_oc_fin, dim3(1), dim3(kFinBlock), 0, s, red_blocks(n), ws.partials, oc);
 }

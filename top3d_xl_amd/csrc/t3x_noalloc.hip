@@ -2,7 +2,7 @@
 // any device allocation, for callers that cannot allocate (code under HIP
 // graph capture, serving loops, harnesses that forbid hipMalloc).
 //
-// The kernels are the ones behind t3x_oc (k-ary bisection, fixed-order
+// The kernels are the ones behind t3x_oc (bisection by brackets, fixed-order
 // reductions); their scratch (reduction partials, the bisection state and the
 // volume sum) lives in `scratch`, a file-scope device array of fixed size.
 // Each GPU holds its own copy at its own address: the address is looked up
@@ -25,8 +25,9 @@ using namespace t3x;
 namespace {
 
 // Layout (doubles): partials of the widest reduction (15 bisection
-// candidates, at most kMaxRedBlocks blocks, rounded up to 16 values per
-// block), then the 8 bisection slots, then the volume sum.
+// candidates, at most kMaxRedBlocks blocks) and the search's candidates behind
+// them, together 16 values per block, then the 8 bisection slots, then the
+// volume sum.
 constexpr long long kPartialDoubles = 16LL * kMaxRedBlocks;
 constexpr long long kOcSlot = kPartialDoubles;
 constexpr long long kSumSlot = kOcSlot + 8;
@@ -99,17 +100,11 @@ extern "C" int t3x_oc_noalloc(long long nCells, double* x, const double* xPhys, 
   double* oc = sp + kOcSlot;
   double* vsum = sp + kSumSlot;
   double hb[8];
-  // fval = mean(xPhys) - V0 (145); l1 = 0, l2 = 1e9 (146)
   launch_masked_sum(s, nCells, nullptr, xPhys, nullptr, 0, ws, vsum);
-  if ((e = hipMemcpyAsync(hb, vsum, sizeof(double), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-      (e = hipStreamSynchronize(s)) != hipSuccess)
-    return fail(e, "volume sum");
-  const double fval = hb[0] / (double)nCells - V0;
-  const double init[8] = {0.0, 1e9, fval, 0.0, 0.0, 0.0, 0.0, 0.0};
-  launch_set_vals(s, oc, 8, init);
-  for (int pass = 0; pass < 64; ++pass) {
-    launch_oc_pass(s, nCells, nullptr, passive, x, dc, ws, oc, 3);
-    if (pass % 8 == 7) {
+  launch_oc_begin(s, vsum, (double)nCells, V0, ws, oc);  // 145-146
+  for (int pass = 0; pass < kOcMaxPasses; ++pass) {
+    launch_oc_pass(s, nCells, nullptr, passive, x, dc, ws, oc);
+    if (oc_check_after(pass)) {
       if ((e = hipMemcpyAsync(hb, oc, 8 * sizeof(double), hipMemcpyDeviceToHost, s)) != hipSuccess ||
           (e = hipStreamSynchronize(s)) != hipSuccess)
         return fail(e, "bisection");
