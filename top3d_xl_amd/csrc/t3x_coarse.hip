@@ -650,9 +650,7 @@ __device__ __forceinline__ double wave_dot(const double* __restrict__ m, const d
   }
   for (; j < len; j += 64) s0 = fma(m[j], v[j], s0);
   double s = (s0 + s1) + (s2 + s3);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  return s;
+  return wave_sum(s);
 }
 
 // forward phase 0: gather the permuted right-hand side and va_b = Dinv_b v_b,
@@ -706,9 +704,7 @@ __global__ __launch_bounds__(CT) void k_solve_f0(int n, int np, int SB, const lo
   }
 #pragma unroll
   for (int r = 0; r < kOwnPerWave; ++r) {
-    double t = s[r];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+    const double t = wave_sum(s[r]);
     if (lane == 0) va[row0 + kOwnPerWave * w + r] = t;
   }
 }
@@ -766,9 +762,7 @@ __global__ void k_solve_scatter(int n, const long long* __restrict__ map, const 
 constexpr unsigned kChainSpin = 1u << 20;  // polls per wait (~1 s) before the launch gives up
 
 __device__ __forceinline__ double chain_wave_sum(double s) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  return s;
+  return wave_sum(s);
 }
 // entry i of a tagged vector: words 2i (high half of the value) and 2i + 1 (low half)
 __device__ __forceinline__ void chain_put(unsigned long long* w, int i, double v, unsigned tag) {

@@ -29,15 +29,44 @@ __device__ __forceinline__ dim3 xcd_tile_order() {
   return dim3(t % gridDim.x, (t / gridDim.x) % gridDim.y, t / (gridDim.x * gridDim.y));
 }
 
+// Reduction over the 64 lanes of a wave, all of them active; the total in every
+// lane.  The pairs are those of a butterfly over lane bits 32, 16, 8, 4, 2, 1
+// (the operands of + and max commute, so the bits are a shfl_down tree's too).
+// Register swaps between rows and rotations within rows of 16 lanes instead of
+// LDS permutes: a step's latency is an add's, 6 steps 0.05 against 0.3 us.
+__device__ __forceinline__ double lanes_double(unsigned lo, unsigned hi) {
+  return __hiloint2double((int)hi, (int)lo);
+}
+template <int ROR>
+__device__ __forceinline__ double row_rotate(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + ROR, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + ROR, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+template <class Op>
+__device__ __forceinline__ double wave_reduce(double v, Op op) {
+  {
+    const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    v = op(lanes_double(l[0], h[0]), lanes_double(l[1], h[1]));
+  }
+  {
+    const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    v = op(lanes_double(l[0], h[0]), lanes_double(l[1], h[1]));
+  }
+  v = op(v, row_rotate<8>(v));
+  v = op(v, row_rotate<4>(v));
+  v = op(v, row_rotate<2>(v));
+  return op(v, row_rotate<1>(v));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+  return wave_reduce(v, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-  return v;
+  return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
 }
 
 // Block-wide sum of NV values per thread (result valid in thread 0); NT:
