@@ -220,6 +220,8 @@ int t3x_vcycle(t3x_problem* h, const double* r, double* x);
 /* Solving_PCG(@Solving_KbyU_MatrixFree, @Solving_Vcycle, ...) (600-639); x holds x0 on entry.
  * With params.precision = 1 the preconditioner is the FP32 V-cycle. */
 int t3x_pcg(t3x_problem* h, const double* b, double* x, double tol, int maxIT, int* its, double* resnorm);
+/* t3x_pcg from x0 = 0: x is written only */
+int t3x_pcg_zero(t3x_problem* h, const double* b, double* x, double tol, int maxIT, int* its, double* resnorm);
 /* TopOpti_ComputeUnitCompliance (579-598) */
 int t3x_compliance(t3x_problem* h, const double* U, double* ce);
 /* The load vector F_ (1315-1321; which = 0) or the displacement U_ of the
@@ -234,6 +236,9 @@ int t3x_filter(t3x_problem* h, int slot, const double* src, double* dst, int* it
 /* OC bisection (145-155): x updated in place, returns change and bisection count */
 int t3x_oc(t3x_problem* h, double* x, const double* xPhys, const double* dc, double V0, double* change,
            int* nBisect);
+/* t3x_oc with the result in another array */
+int t3x_oc_to(t3x_problem* h, const double* x, double* xNew, const double* xPhys, const double* dc, double V0,
+              double* change, int* nBisect);
 /* One MMAseq update for m = 1 (1804-2049) on the n cells of the handle:
  * xval, xold1, xold2, low, upp updated in place. */
 int t3x_mma(t3x_problem* h, int iter, double* xval, const double* xmin, const double* xmax, double* xold1,

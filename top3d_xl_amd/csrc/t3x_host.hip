@@ -20,6 +20,7 @@
 #include "t3x_pool.h"
 #include "t3x_kernels.h"
 #include "t3x_reduce.h"
+#include "t3x_stage.h"
 
 using namespace t3x;
 
@@ -248,6 +249,8 @@ struct t3x_problem {
   double* oc = nullptr;   // 8
   double* mm = nullptr;   // MM_COUNT
   double* hbuf = nullptr; // pinned read-back
+  HostStage ownStage;     // transfers of host arrays (a lent one on pooled resources)
+  HostStage* stage = &ownStage;
   // MMA state (dense cells)
   double *mx = nullptr, *mxold1 = nullptr, *mxold2 = nullptr, *mlow = nullptr, *mupp = nullptr, *malpha = nullptr,
          *mbeta = nullptr, *mp0 = nullptr, *mq0 = nullptr, *mpij = nullptr, *mqij = nullptr, *mxmin = nullptr,
@@ -265,8 +268,7 @@ struct t3x_problem {
       const size_t off = (arenaUsed + 255) & ~(size_t)255;
       if (off + nb > arenaSize) throw HipError("device memory slot exhausted (footprint estimate exceeded)");
       T* p = (T*)(arena + off);
-      T3X_HIP(hipMemsetAsync(p, 0, nb, stream));
-      T3X_HIP(hipStreamSynchronize(stream));
+      T3X_HIP(hipMemsetAsync(p, 0, nb, stream));  // all work on the array follows on this stream
       arenaUsed = off + nb;
       bytes += (long long)nb;
       return p;
@@ -334,13 +336,10 @@ struct t3x_problem {
   const uint8_t* design_mask() const { return active ? active : lv[0].emask; }
   bool standard() const { return P.vcycle == 1; }  // 'Standard' V-cycle (FP64 or, mixed, FP32)
   void sync() { T3X_HIP(hipStreamSynchronize(stream)); }
-  // Host-to-device upload ordered on the problem stream (a plain hipMemcpy from
-  // pageable memory may return before its DMA lands and is not ordered with a
-  // non-blocking stream), waited for so the host buffer may be released.
-  void upload(void* dst, const void* src, size_t bytes) {
-    T3X_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
-    sync();
-  }
+  // Host-to-device upload ordered on the problem stream; the host buffer may be
+  // released on return.
+  void upload(void* dst, const void* src, size_t bytes) { T3X_HIP(stage->to_device(dst, src, bytes, stream)); }
+  void download(void* dst, const void* src, size_t bytes) { T3X_HIP(stage->to_host(dst, src, bytes, stream)); }
 };
 
 namespace {
@@ -1437,8 +1436,7 @@ int opt_result(t3x_problem& P, t3x_result* O) {
   }
   if (O->xPhys) {
     launch_gather_compact(s, P.dCellMap, P.nCells, 1, NN, P.xPhys, P.tmp3);
-    T3X_HIP(hipMemcpyAsync(O->xPhys, P.tmp3, P.nCells * sizeof(double), hipMemcpyDeviceToHost, s));
-    P.sync();
+    P.download(O->xPhys, P.tmp3, P.nCells * sizeof(double));
   }
   O->cSolid = S.cSolid;
   O->loops = n;
@@ -1455,9 +1453,7 @@ int run(t3x_problem& P, int mode, double V0, int nLoop, double rMin, double rHat
     if (rc < 0) return -rc;
     if (O->xSnap && k < O->nSnap && P.opt.loop > k) {
       launch_gather_compact(P.stream, P.dCellMap, P.nCells, 1, P.NN(), P.xPhys, P.tmp3);
-      T3X_HIP(hipMemcpyAsync(O->xSnap + (size_t)k * P.nCells, P.tmp3, P.nCells * sizeof(double),
-                             hipMemcpyDeviceToHost, P.stream));
-      P.sync();
+      P.download(O->xSnap + (size_t)k * P.nCells, P.tmp3, P.nCells * sizeof(double));
     }
     if (rc == 1) break;
   }
@@ -1469,26 +1465,24 @@ void upload_nodal(t3x_problem& P, const double* h, double* d) {
   hipStream_t s = P.stream;
   launch_fill(s, d, 0.0, 3 * P.NN());
   double* stage = P.tmp3;  // compact staging (3*nNodes <= 3*NN)
-  T3X_HIP(hipMemcpyAsync(stage, h, 3 * (size_t)P.nNodes * sizeof(double), hipMemcpyHostToDevice, s));
+  P.upload(stage, h, 3 * (size_t)P.nNodes * sizeof(double));
   launch_scatter_compact(s, P.dNodeMap, P.nNodes, 3, P.NN(), stage, d);
 }
 void download_nodal(t3x_problem& P, const double* d, double* h) {
   hipStream_t s = P.stream;
   launch_gather_compact(s, P.dNodeMap, P.nNodes, 3, P.NN(), d, P.tmp3);
-  T3X_HIP(hipMemcpyAsync(h, P.tmp3, 3 * (size_t)P.nNodes * sizeof(double), hipMemcpyDeviceToHost, s));
-  P.sync();
+  P.download(h, P.tmp3, 3 * (size_t)P.nNodes * sizeof(double));
 }
 void upload_cells(t3x_problem& P, const double* h, double* d) {
   hipStream_t s = P.stream;
   launch_fill(s, d, 0.0, P.NN());
-  T3X_HIP(hipMemcpyAsync(P.tmp3, h, (size_t)P.nCells * sizeof(double), hipMemcpyHostToDevice, s));
+  P.upload(P.tmp3, h, (size_t)P.nCells * sizeof(double));
   launch_scatter_compact(s, P.dCellMap, P.nCells, 1, P.NN(), P.tmp3, d);
 }
 void download_cells(t3x_problem& P, const double* d, double* h) {
   hipStream_t s = P.stream;
   launch_gather_compact(s, P.dCellMap, P.nCells, 1, P.NN(), d, P.tmp3);
-  T3X_HIP(hipMemcpyAsync(h, P.tmp3, (size_t)P.nCells * sizeof(double), hipMemcpyDeviceToHost, s));
-  P.sync();
+  P.download(h, P.tmp3, (size_t)P.nCells * sizeof(double));
 }
 
 template <class F>
@@ -1522,6 +1516,7 @@ static int create_impl(const uint8_t* voxels, int nely, int nelx, int nelz, int 
     P->ownStream = false;
     P->hbuf = slot->hostBuf;
     P->ownHostBuf = false;
+    P->stage = slot->stage;
     P->oneLaunchCoarse = slot->oneLaunchCoarse;
   }
   P->nely = nely; P->nelx = nelx; P->nelz = nelz;
@@ -1895,12 +1890,14 @@ int t3x_vcycle(t3x_problem* h, const double* r, double* x) {
   });
 }
 
-int t3x_pcg(t3x_problem* h, const double* b, double* x, double tol, int maxIT, int* its, double* resnorm) {
+static int pcg_entry(t3x_problem* h, const double* b, double* x, bool zero, double tol, int maxIT, int* its,
+                     double* resnorm) {
   return guarded(h, [&] {
     if (!h->assembled) { h->err = "t3x_pcg before t3x_assemble"; return (int)T3X_ERR_INPUT; }
     if (!h->bvec) h->bvec = h->alloc<double>(3 * h->NN());
     upload_nodal(*h, b, h->bvec);
-    upload_nodal(*h, x, h->U);
+    if (zero) launch_fill(h->stream, h->U, 0.0, 3 * h->NN());
+    else upload_nodal(*h, x, h->U);
     bool warned = false;
     double res = 0.0;
     const int it = pcg_elastic(*h, h->bvec, h->U, tol, maxIT, &res, &warned);
@@ -1909,6 +1906,12 @@ int t3x_pcg(t3x_problem* h, const double* b, double* x, double tol, int maxIT, i
     if (resnorm) *resnorm = res;
     return warned ? (int)T3X_WARN_MAXIT : (int)T3X_OK;
   });
+}
+int t3x_pcg(t3x_problem* h, const double* b, double* x, double tol, int maxIT, int* its, double* resnorm) {
+  return pcg_entry(h, b, x, false, tol, maxIT, its, resnorm);
+}
+int t3x_pcg_zero(t3x_problem* h, const double* b, double* x, double tol, int maxIT, int* its, double* resnorm) {
+  return pcg_entry(h, b, x, true, tol, maxIT, its, resnorm);
 }
 
 int t3x_compliance(t3x_problem* h, const double* U, double* ce) {
@@ -1953,12 +1956,16 @@ int t3x_filter(t3x_problem* h, int slot, const double* src, double* dst, int* it
 
 int t3x_oc(t3x_problem* h, double* x, const double* xPhys, const double* dc, double V0, double* change,
            int* nBisect) {
+  return t3x_oc_to(h, x, x, xPhys, dc, V0, change, nBisect);
+}
+int t3x_oc_to(t3x_problem* h, const double* x, double* xNew, const double* xPhys, const double* dc, double V0,
+              double* change, int* nBisect) {
   return guarded(h, [&] {
     upload_cells(*h, x, h->ca);
     upload_cells(*h, xPhys, h->cb);
     upload_cells(*h, dc, h->cc);
     const double ch = oc_update(*h, h->ca, h->cb, h->cc, V0, nBisect);
-    download_cells(*h, h->ca, x);
+    download_cells(*h, h->ca, xNew);
     if (change) *change = ch;
     return (int)T3X_OK;
   });

@@ -9,6 +9,8 @@
 
 namespace t3x {
 
+class HostStage;
+
 // Device memory, stream and pinned host buffer lent to one problem: its
 // device arrays are carved out of [base, base + size) (at most the
 // t3x_footprint of the model), its work runs on `stream`, and destroying the
@@ -18,6 +20,7 @@ struct PoolSlot {
   size_t size = 0;
   hipStream_t stream = nullptr;
   double* hostBuf = nullptr;  // 256 doubles, pinned
+  HostStage* stage = nullptr;  // host transfers on `stream`
   // coarsest solve in one launch per recurrence where the process's share of
   // the device's work-group slots allows it
   bool oneLaunchCoarse = true;

@@ -27,6 +27,7 @@
 #include "../../include/t3x.h"
 #include "../../include/t3x_serve.h"
 #include "t3x_pool.h"
+#include "t3x_stage.h"
 
 namespace {
 
@@ -41,6 +42,7 @@ struct Pending {
 struct WorkerRes {
   hipStream_t stream = nullptr;
   double* hostBuf = nullptr;
+  t3x::HostStage stage;
 };
 
 struct Finished {
@@ -69,7 +71,7 @@ struct t3x_server {
 
   double now() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
   void worker();
-  void run_one(const Pending& p, const WorkerRes& w, Finished& f);
+  void run_one(const Pending& p, WorkerRes& w, Finished& f);
   static size_t rounded(long long bytes) { return ((size_t)bytes + 255) & ~(size_t)255; }
   // first free range holding `bytes`, or freeRanges.end()
   std::map<size_t, size_t>::iterator find_fit(long long bytes) {
@@ -101,7 +103,7 @@ struct t3x_server {
   }
 };
 
-void t3x_server::run_one(const Pending& p, const WorkerRes& w, Finished& f) {
+void t3x_server::run_one(const Pending& p, WorkerRes& w, Finished& f) {
   const t3x_request& r = p.req;
   const int ny = r.nely, nx = r.nelx, nz = r.nelz;
   std::vector<uint8_t> vox((size_t)ny * nx * nz, 1);
@@ -126,6 +128,7 @@ void t3x_server::run_one(const Pending& p, const WorkerRes& w, Finished& f) {
   slot.size = rounded(p.bytes);
   slot.stream = w.stream;
   slot.hostBuf = w.hostBuf;
+  slot.stage = &w.stage;
   slot.oneLaunchCoarse = true;  // bounded process-wide by device occupancy (t3x_host)
   int rc = t3x::create_pooled(vox.data(), ny, nx, nz, (int)fixN.size(), fixN.data(), fixS.data(), (int)loadN.size(),
                               loadN.data(), loadV.data(), &cfg.params, slot, &h);

@@ -1,0 +1,186 @@
+// Pinned-ring host transfers (t3x_stage.h).
+#include "t3x_stage.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+#include <cstring>
+#include <system_error>
+#include <thread>
+
+namespace t3x {
+
+struct StageJob {
+  char *dev, *host;
+  size_t bytes, chunk, chunks;
+  int slots;
+  bool up;
+  hipStream_t s;
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{0};
+  std::atomic<size_t> issued[32] = {};  // per slot: chunks sent down the stream so far
+
+  void fail(hipError_t e) {
+    int none = 0;
+    err.compare_exchange_strong(none, (int)e);
+  }
+};
+
+// 16 bytes per thread, both sides 16-byte aligned; the last n % 16 bytes by the
+// last thread
+__global__ __launch_bounds__(256) void k_stage_copy(const char* __restrict__ src, char* __restrict__ dst, unsigned n) {
+  const unsigned i = (blockIdx.x * 256 + threadIdx.x) * 16;
+  if (i + 16 <= n) *(uint4*)(dst + i) = *(const uint4*)(src + i);
+  else
+    for (unsigned j = i; j < n; ++j) dst[j] = src[j];
+}
+
+HostStage::~HostStage() {
+  if (busy_) (void)hipEventSynchronize(ev_[last_]);
+  for (hipEvent_t e : ev_)
+    if (e) (void)hipEventDestroy(e);
+  if (ring_) (void)hipHostFree(ring_);
+}
+
+// a ring for a copy of this size
+bool HostStage::reserve(size_t bytes) {
+  size_t want = kMinRing;
+  while (want < kMaxRing && want < bytes) want *= 2;
+  if (ringBytes_ >= want) return true;
+  if (failed_) return ringBytes_ > 0;
+  if (busy_ && hipEventSynchronize(ev_[last_]) != hipSuccess) return false;
+  busy_ = false;
+  char* ring = nullptr;
+  bool ok = hipHostMalloc((void**)&ring, want, hipHostMallocCoherent) == hipSuccess;
+  for (hipEvent_t& e : ev_)
+    if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (!ok) {  // the ring that is there, if any, serves on
+    (void)hipGetLastError();
+    if (ring) (void)hipHostFree(ring);
+    failed_ = true;
+    return ringBytes_ > 0;
+  }
+  if (ring_) (void)hipHostFree(ring_);
+  ring_ = ring;
+  ringBytes_ = want;
+  return true;
+}
+
+// Chunk c between its slot and the device, and the slot's event behind it
+// where somebody waits for it.
+hipError_t HostStage::issue(StageJob& job, size_t c) {
+  const int slot = (int)(c % job.slots);
+  char *dev = job.dev + c * job.chunk, *pin = ring_ + slot * job.chunk;
+  const size_t n = std::min(job.chunk, job.bytes - c * job.chunk);
+  hipError_t e = hipSuccess;
+  if ((uintptr_t)dev % 16 == 0) {
+    hipLaunchKernelGGL(k_stage_copy, dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0, job.s, job.up ? pin : dev,
+                       job.up ? dev : pin, (unsigned)n);
+    e = hipGetLastError();
+  } else {
+    e = hipMemcpyAsync(job.up ? dev : pin, job.up ? pin : dev, n, job.up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost,
+                       job.s);
+  }
+  if (e == hipSuccess && (!job.up || c + job.slots < job.chunks)) e = hipEventRecord(ev_[slot], job.s);
+  job.issued[slot].store(c / job.slots + 1, std::memory_order_release);
+  return e;
+}
+
+// One thread's share: the next chunk that no thread has taken, one after the
+// other.  An upload fills the chunk's slot once the chunk before it in that
+// slot has left it; a download waits for the chunk, empties the slot and sends
+// the next chunk of that slot.
+hipError_t HostStage::part(StageJob& job) {
+  for (;;) {
+    const size_t c = job.next.fetch_add(1, std::memory_order_relaxed);
+    if (c >= job.chunks || job.err.load(std::memory_order_relaxed)) return hipSuccess;
+    const int slot = (int)(c % job.slots);
+    const size_t round = c / job.slots + (job.up ? 0 : 1);
+    while (job.issued[slot].load(std::memory_order_acquire) < round) {  // by the thread that had the slot before
+      if (job.err.load(std::memory_order_relaxed)) return hipSuccess;
+      std::this_thread::yield();
+    }
+    char *host = job.host + c * job.chunk, *pin = ring_ + slot * job.chunk;
+    const size_t n = std::min(job.chunk, job.bytes - c * job.chunk);
+    hipError_t e = round ? hipEventSynchronize(ev_[slot]) : hipSuccess;
+    if (e != hipSuccess) return e;
+    if (job.up) {
+      std::memcpy(pin, host, n);
+      e = issue(job, c);
+    } else {
+      std::memcpy(host, pin, n);
+      if (c + job.slots < job.chunks) e = issue(job, c + job.slots);
+    }
+    if (e != hipSuccess) return e;
+  }
+}
+
+hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStream_t s) {
+  const size_t chunk = chunk_of(bytes);
+  StageJob job{dev, host, bytes, chunk, (bytes + chunk - 1) / chunk, (int)std::min<size_t>(ringBytes_ / chunk, kMaxSlots),
+               up, s};
+  static_assert(sizeof(job.issued) / sizeof(job.issued[0]) == kMaxSlots, "a count per slot");
+  hipError_t e = hipSuccess;
+  if (up && busy_) e = hipEventSynchronize(ev_[last_]);  // (a download follows it on the stream)
+  if (e != hipSuccess) return e;
+  if (!up)
+    for (size_t c = 0; e == hipSuccess && c < std::min<size_t>(job.chunks, job.slots); ++c) e = issue(job, c);
+  int device = 0;
+  const int nt = hipGetDevice(&device) == hipSuccess ? threads_of(bytes) : 1;
+  std::thread th[kMaxThreads];
+  auto run = [&](int t) {
+    hipError_t r = t ? hipSetDevice(device) : e;
+    if (r == hipSuccess) r = part(job);
+    if (r != hipSuccess) job.fail(r);
+  };
+  if (e == hipSuccess) {
+    try {
+      for (int t = 1; t < nt; ++t) th[t] = std::thread(run, t);
+    } catch (const std::system_error&) {  // no more threads: those that run take all chunks
+    }
+  }
+  run(0);
+  for (std::thread& t : th)
+    if (t.joinable()) t.join();
+  e = (hipError_t)job.err.load();
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);  // no slot is left to a chunk in flight
+    busy_ = false;
+    return e;
+  }
+  if (up) {
+    last_ = (int)((job.chunks - 1) % job.slots);
+    e = hipEventRecord(ev_[last_], s);
+    busy_ = e == hipSuccess;
+  } else {
+    busy_ = false;
+  }
+  return e;
+}
+
+// Memory that the runtime knows (pinned, registered, managed, device) is at
+// the link's rate without the ring.
+static bool plain_memory(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
+hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  if (bytes == 0) return hipSuccess;
+  if (plain_memory(src) && reserve(bytes)) return move((char*)dst, (char*)src, bytes, true, s);
+  const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
+hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  if (bytes == 0) return hipSuccess;
+  if (plain_memory(dst) && reserve(bytes)) return move((char*)src, (char*)dst, bytes, false, s);
+  const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
+}  // namespace t3x

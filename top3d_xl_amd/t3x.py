@@ -97,12 +97,13 @@ def load_library():
     L.t3x_assemble.argtypes = [vp]
     L.t3x_apply_K.argtypes = [vp, _dp, _dp]
     L.t3x_vcycle.argtypes = [vp, _dp, _dp]
-    L.t3x_pcg.argtypes = [vp, _dp, _dp, C.c_double, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]
+    L.t3x_pcg.argtypes = L.t3x_pcg_zero.argtypes = [vp, _dp, _dp, C.c_double, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]
     L.t3x_compliance.argtypes = [vp, _dp, _dp]
     L.t3x_get_nodal.argtypes = [vp, C.c_int, C.c_int, _dp]
     L.t3x_filter_setup.argtypes = [vp, C.c_int, C.c_double]
     L.t3x_filter.argtypes = [vp, C.c_int, _dp, _dp, C.POINTER(C.c_int)]
     L.t3x_oc.argtypes = [vp, _dp, _dp, _dp, C.c_double, C.POINTER(C.c_double), C.POINTER(C.c_int)]
+    L.t3x_oc_to.argtypes = [vp, _dp, _dp, _dp, _dp, C.c_double, C.POINTER(C.c_double), C.POINTER(C.c_int)]
     L.t3x_mma.argtypes = [vp, C.c_int, _dp, _dp, _dp, _dp, _dp, _dp, C.c_double, _dp, _dp, _dp,
                           C.POINTER(C.c_int)]
     L.t3x_footprint.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(Params), C.c_int,
@@ -127,8 +128,8 @@ def load_library():
 
 EXPORTED = ["t3x_default_params", "t3x_create", "t3x_create_multi", "t3x_num_load_cases", "t3x_destroy", "t3x_last_error", "t3x_info", "t3x_run",
             "t3x_opt_begin", "t3x_opt_step", "t3x_opt_result", "t3x_kernel_time", "t3x_kernel_time_reset",
-            "t3x_set_modulus", "t3x_assemble", "t3x_apply_K", "t3x_vcycle", "t3x_pcg", "t3x_compliance", "t3x_get_nodal",
-            "t3x_filter_setup", "t3x_filter", "t3x_oc", "t3x_mma", "t3x_footprint", "t3x_memory", "t3x_stream_copy", "t3x_set_passive",
+            "t3x_set_modulus", "t3x_assemble", "t3x_apply_K", "t3x_vcycle", "t3x_pcg", "t3x_pcg_zero", "t3x_compliance", "t3x_get_nodal",
+            "t3x_filter_setup", "t3x_filter", "t3x_oc", "t3x_oc_to", "t3x_mma", "t3x_footprint", "t3x_memory", "t3x_stream_copy", "t3x_set_passive",
             "t3x_set_passive_layers", "t3x_get_passive",
             "t3x_server_create", "t3x_server_submit", "t3x_server_poll", "t3x_server_release",
             "t3x_server_stats", "t3x_server_destroy", "t3x_oc_noalloc"]
@@ -220,43 +221,44 @@ class Problem:
         self._check(self.L.t3x_assemble(self.h))
 
     def apply_K(self, u):
-        y = np.zeros(3 * self.nN)
+        y = np.empty(3 * self.nN)  # result arrays are written whole
         self._check(self.L.t3x_apply_K(self.h, np.ascontiguousarray(u, dtype=np.float64), y))
         return y
 
     def vcycle(self, r):
-        x = np.zeros(3 * self.nN)
+        x = np.empty(3 * self.nN)
         self._check(self.L.t3x_vcycle(self.h, np.ascontiguousarray(r, dtype=np.float64), x))
         return x
 
     def pcg(self, b, x0=None, tol=1e-3, maxit=800):
-        x = np.zeros(3 * self.nN) if x0 is None else np.array(x0, dtype=np.float64)
+        x = np.empty(3 * self.nN) if x0 is None else np.array(x0, dtype=np.float64)
+        solve = self.L.t3x_pcg_zero if x0 is None else self.L.t3x_pcg
         its = C.c_int(0)
         res = C.c_double(0.0)
-        self._check(self.L.t3x_pcg(self.h, np.ascontiguousarray(b, dtype=np.float64), x, tol, maxit,
-                                   C.byref(its), C.byref(res)))
+        self._check(solve(self.h, np.ascontiguousarray(b, dtype=np.float64), x, tol, maxit, C.byref(its),
+                          C.byref(res)))
         return x, its.value, res.value
 
     def compliance(self, U):
-        ce = np.zeros(self.nE)
+        ce = np.empty(self.nE)
         self._check(self.L.t3x_compliance(self.h, np.ascontiguousarray(U, dtype=np.float64), ce))
         return ce
 
     def load_vector(self, case=0):
         """F_ of a load case (t3x_get_nodal), compact interleaved nodal order."""
-        out = np.zeros(3 * self.nN)
+        out = np.empty(3 * self.nN)
         self._check(self.L.t3x_get_nodal(self.h, 0, int(case), out))
         return out
 
     def displacement(self, case=0):
         """U_ of a load case after the last solve (t3x_get_nodal)."""
-        out = np.zeros(3 * self.nN)
+        out = np.empty(3 * self.nN)
         self._check(self.L.t3x_get_nodal(self.h, 1, int(case), out))
         return out
 
     def xphys(self):
         """The current physical densities (t3x_opt_result), compact cell order."""
-        x = np.zeros(self.nE)
+        x = np.empty(self.nE)
         R = Result(x.ctypes.data, None, None, None, None, None, None, None, 0, None, 0.0, 0, 0)
         self._check(self.L.t3x_opt_result(self.h, C.byref(R)))
         return x
@@ -265,18 +267,22 @@ class Problem:
         self._check(self.L.t3x_filter_setup(self.h, slot, float(r)))
 
     def filter(self, slot, src):
-        dst = np.zeros(self.nE)
+        dst = np.empty(self.nE)
         its = C.c_int(0)
         self._check(self.L.t3x_filter(self.h, slot, np.ascontiguousarray(src, dtype=np.float64), dst,
                                       C.byref(its)))
         return dst, its.value
 
     def oc(self, x, xPhys, dc, V0):
-        xx = np.array(x, dtype=np.float64)
+        x = np.asarray(x, dtype=np.float64)
+        if not x.flags.c_contiguous:
+            x = np.array(x)
+        xx = np.empty(x.shape)
         ch = C.c_double(0.0)
         nb = C.c_int(0)
-        self._check(self.L.t3x_oc(self.h, xx, np.ascontiguousarray(xPhys, dtype=np.float64),
-                                  np.ascontiguousarray(dc, dtype=np.float64), float(V0), C.byref(ch), C.byref(nb)))
+        self._check(self.L.t3x_oc_to(self.h, x, xx, np.ascontiguousarray(xPhys, dtype=np.float64),
+                                     np.ascontiguousarray(dc, dtype=np.float64), float(V0), C.byref(ch),
+                                     C.byref(nb)))
         return xx, ch.value, nb.value
 
     def mma(self, iter_, xval, xmin, xmax, xold1, xold2, dfdx, gx, dgdx, low, upp):
@@ -338,7 +344,7 @@ class Problem:
     def run(self, mode, V0, nLoop, rMin, rHat=0.0, nSnap=0):
         nE = self.nE
         n = max(nLoop, 1)
-        xPhys = np.zeros(nE)
+        xPhys = np.empty(nE)
         nc = self.num_cases
         cH, vH, conH, sH = (np.zeros(n) for _ in range(4))
         its = np.zeros(n * nc, dtype=np.int32)
