@@ -138,14 +138,16 @@ __device__ __forceinline__ void tile16_syrk(double (*sC)[TB + 1], const double (
 // caller's side work (side(w, b) on waves w = 1 .. PW - 1 while panel b is
 // factored; the columns before it are final) run while wave 0 factors on.  The
 // upper halves of the diagonal tiles are updated too and never read.
-// Bound: the latency chain of 64 pivots (broadcast, reciprocal square root,
-// scale, update of the next column); the updates of the columns after that fill
-// its waits, their factors broadcast through LDS (7.2 us a tile; all of them by
-// readlane 8.0).
+// The next pivot is formed in every lane from entries broadcast before this
+// column is scaled (the same product and update as in its own lane), so no
+// broadcast lies on the chain from pivot to pivot; scaled columns go to sA as
+// they are finished, and the factors of the updates further right are read back
+// from there.  Bound: instruction issue of the one wave, 185 cycles a column
+// (about 40 instructions at 4 to 5 cycles each; the chain itself, reciprocal
+// square root, scale and update, is 64).
 template <class Side>
 __device__ __forceinline__ void tile_potrf(double (*sA)[TB + 1], double (*sD)[16][17], int* status, Side side) {
   constexpr int PB = 16;
-  __shared__ double sC[2][TB];  // wave 0's columns, for broadcasts
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kq = lane >> 4;
   // the rank-16 update of panel b on 16x16 tile (I, J)
   auto update = [&](int b, int I, int J) {
@@ -169,33 +171,60 @@ __device__ __forceinline__ void tile_potrf(double (*sA)[TB + 1], double (*sD)[16
       bool bad = false;
       double piv = readlane_d(p[0], b0);
       double rs = rsqrt_nr(piv);
+      // this column's entries (b0 + k + 1, k), (b0 + k + 2, k) before scaling and
+      // the next diagonal entry before this column's update, in every lane
+      double a1 = readlane_d(p[0], b0 + 1), a2 = readlane_d(p[0], b0 + 2), d1 = readlane_d(p[1], b0 + 1);
       double c[PB] = {};  // column k - 1's entries (b0 + kk, k - 1), kk >= k + 2
 #pragma unroll
       for (int k = 0; k < PB; ++k) {
         bad |= !(piv > 0.0);
-        p[k] *= rs;  // the pivot's lane gets sqrt(piv), lanes below L(i, c)
-        sC[k & 1][lane] = p[k];
-        wave_lds_fence();
-        auto rank1 = [&](int kk) { p[kk] = fma(-p[k], readlane_d(p[k], b0 + kk), p[kk]); };
-        if (k + 1 < PB) {
-          rank1(k + 1);
-          piv = readlane_d(p[k + 1], b0 + k + 1);
-          const double y = __builtin_amdgcn_rsq(piv);  // rsqrt_nr(piv) for the next column
-          if (k > 0) {
-#pragma unroll
-            for (int kk = k + 2; kk < PB; ++kk) p[kk] = fma(-p[k - 1], c[kk], p[kk]);
-          }
-          if (k + 2 < PB) rank1(k + 2);
-#pragma unroll
-          for (int kk = k + 3; kk < PB; ++kk) c[kk] = sC[k & 1][b0 + kk];
-          const double h = fma(-piv * y, y, 1.0);
-          rs = fma(y * h, 0.5, y);
+        const double l1 = a1 * rs;
+        if (k + 1 == PB) {
+          p[k] *= rs;
+          break;
         }
-      }
-      if (lane >= b0) {  // (entries right of the diagonal are never read)
+        piv = fma(-l1, l1, d1);  // what the update below leaves in the next pivot's lane
+        const double y = __builtin_amdgcn_rsq(piv);  // rsqrt_nr(piv) for the next column
+        __builtin_amdgcn_sched_barrier(0);
+        p[k] *= rs;               // the pivot's lane gets sqrt(piv), lanes below L(i, c)
+        sA[lane][b0 + k] = p[k];  // (entries right of the diagonal are never read)
+        wave_lds_fence();
+        double cn[PB] = {};
 #pragma unroll
-        for (int k = 0; k < PB; ++k) sA[lane][b0 + k] = p[k];
+        for (int kk = k + 3; kk < PB; ++kk) cn[kk] = sA[b0 + kk][b0 + k];
+        __builtin_amdgcn_sched_barrier(0);
+        auto upd = [&](int kk) {  // column k - 1 on column kk
+          if (k > 0) p[kk] = fma(-p[k - 1], c[kk], p[kk]);
+        };
+        p[k + 1] = fma(-p[k], l1, p[k + 1]);
+        if (k + 2 < PB) {
+          const double l2 = a2 * rs;
+          upd(k + 2);
+          p[k + 2] = fma(-p[k], l2, p[k + 2]);
+          a1 = readlane_d(p[k + 1], b0 + k + 2);
+          if (k + 3 < PB) a2 = readlane_d(p[k + 1], b0 + k + 3);
+          d1 = readlane_d(p[k + 2], b0 + k + 2);
+        }
+        // the reciprocal square root's chain, other columns' updates in its waits
+        const int m = (PB - k - 3 + 3) / 4;
+        auto fill = [&](int q) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = k + 3 + q * m; kk < PB && kk < k + 3 + (q + 1) * m; ++kk) upd(kk);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        const double t = -piv * y;
+        fill(0);
+        const double h = fma(t, y, 1.0);
+        fill(1);
+        const double yh = y * h;
+        fill(2);
+        rs = fma(yh, 0.5, y);
+        fill(3);
+#pragma unroll
+        for (int kk = k + 3; kk < PB; ++kk) c[kk] = cn[kk];
       }
+      sA[lane][b0 + PB - 1] = p[PB - 1];
       if (bad && lane == 0) *status = 1;
     } else {
       if (b > 0) {  // the rest of panel b - 1's update: tiles right of this panel
@@ -423,9 +452,9 @@ __global__ __launch_bounds__(FT) void k_chol_diag(BandView V, int d0, double* __
 // Bound: group (0, 0)'s latency chain; all it does but that chain (the tiles
 // of X X^T past the first 16 columns, L(I, J) to the scratch panel, the
 // inverses, the stores of finished columns) runs beside the pivots.  20.9 ->
-// 15.9 us a launch at 128x256x128 and 256x512x256 (20.3 -> 14.4 at 50x100x50);
+// 15.3 us a launch at 128x256x128 (20.3 -> 14.0 at 50x100x50, 14.3 at 96x192x96);
 // its parts there, with four waves and in sequence / now: staging 3.6 / 2.3,
-// inverses and substitution 3.3 / 2.7, product 3.0 / 0.75, pivots 8.0 / 7.4,
+// inverses and substitution 3.3 / 2.7, product 3.0 / 0.75, pivots 8.0 / 6.8,
 // store 1.6 / 0.4 us.
 __global__ __launch_bounds__(FT) void k_chol_panel(BandView V, int J, int nrt, int nrtPrev, double* __restrict__ pan,
                                                    int panStride, int* status) {
