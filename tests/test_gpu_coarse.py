@@ -64,3 +64,29 @@ def test_one_launch_equals_a_launch_per_block():
         assert not one  # the last, largest one does not
     finally:
         hog.close()
+
+
+# everything in one launch (SB 128), and a launch per direction with even and odd numbers of blocks
+@pytest.mark.parametrize("shape,handles", [((20, 17, 60), 41), ((104, 208, 104), 9), ((96, 192, 96), 9)], ids=str)
+def test_handles_on_two_sets_one_set_and_none_agree(shape, handles):
+    """Above SB 512 the first handle of a process takes a recurrence's blocks with
+    two sets of work-groups in turn, later ones with one set, those beyond the
+    device's capacity with a launch per block: the same bits."""
+    import top3d_xl_amd as t3x
+    ms = [t3x.Problem(np.ones(shape, bool)) for _ in range(handles)]
+    try:
+        rng = np.random.default_rng(7)
+        E = 1e-6 + rng.random(ms[0].nE) ** 3
+        r = rng.standard_normal((3, 3 * ms[0].nN))
+        r[1, ::7] = 0.0
+        first = None
+        for m in ms:
+            m.set_modulus(E)
+            m.assemble()
+            z = [m.vcycle(v) for v in r]  # (the words' two places, in turn)
+            first = first or z
+            assert all(np.array_equal(a, b) for a, b in zip(z, first))
+        print(f"\n[gpu-coarse] {shape}: {sum(m.one_launch_coarse for m in ms)} of {handles} in one launch", flush=True)
+    finally:
+        for m in ms:
+            m.close()

@@ -8,13 +8,14 @@
 namespace t3x {
 
 // Device words of the one-launch recurrences (k_solve_chain, k_solve_fused),
-// zeroed at set-up: per work-group the tag its next launch starts from (equal
-// across the groups between launches), and a failure word set when a wait
-// expired (cleared by the host).
+// zeroed at set-up: per work-group the number of solves so far (equal across
+// the groups between solves), and a failure word set when a wait expired (it
+// stays set).
 constexpr int kChainMaxSB = 2048;             // largest solve block of the one-launch recurrences
+constexpr int kFusedMaxSB = 512;              // largest solved whole in one launch
 constexpr int kChainMaxWG = kChainMaxSB / 4;  // their work-groups at most
 struct ChainState {
-  unsigned tag[kChainMaxWG];
+  unsigned turn[kChainMaxWG];
   int fail;
   int pad[3];
 };
@@ -26,6 +27,8 @@ struct CoarseSolver {
   int np = 0;    // padded order (multiple of SB)
   int nblk = 0;  // np / SB
   ChainState* chain = nullptr;  // device words of the one-launch recurrences (null: a launch per block)
+  int sets = 1;  // of work-groups that take the blocks of a recurrence in turn (k_solve_chain)
+  bool sets_apply() const { return SB > kFusedMaxSB && SB <= kChainMaxSB / 2; }
   bool one_launch() const { return chain && SB <= kChainMaxSB; }
   // parts per million of the current device's work-group slots (its
   // occupancy for the recurrences' registers and LDS) that one launch of the
@@ -44,7 +47,7 @@ struct CoarseSolver {
   // FP64 solve; the right-hand side is gathered from / the solution scattered
   // to dense level vectors of either precision.  va, vb: np doubles each (a
   // launch per block) or 3 np (one launch per recurrence: np doubles, then
-  // 2 np tagged words).
+  // 2 np words, zero before the first solve).
   void solve(hipStream_t s, const long long* map, const double* rdense, double* xdense, const double* Dinv,
              const double* DT, const double* Gm, const double* H, double* va, double* vb, const int* fl) const;
   void solve(hipStream_t s, const long long* map, const float* rdense, float* xdense, const double* Dinv,

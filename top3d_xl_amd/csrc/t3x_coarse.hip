@@ -21,7 +21,7 @@
 //     Dinv_b, G_b come from one batched blocked TRSM on [I | L_{b,b-1}],
 //     H_b from a batched GEMM.
 //  3. the two recurrences in one or two launches whose work-groups hand the
-//     blocks on through tagged words, or as a chain of 2*nblk+1 small launches,
+//     blocks on entry by entry, or as a chain of 2*nblk+1 small launches,
 //     instead of one dependent step per 64 rows.
 //
 // Everything else synchronises at kernel boundaries: on MI355X a device-wide barrier inside a kernel (cooperative grid sync, or fences that
@@ -768,116 +768,131 @@ __global__ void k_solve_scatter(int n, const long long* __restrict__ map, const 
 // ---- 3b. the recurrences without a launch per block ------------------------
 // A launch per block costs ~7.5 us of dispatch, ramp and drain against
 // ~1.5 us of data.  Here one launch per recurrence (forward after
-// k_solve_f0, backward after k_solve_b0) walks all its blocks: G work-groups
-// of 4 waves, wave w of the grid owning row w of every block.  A block's rows
-// carry their own readiness: each FP64 entry travels as two 64-bit words (32
-// bits of the value, 32 bits of tag), written with agent-scope stores
-// (coherent across the XCDs' L2s), and a group that needs block b - 1
-// (forward) or b + 1 (backward) polls those words until every entry shows the
-// tag of that block in this launch.  The row of G_b (or H_b) and the row's
-// own term for the next block are loaded right after a block is written, so
-// they arrive while the group waits; a step is then one poll, one 64-lane dot
-// product and one store.  Tags: a launch pair takes its first tag from
-// ChainState (the backward launch advances every group's word by nblk),
-// block b carries first + b + 1 forward and first + nblk - b backward, so
-// words left by an earlier launch never match.  All G = ceil(SB / 4) groups
-// must be resident together: 4 waves and SB doubles of LDS each, far below
-// the device's capacity.  Each wait is bounded: after kChainSpin polls the
-// launch sets fail, every group stops waiting (the solve is then garbage) and
-// the caller reports the error.  Measured alternatives (same operators):
-// one launch for everything with a published count per block, 7.6 us per
-// block; the same with an agent-scope release/acquire pair, which writes back
-// and invalidates the L2, 30 us per block.
+// k_solve_f0, backward after k_solve_b0) walks all its blocks.  The work-groups
+// form SETS sets that take the blocks in turn; a set's groups of 4 waves own
+// all SB rows of its blocks, SETS rows per wave.  A block's rows carry their
+// own readiness: an entry is one 64-bit word, written with an agent-scope store
+// (coherent across the XCDs' L2s), and a group that needs the block before
+// polls its words until none is unset.  Every vector has two places, for
+// launches in turn (ChainState's count, advanced by the backward launch); the
+// rows' owners clear the other one, which the launch before filled and nobody
+// reads any more.  (Words of half a value and a tag each, 2 SB of them a block,
+// took 2 us more of 60 a recurrence.)
+// Bound: with one set, a block's hand-over (1.5 us) and then its operator rows
+// (7.4 MB at SB 960, 1.6 us from HBM): a group asks for its next rows when its
+// block is written, and loads return in order, so its polls see nothing before
+// those rows are there.  (Asked for ahead of the product instead, in a second
+// register set, they delay the store: 89 against 53 us a recurrence.)  With two
+// sets one set's rows arrive while the other one's block is formed: 62.9 ->
+// 48.3 us forward, 58.2 -> 49.5 us backward at 128x256x128 (18 blocks), 53 ->
+// 46 us at 96x192x96.  480 groups of one row per wave: 49 us and twice the
+// share of the device; 3 or 4 sets 53 to 72 us.
+// All groups must be resident together: 4 waves and SB doubles of LDS each, far
+// below the device's capacity; two sets keep to 128 registers for that (a
+// share of 23.4% of the device at SB 960, one set 18.8%).  Each wait is bounded:
+// after kChainSpin polls the launch sets fail, every group stops waiting (the
+// solve is then garbage) and the caller reports the error; fail stays set.
+// Measured alternatives (same operators): one launch for everything with a
+// published count per block, 7.6 us per block; the same with an agent-scope
+// release/acquire pair, which writes back and invalidates the L2, 30 us.
 constexpr unsigned kChainSpin = 1u << 20;  // polls per wait (~1 s) before the launch gives up
 
-__device__ __forceinline__ double chain_wave_sum(double s) {
-  return wave_sum(s);
+// An entry of an exchanged vector is one word: the value's bits with this
+// signalling NaN's taken off (exclusive or), so 0 is "not there yet": a value
+// formed by arithmetic is never a signalling NaN.
+constexpr unsigned long long kUnset = 0x7FF0000000000001ull;
+__device__ __forceinline__ void chain_put(unsigned long long* w, double v) {
+  __hip_atomic_store(w, (unsigned long long)__double_as_longlong(v) ^ kUnset, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
-// entry i of a tagged vector: words 2i (high half of the value) and 2i + 1 (low half)
-__device__ __forceinline__ void chain_put(unsigned long long* w, int i, double v, unsigned tag) {
-  const unsigned long long d = (unsigned long long)__double_as_longlong(v);
-  __hip_atomic_store(w + 2 * i, (d & 0xFFFFFFFF00000000ull) | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(w + 2 * i + 1, (d << 32) | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void chain_clear(unsigned long long* w) {
+  __hip_atomic_store(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ unsigned long long chain_get(const unsigned long long* w) {
+  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double chain_value(unsigned long long w) { return __longlong_as_double((long long)(w ^ kUnset)); }
 
 // FWD: y_b = a_b - G_b y_{b-1} (a = Dinv_b v_b from k_solve_f0, overwritten
 // by y for k_solve_b0); backward: x_b = a_b - H_b x_{b+1} (a = Dinv_b^T y_b
 // from k_solve_b0), scattered to xdense as formed.  PT: block entries per
 // thread (SB <= PT * CT).
-template <typename TV, int PT, bool FWD>
-__global__ __launch_bounds__(CT) void k_solve_chain(int n, int SB, int nblk, const long long* __restrict__ map,
+template <typename TV, int PT, int SETS, bool FWD>
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(SETS == 2 ? 4 : 1))) void k_solve_chain(int n, int SB, int nblk, const long long* __restrict__ map,
                                                     TV* __restrict__ xdense, const double* __restrict__ M,
                                                     double* __restrict__ a, unsigned long long* W, ChainState* st,
                                                     const int* fl) {
   if (fl && fl[FL_DONE]) return;
   constexpr int NCH = PT * CT / 64;  // 64-column chunks of a row
+  constexpr int RPW = SETS;          // rows per wave: the grid is as large in either form
   extern __shared__ double chainNbr[];  // the neighbour block
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (CT / 64) + (threadIdx.x >> 6);
-  const bool act = row < SB;
-  const unsigned tag0 = st->tag[blockIdx.x];  // written by this group's previous backward launch
-  auto tag_of = [&](int b) { return FWD ? tag0 + b + 1 : tag0 + (nblk - b); };
-  const int step = FWD ? 1 : -1;
-  auto in_range = [&](int b) { return b >= 0 && b < nblk; };
-  double rg[NCH], ab = 0.0;
-  auto prefetch = [&](int b) {  // row of M_b and this row's own term, all loads in flight together
-    const double* m = M + ((size_t)b * SB + row) * SB;
+  const int set = blockIdx.x % SETS;
+  const int row0 = (blockIdx.x / SETS * (CT / 64) + (threadIdx.x >> 6)) * RPW;  // RPW divides SB
+  const int mine = row0 + min(lane, RPW - 1);  // the row whose entry this lane stores (lanes < RPW)
+  const bool act = row0 < SB;
+  const unsigned turn = st->turn[blockIdx.x];  // advanced by this group's previous backward launch
+  unsigned long long *Wn = W + (size_t)(turn & 1) * nblk * SB, *Wo = W + (size_t)(~turn & 1) * nblk * SB;
+  auto block_at = [&](int k) { return FWD ? k : nblk - 1 - k; };  // the k-th block of the recurrence
+  double rg[RPW][NCH], ab = 0.0;
+  long long to = 0;  // where the entry goes (read with the row: the store must not wait for it)
+  auto load_own = [&](int b) {
+    ab = a[(size_t)b * SB + mine];
+    if (!FWD) to = map[min(b * SB + mine, n - 1)];
+  };
+  auto prefetch = [&](int b) {  // rows of M_b and their own terms, all loads in flight together
+    const double* m = M + ((size_t)b * SB + row0) * SB;
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int j = lane + 64 * c;
-      rg[c] = j < SB ? m[j] : 0.0;
-    }
-    ab = a[(size_t)b * SB + row];
+    for (int r = 0; r < RPW; ++r)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const int j = lane + 64 * c;
+        rg[r][c] = j < SB ? m[(size_t)r * SB + j] : 0.0;
+      }
+    load_own(b);
   };
   auto emit = [&](int b, double v) {
-    const int g = b * SB + row;
-    chain_put(W, g, v, tag_of(b));
+    if (lane >= RPW) return;
+    const int g = b * SB + mine;
+    chain_put(Wn + g, v);
     if (FWD) a[g] = v;
-    else if (g < n) xdense[map[g]] = (TV)v;
+    else if (g < n) xdense[to] = (TV)v;
+    chain_clear(Wo + g);
   };
-  // the first block is its own term
-  int b = FWD ? 0 : nblk - 1;
-  if (act) {
-    ab = a[(size_t)b * SB + row];
-    if (lane == 0) emit(b, ab);
+  int k = set;
+  if (act && k == 0) {  // the first block is its own term
+    load_own(block_at(0));
+    emit(block_at(0), ab);
   }
-  b += step;
-  if (in_range(b) && act) prefetch(b);
-  for (; in_range(b); b += step) {
-    {  // block b - step into LDS once every entry carries its tag
-      const int nb = b - step;
-      const unsigned tag = tag_of(nb);
+  if (k == 0) k = SETS;
+  if (act && k < nblk) prefetch(block_at(k));
+  for (; k < nblk; k += SETS) {
+    {  // the block before into LDS once every entry is there
+      const unsigned long long* w0 = Wn + block_at(k - 1) * SB;
       unsigned pending = 0;
 #pragma unroll
-      for (int k = 0; k < PT; ++k)
-        if (threadIdx.x + k * CT < SB) pending |= 1u << k;
-      double v[PT];
+      for (int u = 0; u < PT; ++u)
+        if ((int)threadIdx.x + u * CT < SB) pending |= 1u << u;
       unsigned polls = 0;
       while (pending) {
-        unsigned long long hi[PT], lo[PT];
+        unsigned long long w[PT];
 #pragma unroll
-        for (int k = 0; k < PT; ++k)
-          if (pending & (1u << k)) {
-            const int i = nb * SB + threadIdx.x + k * CT;
-            hi[k] = __hip_atomic_load(W + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lo[k] = __hip_atomic_load(W + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
+        for (int u = 0; u < PT; ++u)
+          if (pending & (1u << u)) w[u] = chain_get(w0 + threadIdx.x + u * CT);
 #pragma unroll
-        for (int k = 0; k < PT; ++k)
-          if ((pending & (1u << k)) && (unsigned)hi[k] == tag && (unsigned)lo[k] == tag) {
-            v[k] = __longlong_as_double((long long)((hi[k] & 0xFFFFFFFF00000000ull) | (lo[k] >> 32)));
-            pending &= ~(1u << k);
+        for (int u = 0; u < PT; ++u)
+          if ((pending & (1u << u)) && w[u]) {
+            chainNbr[threadIdx.x + u * CT] = chain_value(w[u]);
+            pending &= ~(1u << u);
           }
         if (!pending) break;
+        // (given up: what is left in chainNbr makes the solve garbage, as reported)
         if (__hip_atomic_load(&st->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
         if (++polls > kChainSpin) {
           __hip_atomic_store(&st->fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           break;
         }
       }
-#pragma unroll
-      for (int k = 0; k < PT; ++k)
-        if (threadIdx.x + k * CT < SB) chainNbr[threadIdx.x + k * CT] = (pending & (1u << k)) ? 0.0 : v[k];
     }
     __syncthreads();
     if (act) {
@@ -885,30 +900,35 @@ __global__ __launch_bounds__(CT) void k_solve_chain(int n, int SB, int nblk, con
       // chunk quadruples while the whole quadruple is in the row, then the
       // remaining chunks into the first), so the result is bitwise that of
       // k_solve_step
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-      bool quad = true;
+      double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < NCH / 4; ++q) {
-        const int j = lane + 256 * q;
-        quad = quad && j + 192 < SB;
-        if (quad) {
-          s0 = fma(rg[4 * q], chainNbr[j], s0);
-          s1 = fma(rg[4 * q + 1], chainNbr[j + 64], s1);
-          s2 = fma(rg[4 * q + 2], chainNbr[j + 128], s2);
-          s3 = fma(rg[4 * q + 3], chainNbr[j + 192], s3);
-        } else {
+      for (int r = 0; r < RPW; ++r) {
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        bool quad = true;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (j + 64 * r < SB) s0 = fma(rg[4 * q + r], chainNbr[j + 64 * r], s0);
+        for (int q = 0; q < NCH / 4; ++q) {
+          const int j = lane + 256 * q;
+          quad = quad && j + 192 < SB;
+          if (quad) {
+            s0 = fma(rg[r][4 * q], chainNbr[j], s0);
+            s1 = fma(rg[r][4 * q + 1], chainNbr[j + 64], s1);
+            s2 = fma(rg[r][4 * q + 2], chainNbr[j + 128], s2);
+            s3 = fma(rg[r][4 * q + 3], chainNbr[j + 192], s3);
+          } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (j + 64 * u < SB) s0 = fma(rg[r][4 * q + u], chainNbr[j + 64 * u], s0);
+          }
         }
+        const double t = wave_sum((s0 + s1) + (s2 + s3));
+        if (lane == r) s = t;
       }
-      const double s = ab - chain_wave_sum((s0 + s1) + (s2 + s3));
-      if (lane == 0) emit(b, s);
-      if (in_range(b + step)) prefetch(b + step);
+      emit(block_at(k), ab - s);
+      if (k + SETS < nblk) prefetch(block_at(k + SETS));
     }
     __syncthreads();  // chainNbr free
   }
-  if (!FWD && threadIdx.x == 0) st->tag[blockIdx.x] = tag0 + nblk;
+  if (!FWD && threadIdx.x == 0) st->turn[blockIdx.x] = turn + 1;
 }
 
 // SB <= kFusedMaxSB: the own terms and both recurrences in one launch.  The
@@ -917,21 +937,21 @@ __global__ __launch_bounds__(CT) void k_solve_chain(int n, int SB, int nblk, con
 // back's (DT y) when the block before arrives.  Against k_solve_f0, two
 // k_solve_chain and k_solve_b0 that is three launches and two passes over the
 // vectors less, with the same sums in the same order.  Words and polls as in
-// k_solve_chain, but y and x have words of their own, so a word is written
-// once per solve and one tag per solve serves every block.  Rows: one per wave;
-// NW waves per group, few, so that a block's loads spread over many CUs.
-// Bound: the hand-over, 1.9 us a step.  50x100x50 (SB 256, 11 blocks): 42 us
-// against 51 us and three launches; 2 waves per group against 4: 42.4 / 42.9
-// us, at SB 384 70 / 76 us.  Groups with waves that only poll, beside the row
-// waves, were slower (62 us; at SB 960 163 against 92 us a direction: polls
-// that do not wait for the operator rows compete with them for memory).
-constexpr int kFusedMaxSB = 512;
+// k_solve_chain.  Rows: one per wave; NW waves per group, few, so that a
+// block's loads spread over many CUs.
+// Bound: the hand-over, 1.4 us a step.  50x100x50 (SB 256, 11 blocks): 36.3 us,
+// 39 with words of half a value, against 51 us and three launches; 2 waves per
+// group against 4: 42.4 / 42.9 us (words of half a value), at SB 384 70 / 76 us.
+// Two sets of groups in turn: 34.9 us and twice the share of the device.  Groups
+// with waves that only poll, beside the row waves, were slower (62 us; at SB
+// 960 163 against 92 us a direction: polls that do not wait for the operator
+// rows compete with them for memory).
 struct FusedArgs {
   int n, SB, nblk;
   const long long* map;
   const double *Dinv, *DT, *Gm, *H;
   double* vb;                 // own terms of the way back
-  unsigned long long *W, *X;  // tagged y and x
+  unsigned long long *W, *X;  // exchanged y and x, two places each
   ChainState* st;
 };
 // NCH: 64-column chunks of a row (SB <= 64 NCH), PT = NCH / NW entries polled per thread
@@ -944,9 +964,10 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
   const int SB = A.SB, nblk = A.nblk;
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * NW + (threadIdx.x >> 6);  // SB is a multiple of NW: row < SB
-  const unsigned tag = A.st->tag[blockIdx.x] + 1;  // one above this group's last solve
+  const unsigned turn = A.st->turn[blockIdx.x];
+  const size_t wn = (size_t)(turn & 1) * nblk * SB, wo = (size_t)(~turn & 1) * nblk * SB;
   int step = 0;
-  // block b of Wd into the next buffer once every entry carries the tag
+  // block b of Wd into the next buffer once every entry is there
   auto poll = [&](const unsigned long long* Wd, int b) -> const double* {
     double* sY = chainNbr + (step++ & 1) * SB;
     unsigned pending = 0;
@@ -955,18 +976,14 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
       if ((int)threadIdx.x + k * NT < SB) pending |= 1u << k;
     unsigned polls = 0;
     while (pending) {
-      unsigned long long hi[PT], lo[PT];
+      unsigned long long w[PT];
 #pragma unroll
       for (int k = 0; k < PT; ++k)
-        if (pending & (1u << k)) {
-          const int i = b * SB + threadIdx.x + k * NT;
-          hi[k] = __hip_atomic_load(Wd + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          lo[k] = __hip_atomic_load(Wd + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        if (pending & (1u << k)) w[k] = chain_get(Wd + b * SB + threadIdx.x + k * NT);
 #pragma unroll
       for (int k = 0; k < PT; ++k)
-        if ((pending & (1u << k)) && (unsigned)hi[k] == tag && (unsigned)lo[k] == tag) {
-          sY[threadIdx.x + k * NT] = __longlong_as_double((long long)((hi[k] & 0xFFFFFFFF00000000ull) | (lo[k] >> 32)));
+        if ((pending & (1u << k)) && w[k]) {
+          sY[threadIdx.x + k * NT] = chain_value(w[k]);
           pending &= ~(1u << k);
         }
       if (!pending) break;
@@ -1009,7 +1026,7 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
           if (j + 64 * u < len) s0 = fma(r[4 * q + u], v[j + 64 * u], s0);
       }
     }
-    return chain_wave_sum((s0 + s1) + (s2 + s3));
+    return wave_sum((s0 + s1) + (s2 + s3));
   };
   auto op_row = [&](const double* M, int b) { return M + ((size_t)b * SB + row) * SB; };
   double rg[NCH], rt[NCH], rd[NCH], rv[NCH];  // rows of G or H, of DT from the diagonal on, of Dinv; the right-hand side
@@ -1022,10 +1039,13 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
     }
     load(op_row(A.Dinv, b), SB, rd);
   };
+  long long to = 0;  // where the row's entry of x goes (read ahead: the store must not wait for it)
+  auto load_to = [&](int b) { to = A.map[min(b * SB + row, A.n - 1)]; };
   auto emit_x = [&](int b, double v) {
     const int g = b * SB + row;
-    chain_put(A.X, g, v, tag);
+    chain_put(A.X + wn + g, v);
     if (g < A.n) xdense[A.map[g]] = (TV)v;
+    chain_clear(A.X + wo + g);
   };
   load_own(0);
   for (int b = 0; b < nblk; ++b) {  // forwards
@@ -1033,13 +1053,16 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
 #pragma unroll
     for (int c = 0; c < NCH; ++c)  // k_solve_f0's order
       if (lane + 64 * c <= row) y = fma(rd[c], rv[c], y);
-    y = chain_wave_sum(y);
+    y = wave_sum(y);
     const double* sY = nullptr;
     if (b > 0) {
-      sY = poll(A.W, b - 1);
+      sY = poll(A.W + wn, b - 1);
       y -= dot(rg, sY, SB);
     }
-    if (lane == 0) chain_put(A.W, b * SB + row, y, tag);
+    if (lane == 0) {
+      chain_put(A.W + wn + b * SB + row, y);
+      chain_clear(A.W + wo + b * SB + row);
+    }
     if (b + 1 < nblk) {
       load(op_row(A.Gm, b + 1), SB, rg);
       load_own(b + 1);
@@ -1051,7 +1074,7 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
     load(op_row(A.DT, b) + row, SB - row, rt);
   }
   {  // x of the last block is its own term
-    const double* sY = poll(A.W, nblk - 1);
+    const double* sY = poll(A.W + wn, nblk - 1);
     const double x = dot(rt, sY + row, SB - row);
     if (lane == 0) emit_x(nblk - 1, x);
   }
@@ -1059,11 +1082,11 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
     load(op_row(A.H, b), SB, rg);
     double own = 0.0;
     if (lane == 0) own = A.vb[(size_t)b * SB + row];  // this lane's own store
-    const double* sY = poll(A.X, b + 1);
+    const double* sY = poll(A.X + wn, b + 1);
     const double x = own - dot(rg, sY, SB);
     if (lane == 0) emit_x(b, x);
   }
-  if (threadIdx.x == 0) A.st->tag[blockIdx.x] = tag;
+  if (threadIdx.x == 0) A.st->turn[blockIdx.x] = turn + 1;
 }
 
 // ---- host side -----------------------------------------------------------
@@ -1078,6 +1101,12 @@ static FusedForm<TV> fused_form(int SB) {
   return {2, k_solve_fused<TV, 2, 8>};
 }
 static size_t fused_lds(int SB) { return 2 * (size_t)SB * sizeof(double); }
+
+template <typename TV, bool FWD>
+static auto chain_form(int SB, int sets) {
+  if (SB > 4 * CT) return k_solve_chain<TV, kChainMaxSB / CT, 1, FWD>;
+  return sets == 2 ? k_solve_chain<TV, 4, 2, FWD> : k_solve_chain<TV, 4, 1, FWD>;
+}
 
 long long CoarseSolver::chain_share() const {
   constexpr long long kNever = 2000000;
@@ -1095,8 +1124,8 @@ long long CoarseSolver::chain_share() const {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, ff.fn, 64 * ff.waves, lds) != hipSuccess) return kNever;
   } else {
     const size_t lds = (size_t)SB * sizeof(double);
-    auto fwd = SB <= 4 * CT ? k_solve_chain<double, 4, true> : k_solve_chain<double, kChainMaxSB / CT, true>;
-    auto bwd = SB <= 4 * CT ? k_solve_chain<float, 4, false> : k_solve_chain<float, kChainMaxSB / CT, false>;
+    auto fwd = chain_form<double, true>(SB, sets);
+    auto bwd = chain_form<float, false>(SB, sets);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fwd, CT, lds) != hipSuccess) return kNever;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, bwd, CT, lds) != hipSuccess) return kNever;
   }
@@ -1157,9 +1186,9 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
     return;
   }
   const dim3 ownGrid(np / kOwnRows);
-  if (C.one_launch()) {  // va, vb: np plain doubles, then 2 np tagged words each
-    auto fwd = SB <= 4 * CT ? k_solve_chain<TV, 4, true> : k_solve_chain<TV, kChainMaxSB / CT, true>;
-    auto bwd = SB <= 4 * CT ? k_solve_chain<TV, 4, false> : k_solve_chain<TV, kChainMaxSB / CT, false>;
+  if (C.one_launch()) {  // va, vb: np plain doubles, then 2 np words each
+    auto fwd = chain_form<TV, true>(SB, C.sets);
+    auto bwd = chain_form<TV, false>(SB, C.sets);
     const dim3 grid((SB + wpb - 1) / wpb);
     hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
                        fl);
