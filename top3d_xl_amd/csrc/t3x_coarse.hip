@@ -359,25 +359,10 @@ __device__ __forceinline__ void tile_trsm_rt(double (*sX)[TB + 1], const double 
   }
 }
 
-// Stages a 64x64 tile of the band (rows i0.., columns k0..) into LDS: all 16
-// loads of a thread are issued before the stores.
-__device__ __forceinline__ void stage_tile(BandView V, int i0, int k0, double (*sT)[TB + 1]) {
-  double v[TB * TB / CT];
-#pragma unroll
-  for (int u = 0; u < TB * TB / CT; ++u) {
-    const int t = threadIdx.x + u * CT;
-    v[u] = V.get(i0 + t / TB, k0 + t % TB);
-  }
-#pragma unroll
-  for (int u = 0; u < TB * TB / CT; ++u) {
-    const int t = threadIdx.x + u * CT;
-    sT[t / TB][t % TB] = v[u];
-  }
-}
-// Two or three tiles at once (one memory round trip), by FT threads: (i0, k0) ->
-// s0, (i1, k1) -> s1 and, with THREE, (i2, k2) -> s2.  THREE is a compile-time
-// choice: a load under a run-time condition makes the compiler wait for the
-// loads before it at every branch.
+// Stages two or three 64x64 tiles of the band in one memory round trip, by FT
+// threads: (i0, k0) -> s0, (i1, k1) -> s1 and, with THREE, (i2, k2) -> s2.
+// THREE is a compile-time choice: a load under a run-time condition makes the
+// compiler wait for the loads before it at every branch.
 template <bool THREE>
 __device__ __forceinline__ void stage_tiles(BandView V, int i0, int k0, double (*s0)[TB + 1], int i1, int k1,
                                             double (*s1)[TB + 1], int i2, int k2, double (*s2)[TB + 1]) {
@@ -559,42 +544,40 @@ __global__ __launch_bounds__(CT) void k_tile_inverses(BandView V, double* __rest
 // ---- 2. solve-block operators -------------------------------------------
 // WG (b, p): columns p*64.. of X = L_bb^{-1} [I | L_{b,b-1}], SB x 2SB.
 // Output: Dinv_b (SB x SB row-major) and its transpose DT_b, G_b (SB x SB).
-__global__ __launch_bounds__(CT) void k_trsm_blocks(BandView V, int SB, const double* __restrict__ tinv,
-                                                    double* __restrict__ Dinv, double* __restrict__ DT,
-                                                    double* __restrict__ Gm) {
-  // two tiles of LDS (66.6 KB: two work-groups per CU); the right-hand side
-  // minus the accumulated products is formed in sX once the products are done
-  __shared__ double sL[TB][TB + 1];
-  __shared__ double sX[TB][TB + 1];
-  // (dispatch order: the strips' work differs, from one tile pair to st(st+1)/2;
-  // an XCD-contiguous order measured 2.44 against 2.34 ms at 256x512x256)
-  const int npan = 2 * SB / TB;
-  const int b = blockIdx.x / npan, p = blockIdx.x % npan;
-  const int st = SB / TB;
-  const bool ident = p < st;
-  if (!ident && b == 0) return;  // G_0 is unused
-  const int base = b * SB;
-  double* Out = ident ? Dinv + (size_t)b * SB * SB : Gm + (size_t)b * SB * SB;
-  const int col0 = ident ? p * TB : (p - st) * TB;
-  const int Ist = ident ? p : 0;  // rows above the diagonal panel of L^{-1} are zero
-  for (int I = 0; I < st; ++I) {
-    if (I < Ist) {
-      for (int t = threadIdx.x; t < TB * TB; t += CT) {
-        const int a = t / TB, c = t % TB;
-        Out[(size_t)(I * TB + a) * SB + col0 + c] = 0.0;
-      }
-      continue;
+// A step multiplies two 64x64 tiles from LDS; the next step's tiles are loaded
+// into registers beside it.  Bound: the loads (64 KB a step, mostly past the
+// L2, few in flight per CU); the matrix cores are busy a sixth of the time.
+// 2.34 -> 1.55 ms at 256x512x256 (SB 960, 30 blocks), 81 -> 52 us at
+// 50x100x50; two waves per SIMD are worth the 248 registers (one: 2.73 ms).
+template <bool IDENT>
+__device__ __forceinline__ void trsm_strip(BandView V, int SB, int b, int col0, const double* __restrict__ tinv,
+                                           double* Out, double* __restrict__ DT, double (*sL)[TB + 1],
+                                           double (*sX)[TB + 1]) {
+  constexpr int U = TB * TB / CT;
+  const int st = SB / TB, base = b * SB;
+  const int Ist = IDENT ? col0 / TB : 0;  // rows above the diagonal panel of L^{-1} are zero
+  const int tr = threadIdx.x / TB, tc = threadIdx.x % TB;  // element u of this thread: row tr + 4 u, column tc
+  constexpr int RU = CT / TB;
+  double vl[U], vx[U], rr[2][2][4];
+  const int W = V.W();
+  auto load_l = [&](int I, int K) {  // L_bb(I, K): I > K, all its rows exist, the far corner may be outside the band
+    const int d = (I - K) * TB + tr - tc;
+    const double* l = V.B + (size_t)(base + I * TB + tr) * W;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double v = l[RU * u * W + min(d + RU * u, V.bw)];
+      vl[u] = d + RU * u <= V.bw ? v : 0.0;
     }
-    // T = R_I - sum_{K<I} L_bb(I,K) X_K
-    cd4 acc[2][2] = {};
-    for (int K = Ist; K < I; ++K) {
-      if ((I * TB) - (K * TB + TB - 1) > V.bw) continue;  // L tile outside the band
-      stage_tile(V, base + I * TB, base + K * TB, sL);
-      for (int t = threadIdx.x; t < TB * TB; t += CT) sX[t / TB][t % TB] = Out[(size_t)(K * TB + t / TB) * SB + col0 + t % TB];
-      __syncthreads();
-      tile_gemm_nn_mfma(sL, sX, acc);
-      __syncthreads();
-    }
+  };
+  auto load_x = [&](int K) {
+    const double* x = Out + (size_t)(K * TB + tr) * SB + col0 + tc;
+#pragma unroll
+    for (int u = 0; u < U; ++u) vx[u] = x[RU * u * SB];
+  };
+  auto load_diag = [&](int I) {  // inv(L_II) and the right-hand side
+    const double* inv = tinv + (size_t)(base / TB + I) * TB * TB + threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < U; ++u) vl[u] = inv[u * CT];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -602,35 +585,87 @@ __global__ __launch_bounds__(CT) void k_trsm_blocks(BandView V, int SB, const do
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
           const int ra = nt_row(a, r4), cc = nt_col(c);
-          const double r = ident ? ((I * TB + ra == col0 + cc) ? 1.0 : 0.0)
-                                 : V.get(base + I * TB + ra, base - SB + col0 + cc);
-          sX[ra][cc] = r - acc[a][c][r4];
+          rr[a][c][r4] = IDENT ? ((I * TB + ra == col0 + cc) ? 1.0 : 0.0)
+                               : V.get(base + I * TB + ra, base - SB + col0 + cc);
         }
-    // X_I = inv(L_II) T
-    const double* inv = tinv + (size_t)(base / TB + I) * TB * TB;
-    for (int t = threadIdx.x; t < TB * TB; t += CT) sL[t / TB][t % TB] = inv[t];
-    __syncthreads();
-    {
-      cd4 acc2[2][2] = {};
-      tile_gemm_nn_mfma(sL, sX, acc2);  // inv(L_II) is lower triangular: the zeros add nothing
+  };
+  // the first tile of row I inside the band
+  auto first = [&](int I) { return max(Ist, (I * TB - TB + 1 - V.bw + TB - 1) / TB); };
+  for (int I = 0; I < Ist; ++I)
+    for (int t = threadIdx.x; t < TB * TB; t += CT) Out[(size_t)(I * TB + t / TB) * SB + col0 + t % TB] = 0.0;
+  load_diag(Ist);
+  for (int I = Ist; I < st; ++I) {
+    // T = R_I - sum_{K<I} L_bb(I,K) X_K
+    cd4 acc[2][2] = {};
+    for (int K = first(I); K < I; ++K) {
 #pragma unroll
-      for (int a2 = 0; a2 < 2; ++a2)
-#pragma unroll
-        for (int c2 = 0; c2 < 2; ++c2)
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            const int a = nt_row(a2, r4), c = nt_col(c2);
-            Out[(size_t)(I * TB + a) * SB + col0 + c] = acc2[a2][c2][r4];
-            if (ident) DT[(size_t)b * SB * SB + (size_t)(col0 + c) * SB + I * TB + a] = acc2[a2][c2][r4];
-          }
+      for (int u = 0; u < U; ++u) {
+        sL[tr + RU * u][tc] = vl[u];
+        sX[tr + RU * u][tc] = vx[u];
+      }
+      __syncthreads();
+      if (K + 1 < I) {
+        load_l(I, K + 1);
+        load_x(K + 1);
+      } else {
+        load_diag(I);
+      }
+      tile_gemm_nn_mfma(sL, sX, acc);
+      __syncthreads();
     }
+    // X_I = inv(L_II) T
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) sX[nt_row(a, r4)][nt_col(c)] = rr[a][c][r4] - acc[a][c][r4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) sL[tr + RU * u][tc] = vl[u];
     __syncthreads();
+    const int K1 = I + 1 < st ? first(I + 1) : I + 1;  // the next row's first tile: X_I itself is not there yet
+    if (K1 <= I) load_l(I + 1, K1);
+    if (K1 < I) load_x(K1);
+    cd4 acc2[2][2] = {};
+    tile_gemm_nn_mfma(sL, sX, acc2);  // inv(L_II) is lower triangular: the zeros add nothing
+#pragma unroll
+    for (int a2 = 0; a2 < 2; ++a2)
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int a = nt_row(a2, r4), c = nt_col(c2);
+          Out[(size_t)(I * TB + a) * SB + col0 + c] = acc2[a2][c2][r4];
+          if (IDENT) DT[(size_t)b * SB * SB + (size_t)(col0 + c) * SB + I * TB + a] = acc2[a2][c2][r4];
+        }
+    __syncthreads();
+    if (K1 == I) load_x(I);
+    else if (K1 > I && I + 1 < st) load_diag(I + 1);
   }
+}
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void k_trsm_blocks(BandView V, int SB, const double* __restrict__ tinv,
+                                                    double* __restrict__ Dinv, double* __restrict__ DT,
+                                                    double* __restrict__ Gm) {
+  // two tiles of LDS (66.6 KB: two work-groups per CU); the right-hand side
+  // minus the accumulated products is formed in sX once the products are done
+  __shared__ double sL[TB][TB + 1];
+  __shared__ double sX[TB][TB + 1];
+  // G's strips first: their work is st(st+1)/2 tile pairs each, that of L^{-1}'s
+  // falls to one (block by block 1.72 ms at 256x512x256, so 1.55; blocks kept
+  // to one XCD 1.79 and 2.01: their strips start and end together)
+  const int st = SB / TB, npan = 2 * st, nG = gridDim.x / npan * st;
+  const bool g = (int)blockIdx.x < nG;
+  const int wg = g ? blockIdx.x : blockIdx.x - nG;
+  const int b = wg / st, p = wg % st + (g ? st : 0);
+  if (p < st) trsm_strip<true>(V, SB, b, p * TB, tinv, Dinv + (size_t)b * SB * SB, DT, sL, sX);
+  else if (b > 0) trsm_strip<false>(V, SB, b, (p - st) * TB, tinv, Gm + (size_t)b * SB * SB, DT, sL, sX);  // G_0 is unused
 }
 
 // H_b = Dinv_b^T L_{b+1,b}^T, i.e. H_b(i,j) = sum_k DT_b(i,k) L((b+1)SB + j, b SB + k).
-// One work-group per (b, output tile I, J).
-__global__ __launch_bounds__(CT) void k_h_blocks(BandView V, int SB, int nblk, const double* __restrict__ DT,
+// One work-group per (b, output tile I, J); the next step's tiles are loaded
+// beside a step's product (0.75 -> 0.48 ms at 256x512x256, 25 -> 16.5 us at
+// 50x100x50).
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void k_h_blocks(BandView V, int SB, int nblk, const double* __restrict__ DT,
                                                  double* __restrict__ H) {
   __shared__ double sA[TB][TB + 1];
   __shared__ double sB[TB][TB + 1];
@@ -645,12 +680,32 @@ __global__ __launch_bounds__(CT) void k_h_blocks(BandView V, int SB, int nblk, c
   if (b >= nblk - 1) return;
   const double* D = DT + (size_t)b * SB * SB;
   cd4 acc[2][2] = {};
-  for (int K = I; K < st; ++K) {  // DT_b(i,k) = Dinv_b(k,i) is zero for k < i
-    const int rowL0 = (b + 1) * SB + J * TB, colL0 = b * SB + K * TB;
-    if (rowL0 - (colL0 + TB - 1) > V.bw) continue;
-    for (int t = threadIdx.x; t < TB * TB; t += CT) sA[t / TB][t % TB] = D[(size_t)(I * TB + t / TB) * SB + K * TB + t % TB];
-    stage_tile(V, rowL0, colL0, sB);  // row j, col k
+  // DT_b(i,k) = Dinv_b(k,i) is zero for k < i; L's tiles before K0 are outside the band
+  const int rowL0 = (b + 1) * SB + J * TB;
+  const int K0 = max(I, (rowL0 - b * SB - TB + 1 - V.bw + TB - 1) / TB);
+  constexpr int U = TB * TB / CT, RU = CT / TB;
+  const int tr = threadIdx.x / TB, tc = threadIdx.x % TB, W = V.W();
+  double va[U], vb[U];
+  auto load = [&](int K) {  // the next step's tiles, beside this step's product
+    const double* x = D + (size_t)(I * TB + tr) * SB + K * TB + tc;
+    const int d = rowL0 - (b * SB + K * TB) + tr - tc;  // > 0
+    const double* l = V.B + (size_t)(rowL0 + tr) * W;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      va[u] = x[RU * u * SB];
+      const double v = l[RU * u * W + min(d + RU * u, V.bw)];
+      vb[u] = d + RU * u <= V.bw ? v : 0.0;
+    }
+  };
+  if (K0 < st) load(K0);
+  for (int K = K0; K < st; ++K) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      sA[tr + RU * u][tc] = va[u];
+      sB[tr + RU * u][tc] = vb[u];  // row j, col k
+    }
     __syncthreads();
+    if (K + 1 < st) load(K + 1);
     tile_gemm_nt_mfma(sA, sB, acc);
     __syncthreads();
   }
