@@ -1,5 +1,5 @@
 """The V-cycle's assembly and transfer kernels (k_galerkin_l2_bc,
-k_band_assemble, k_restrict_xz_w, the prolongation's launch shapes, the
+k_band_assemble, k_restrict_xz_w, k_restrict_once, the prolongation's launch shapes, the
 coarsest solve) against the FP64 oracle at the edges of their tiles.
 
 Bars: those of test_gpu_parity, 1e-11 for the V-cycle (two factorisations of
@@ -19,6 +19,8 @@ SHAPES = {
     (31, 33, 9): "ragged in every axis",
     (9, 120, 17): "long: 33 level-2 node columns",
     (64, 40, 40): "17 level-2 nodes in y",
+    (56, 56, 16): "coarsest plane of 8x8 nodes: one full block of 64 outputs",
+    (57, 63, 24): "coarsest plane of 9x9 nodes: a full block and a remainder, padded",
 }
 
 

@@ -220,6 +220,67 @@ __global__ __launch_bounds__(kXzOut * (2 * S - 1)) void k_restrict_xz_w(Geo gf, 
   }
 }
 
+// Both passes at once: wave dz + S - 1 of a block forms, for 64 outputs of one
+// coarse plane and one component, the x sums of its fine plane from y sums of
+// its own, each rounded to the intermediate's type as the passes store it; then
+// one wave adds up over z.  The fine values are read (2 - 1/S)^3 times over, all
+// a thread's loads in one round trip; a launch and the intermediate's round trip
+// are saved (see restrict_impl).
+template <int S, typename TI, typename TM, typename TO>
+__global__ __launch_bounds__(kXzOut * (2 * S - 1)) void k_restrict_once(Geo gf, Geo gc, const TI* __restrict__ rf,
+                                                                     const uint8_t* __restrict__ nmaskC,
+                                                                     TO* __restrict__ rc, const int* fl, Act actF) {
+  if (fl && fl[FL_DONE]) return;
+  __shared__ double sz[2 * S - 1][kXzOut];
+  const int planeC = gc.NY * gc.NX;
+  const int lane = threadIdx.x % kXzOut, w = threadIdx.x / kXzOut;
+  const int idx = blockIdx.x * kXzOut + lane;
+  const int Jz = blockIdx.y, c = blockIdx.z;
+  const long long n = idx + (long long)planeC * Jz;
+  const bool solid = idx < planeC && nmaskC[n];
+  auto in_z = [&](int dz) { return S * Jz + dz >= 0 && S * Jz + dz < gf.NZ; };
+  if (solid && in_z(w - (S - 1))) {
+    const int Jx = idx / gc.NY, Jy = idx - Jx * gc.NY;
+    const int z = S * Jz + w - (S - 1);
+    TI v[2 * S - 1][2 * S - 1];
+#pragma unroll
+    for (int dx = -(S - 1); dx <= S - 1; ++dx)
+#pragma unroll
+      for (int dy = -(S - 1); dy <= S - 1; ++dy) {
+        const int x = S * Jx + dx, y = S * Jy + dy;
+        const long long f = min(max(y, 0), gf.NY - 1) +
+                            gf.NY * (min(max(x, 0), gf.NX - 1) + (long long)gf.NX * z);
+        const bool on = !(actF.chunk && !actF.chunk[f >> 4]);
+        v[dx + S - 1][dy + S - 1] = on ? rf[c * gf.NN + f] : TI(0);
+      }
+    double s = 0.0;
+#pragma unroll
+    for (int dx = -(S - 1); dx <= S - 1; ++dx) {
+      const int x = S * Jx + dx;
+      if (x < 0 || x >= gf.NX) continue;
+      double t = 0.0;
+#pragma unroll
+      for (int dy = -(S - 1); dy <= S - 1; ++dy) {
+        const int y = S * Jy + dy;
+        if (y < 0 || y >= gf.NY) continue;
+        t += hat_w<S>(dy) * (double)v[dx + S - 1][dy + S - 1];
+      }
+      s += hat_w<S>(dx) * (double)(TM)t;
+    }
+    sz[w][lane] = s;
+  }
+  __syncthreads();
+  if (w == 0 && idx < planeC) {
+    double a = 0.0;
+    if (solid) {
+#pragma unroll
+      for (int dz = -(S - 1); dz <= S - 1; ++dz)
+        if (in_z(dz)) a += hat_w<S>(dz) * sz[dz + S - 1][lane];
+    }
+    rc[c * gc.NN + n] = (TO)a;
+  }
+}
+
 // out = omega*(r/d) + P xc + (omega*r)/d on solid nodes, 0 elsewhere (758,
 // 770, 773); optional fused z.r partials (629).  Block (bx, bz) covers 256
 // (y, x) columns and the node planes [bz*zc, bz*zc + zc); a thread walks its
@@ -384,6 +445,7 @@ void k_prolong_add(Geo gf, Geo gc, int zc, const TX* __restrict__ xc,
   }
 }
 
+constexpr long long kOnceOut = 65536;        // coarse nodes up to which a span-2 restriction is one launch
 constexpr long long kXzWideOut = 131072;     // coarse nodes up to which the x-z pass runs its planes side by side
 constexpr size_t kRestrictLds = 48 * 1024;  // LDS bytes of the y pass's rows at most
 
@@ -391,6 +453,15 @@ template <typename TI, typename TM, typename TO>
 void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const TI* rf, TM* tmp,
                    const uint8_t* nmaskC, TO* rc, const int* fl, Act actF) {
   const int plane = gc.NY * gf.NX;
+  // span 2: both passes in one launch while the launch saved is worth the values
+  // read 3.4 times over.  637 outputs 4.6 us against 7.1, 9,537 5.2 / 9.6, 31,213
+  // 6.7 / 9.9, 70,785 11.4 / 11.9, 217,800 18.0 / 16.7.  (Span 4 reads 5.4 times
+  // over: 112 outputs 16.5 us against 9.1, 70,785 109 / 39.)
+  if (span == 2 && gc.NN <= kOnceOut) {
+    const dim3 g((gc.NY * gc.NX + kXzOut - 1) / kXzOut, gc.NZ, 3);
+    hipLaunchKernelGGL((k_restrict_once<2, TI, TM, TO>), g, dim3(kXzOut * 3), 0, s, gf, gc, rf, nmaskC, rc, fl, actF);
+    return;
+  }
   const dim3 g1((plane + kBlock - 1) / kBlock, gf.NZ);
   // the LDS y pass: about one intermediate value per thread (R rows a block)
   // while the rows fit kRestrictLds bytes
