@@ -968,7 +968,8 @@ void vcycle_standard(t3x_problem& P, const double* r, float* z, double* sc, cons
   launch_prolong_add(s, g0, geo(P.lv[1]), P.lv[1].span, P.lv[1].xf, P.x32, P.lv[0].nmask, fl);
   launch_fine_smooth32_sf(s, g0, P.sf, P.E32, P.fix, P.x32, r, P.lv[0].diagf, om, z,
                           fuse ? P.ws.partials : nullptr, fl);
-  if (fuse) launch_fin1(s, fl ? FIN_ZR_LOOP : FIN_ZR_INIT, applyk_sf_blocks(g0), P.ws, sc, (int*)fl, nullptr);
+  if (fuse && fl) launch_fin_zr(s, applyk_sf_blocks(g0), 3 * g0.NN, P.ws, sc, (int*)fl);
+  else if (fuse) launch_fin1(s, FIN_ZR_INIT, applyk_sf_blocks(g0), P.ws, sc, nullptr, nullptr);
   P.tend(TG_VCYCLE, ev);
 }
 
@@ -1006,11 +1007,20 @@ void vcycle_standard64(t3x_problem& P, const double* r, double* z, double* sc, c
   }
   launch_prolong_add(s, g0, geo(P.lv[1]), P.lv[1].span, (const double*)P.lv[1].x, P.x64, P.lv[0].nmask, fl);
   launch_fine_smooth64_sf(s, g0, P.sf, P.E, P.fix, P.x64, r, P.lv[0].diag, om, z, fuse ? P.ws.partials : nullptr, fl);
-  if (fuse) launch_fin1(s, fl ? FIN_ZR_LOOP : FIN_ZR_INIT, applyk_sf_blocks(g0), P.ws, sc, (int*)fl, nullptr);
+  if (fuse && fl) launch_fin_zr(s, applyk_sf_blocks(g0), 3 * g0.NN, P.ws, sc, (int*)fl);
+  else if (fuse) launch_fin1(s, FIN_ZR_INIT, applyk_sf_blocks(g0), P.ws, sc, nullptr, nullptr);
   P.tend(TG_VCYCLE, ev);
 }
 
 // ------------------------------------------------------------- PCG
+// A solver loop's dot products may be left to the updates that need them.
+struct LateScope {
+  RedWs& ws;
+  LateFold fold;
+  explicit LateScope(RedWs& w) : ws(w) { ws.late = &fold; }
+  ~LateScope() { ws.late = nullptr; }
+  LateScope(const LateScope&) = delete;
+};
 // The coarsest solve's failure word (read into hbuf[255] after a solve): a
 // wait of the one-launch recurrences expired, the solve is garbage.
 static void check_chain(t3x_problem& P) {
@@ -1044,6 +1054,7 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
   const int ce = std::max(1, P.P.checkEvery);
   int its = maxIT;
   bool done = false;
+  const LateScope late(P.ws);
   // one iteration: K*p (614-615), r and the residual norm (617-622), z = M r
   // (628-629), y and p (616, 630)
   auto iteration = [&]() {
@@ -1058,11 +1069,11 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
     if (mx) {
       if (P.standard()) vcycle_standard(P, P.r, P.z32, sc, fl, true, true);                // 628-629
       else vcycle_mixed(P, P.r, P.z32, sc, fl, true);
-      launch_pcg_pupdate(s, y, P.p, P.z32, n3, sc, fl, P.fineAct());                        // 616, 630
+      launch_pcg_pupdate(s, y, P.p, P.z32, n3, P.ws, sc, fl, P.fineAct());                        // 616, 630
     } else {
       if (P.standard()) vcycle_standard64(P, P.r, P.z, sc, fl, true);                         // 628-629
       else vcycle(P, P.r, P.z, sc, fl, true);
-      launch_pcg_pupdate(s, y, P.p, P.z, n3, sc, fl, P.fineAct());
+      launch_pcg_pupdate(s, y, P.p, P.z, n3, P.ws, sc, fl, P.fineAct());
     }
   };
   // With params.graphs (and no kernel-group timing) the iteration is captured
@@ -1167,11 +1178,12 @@ int filter_run(t3x_problem& P, int slot, const double* src, double* dst) {
   const int maxIT = P.P.maxIT;
   const int ce = std::max(1, P.P.checkEvery);
   int its = maxIT;
+  const LateScope late(P.ws);
   for (int it = 1; it <= maxIT; ++it) {
     launch_filter_apply(s, g0, kern, P.lv[0].emask, P.fp, P.fq, &P.ws, sc, fl);
     launch_pcg_update(s, P.fx, P.fr, P.fp, P.fq, NN, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct());
     launch_scale_diag(s, P.fz, dinv, P.fr, NN, &P.ws, sc, fl);
-    launch_pcg_pupdate(s, P.fx, P.fp, P.fz, NN, sc, fl, P.fineAct());
+    launch_pcg_pupdate(s, P.fx, P.fp, P.fz, NN, P.ws, sc, fl, P.fineAct());
     if (it % ce == 0 || it == maxIT) {
       T3X_HIP(hipMemcpyAsync(P.hbuf, fl, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
       P.sync();

@@ -58,15 +58,26 @@ __device__ __forceinline__ long long act_node(const Act& a, long long g) {
 }
 
 // Reduction workspace: partials (kMaxRedBlocks * 8 doubles) + one counter.
+// late: where set (by the solver's loop), p.q and z.r of few partials are left
+// for the vector update that consumes them to fold in every block of its own;
+// late->pq, late->zr: how many there are (0: folded).  A left p.q lies at
+// partials + kLateAt: the update that folds it writes partials of its own.
+constexpr int kLateAt = 32768;
+struct LateFold {
+  int pq = 0, zr = 0;
+};
 struct RedWs {
   double* partials;
   unsigned int* counter;
+  LateFold* late = nullptr;
 };
 
 // One-block finalisers: fold nb partials in a fixed order, then apply the
 // solver's scalar step (CG step lengths, convergence flag).
 enum FinOp { FIN_PQ = 0, FIN_ZR_INIT, FIN_ZR_LOOP, FIN_RR, FIN_SUM, FIN_SQRT };
 void launch_fin1(hipStream_t s, int op, int nb, const RedWs& ws, double* sc, int* fl, double* out);
+// FIN_ZR_LOOP of a solve with n unknowns, or left to its launch_pcg_pupdate
+void launch_fin_zr(hipStream_t s, int nb, long long n, const RedWs& ws, double* sc, int* fl);
 
 // ---------------------------------------------------------------- FEM
 // sum-factorised K*u (t3x_applyk_sf.hip): the isotropic unit-brick Ke as
@@ -203,12 +214,12 @@ void launch_dot(hipStream_t s, const double* a, const double* b, long long n, co
 void launch_pcg_update(hipStream_t s, double* y, double* r, const double* p, const double* q, long long n,
                        const RedWs& ws, double* sc, int* fl, const float* dj = nullptr, float* xj = nullptr,
                        double omega = 0.0, Act act = {});
-void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const double* z, long long n, const double* sc,
+void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const double* z, long long n, const RedWs& ws, double* sc,
                         const int* fl, Act act = {});
 void launch_pcg_finish(hipStream_t s, double* y, const double* p, long long n, const double* sc, const int* fl,
                        Act act = {});
 // mixed precision: FP32 z = M r, FP64 y, r, p, q
-void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const float* z, long long n, const double* sc,
+void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const float* z, long long n, const RedWs& ws, double* sc,
                         const int* fl, Act act = {});
 void launch_stream_copy(hipStream_t s, double* dst, const double* src, long long nDoubles);  // nDoubles even
 void launch_convert(hipStream_t s, float* dst, const double* src, long long n);

@@ -47,17 +47,18 @@ __global__ __launch_bounds__(kFinBlock) void k_fin1(int op, int nb, const double
   if (threadIdx.x != 0) return;
   const double t = v[0];
   switch (op) {
-    case FIN_PQ:  // 615
+    case FIN_PQ: {  // 615
+      const double zr = sc[SC_ZRN];  // (SC_ZR: what it was an iteration ago)
       sc[SC_PQ] = t;
-      sc[SC_LAMBDA] = sc[SC_ZR] / t;
-      break;
+      sc[SC_LAMBDA] = zr / t;
+      sc[SC_ZR] = zr;
+    } break;
     case FIN_ZR_INIT:  // 612
-      sc[SC_ZR] = t;
+      sc[SC_ZRN] = t;
       break;
     case FIN_ZR_LOOP:  // 629-631
       sc[SC_ZRN] = t;
       sc[SC_BETA] = t / sc[SC_ZR];
-      sc[SC_ZR] = t;
       break;
     case FIN_RR: {  // 618-622
       const double res = sqrt(t) / sc[SC_NORMB];
@@ -78,6 +79,21 @@ __global__ __launch_bounds__(kFinBlock) void k_fin1(int op, int nb, const double
 void launch_fin1(hipStream_t s, int op, int nb, const RedWs& ws, double* sc, int* fl, double* out) {
   hipLaunchKernelGGL(k_fin1, dim3(1), dim3(kFinBlock), 0, s, op, nb, ws.partials, sc, fl, out);
 }
+// Whether the nb partials of a dot product are left for the update of n elements
+// that needs it: a launch less (2.4 to 3.3 us) against a fold in each of its
+// blocks (0.4 us at 12x24x12, 1.2 at 50x100x50).  The line, in partials read by
+// all its blocks together: 32x64x32 5.61 -> 5.30 ms for a design iteration,
+// 50x100x50 (1.1 M) 8.63 -> 8.41; 64x128x64 (3.6 to 5 M) 10.57 -> 10.80.
+constexpr long long kLateReads = 1 << 21;
+static bool late_fold(const RedWs& ws, int nb, long long n) {
+  static_assert(kLateAt + 4 * kFinBlock <= kMaxPartials, "room for a left p.q");
+  return ws.late && nb <= 4 * kFinBlock && nb * ((n + kBlock - 1) / kBlock) <= kLateReads;
+}
+void launch_fin_zr(hipStream_t s, int nb, long long n, const RedWs& ws, double* sc, int* fl) {
+  const bool late = late_fold(ws, nb, n);
+  if (ws.late) ws.late->zr = late ? nb : 0;
+  if (!late) launch_fin1(s, FIN_ZR_LOOP, nb, ws, sc, fl, nullptr);
+}
 static void fin1(hipStream_t s, int op, int nb, const RedWs& ws, double* sc, int* fl, double* out) {
   launch_fin1(s, op, nb, ws, sc, fl, out);
 }
@@ -97,8 +113,11 @@ __global__ __launch_bounds__(kBlock) void k_fin_max(int nb, const double* __rest
 // =========================================================================
 void launch_apply_K(hipStream_t s, const Geo& g, const SfCoef& cf, const double* E, const uint8_t* fix,
                     const double* u, double* y, const RedWs& ws, double* sc, const int* fl, bool pcgStep) {
-  launch_apply_K_sf(s, g, cf, E, fix, u, y, pcgStep ? ws.partials : nullptr, fl);
-  if (pcgStep) fin1(s, FIN_PQ, applyk_sf_blocks(g), ws, sc, (int*)fl, nullptr);
+  const int nb = applyk_sf_blocks(g);
+  const bool late = pcgStep && late_fold(ws, nb, 3 * g.NN);
+  launch_apply_K_sf(s, g, cf, E, fix, u, y, pcgStep ? ws.partials + (late ? kLateAt : 0) : nullptr, fl);
+  if (ws.late) ws.late->pq = late ? nb : 0;
+  if (pcgStep && !late) fin1(s, FIN_PQ, nb, ws, sc, (int*)fl, nullptr);
 }
 
 // =========================================================================
@@ -738,6 +757,29 @@ void launch_dot(hipStream_t s, const double* a, const double* b, long long n, co
   fin1(s, FIN_SUM, red1_blocks(n), ws, nullptr, nullptr, out);
 }
 
+// The fold of k_fin1 in a block of kBlock threads, for up to 4 kFinBlock
+// partials: its threads' sums, its waves' sums and their sum in its order; the
+// total in every thread.
+__device__ __forceinline__ double fold_here(const double* p, int nb) {
+  constexpr int V = kFinBlock / kBlock;
+  __shared__ double sh[kFinBlock / 64];
+  const int w = threadIdx.x >> 6;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    double a[4] = {};
+    const int b = threadIdx.x + v * kBlock;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (b + u * kFinBlock < nb) a[u] += p[b + u * kFinBlock];
+    const double s = v * kBlock < nb ? wave_sum((a[0] + a[2]) + (a[1] + a[3])) : 0.0;
+    if ((threadIdx.x & 63) == 0) sh[w + v * (kBlock / 64)] = s;
+  }
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < kFinBlock / 64; ++k) s += sh[k];
+  return s;
+}
 // y += lambda p ; r -= lambda q ; resnorm = ||r|| / ||b|| ; convergence flag.
 // r -= lambda q (617) with the r.r reduction.  With xj given (FP32 'Standard'
 // V-cycle), also the first fine Jacobi step of the next preconditioner
@@ -769,18 +811,60 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(double* __restrict__ r, c
   double v[1] = {rr};
   write_partials<1>(v, ws.partials);
 }
+// the same with p.q still to be folded
+__global__ __launch_bounds__(kBlock) void k_pcg_update_late(double* __restrict__ r, const double* __restrict__ q,
+                                                       long long n, RedWs ws, double* sc, int* fl,
+                                                       const float* __restrict__ dj, float* __restrict__ xj,
+                                                       double omega, Act act, int nbPQ) {
+  if (fl[FL_DONE]) return;
+  // y += lambda p (616) is deferred to k_pcg_pupdate, which reads p anyway
+  const long long m = act_items(act, n);
+  const int nc = act_ncomp(act, n);
+  const long long g = (long long)blockIdx.x * kBlock + threadIdx.x;  // one item per thread
+  const long long b = g < m ? act_node(act, g) : 0;
+  const bool on = g < m && !(act.list && b >= act.NN);
+  const double r0 = on ? r[b] : 0.0, q0 = on ? q[b] : 0.0;  // on their way while the fold is made
+  // FIN_PQ, in every block
+  const double t = fold_here(ws.partials + kLateAt, nbPQ), zr = sc[SC_ZRN], lambda = zr / t;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // (read by later kernels only)
+    sc[SC_PQ] = t;
+    sc[SC_LAMBDA] = lambda;
+    sc[SC_ZR] = zr;
+  }
+  double rr = 0.0;
+  auto element = [&](long long i, double rOld, double qi) {
+    const double ri = rOld - lambda * qi;  // 617
+    r[i] = ri;
+    rr += ri * ri;
+    if (xj) {
+      const double dd = (double)dj[i];
+      xj[i] = dd != 0.0 ? (float)(omega * (ri / dd)) : 0.f;
+    }
+  };
+  if (on) {
+    element(b, r0, q0);
+    for (int c = 1; c < nc; ++c) element(b + c * act.NN, r[b + c * act.NN], q[b + c * act.NN]);
+  }
+  double v[1] = {rr};
+  write_partials<1>(v, ws.partials);
+}
 void launch_pcg_update(hipStream_t s, double* y, double* r, const double* p, const double* q, long long n,
                        const RedWs& ws, double* sc, int* fl, const float* dj, float* xj, double omega, Act act) {
   (void)y;
   (void)p;
   const int nb = red1_blocks(act_items(act, n));
-  hipLaunchKernelGGL(k_pcg_update, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act);
+  const int nbPQ = ws.late ? ws.late->pq : 0;
+  if (nbPQ)
+    hipLaunchKernelGGL(k_pcg_update_late, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act, nbPQ);
+  else
+    hipLaunchKernelGGL(k_pcg_update, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act);
   fin1(s, FIN_RR, nb, ws, sc, fl, nullptr);
 }
 
 // y += lambda p (616) for the iteration just finished, then p = z + beta p (630).
-__global__ void k_pcg_pupdate(double* __restrict__ y, double* __restrict__ p, const double* __restrict__ z,
-                              long long n, const double* sc, const int* fl, Act act) {
+template <typename TZ>
+__global__ void k_pcg_pupdate(double* __restrict__ y, double* __restrict__ p, const TZ* __restrict__ z, long long n,
+                              const double* sc, const int* fl, Act act) {
   if (fl[FL_DONE]) return;
   const double beta = sc[SC_BETA], lambda = sc[SC_LAMBDA];
   const long long m = act_items(act, n);
@@ -792,14 +876,45 @@ __global__ void k_pcg_pupdate(double* __restrict__ y, double* __restrict__ p, co
       const long long i = b + c * act.NN;
       const double pi = p[i];
       y[i] = y[i] + lambda * pi;
-      p[i] = z[i] + beta * pi;
+      p[i] = (double)z[i] + beta * pi;
     }
   }
 }
-void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const double* z, long long n, const double* sc,
+// the same with z.r still to be folded (FIN_ZR_LOOP, in every block); one item per thread
+template <typename TZ>
+__global__ __launch_bounds__(kBlock) void k_pcg_pupdate_late(double* __restrict__ y, double* __restrict__ p,
+                                                             const TZ* __restrict__ z, long long n, RedWs ws,
+                                                             double* sc, const int* fl, Act act, int nbZR) {
+  if (fl[FL_DONE]) return;
+  const int nc = act_ncomp(act, n);
+  const long long g = (long long)blockIdx.x * kBlock + threadIdx.x;
+  const bool in = g < act_items(act, n);
+  const long long b = in ? act_node(act, g) : 0;
+  const bool on = in && !(act.list && b >= act.NN);
+  const double p0 = on ? p[b] : 0.0, y0 = on ? y[b] : 0.0, z0 = on ? (double)z[b] : 0.0;  // beside the fold
+  const double t = fold_here(ws.partials, nbZR), beta = t / sc[SC_ZR], lambda = sc[SC_LAMBDA];
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc[SC_ZRN] = t;  // (read by later kernels only)
+  if (!on) return;
+  y[b] = y0 + lambda * p0;
+  p[b] = z0 + beta * p0;
+  for (int c = 1; c < nc; ++c) {
+    const long long i = b + c * act.NN;
+    const double pi = p[i];
+    y[i] = y[i] + lambda * pi;
+    p[i] = (double)z[i] + beta * pi;
+  }
+}
+template <typename TZ>
+static void pcg_pupdate(hipStream_t s, double* y, double* p, const TZ* z, long long n, const RedWs& ws, double* sc,
                         const int* fl, Act act) {
-  hipLaunchKernelGGL(k_pcg_pupdate, dim3(stream_blocks(act_items(act, n))), dim3(kBlock), 0, s, y, p, z, n, sc, fl,
-                     act);
+  const dim3 grid(stream_blocks(act_items(act, n)));
+  const int nbZR = ws.late ? ws.late->zr : 0;
+  if (nbZR) hipLaunchKernelGGL(k_pcg_pupdate_late<TZ>, grid, dim3(kBlock), 0, s, y, p, z, n, ws, sc, fl, act, nbZR);
+  else hipLaunchKernelGGL(k_pcg_pupdate<TZ>, grid, dim3(kBlock), 0, s, y, p, z, n, sc, fl, act);
+}
+void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const double* z, long long n, const RedWs& ws, double* sc,
+                        const int* fl, Act act) {
+  pcg_pupdate(s, y, p, z, n, ws, sc, fl, act);
 }
 // After the loop: the converging iteration skipped its p-update, so its
 // y += lambda p is applied here (no-op if the solve hit maxIT).
@@ -824,27 +939,9 @@ void launch_pcg_finish(hipStream_t s, double* y, const double* p, long long n, c
 }
 
 // Mixed precision: the V-cycle output z is FP32; y, r, p and scalars FP64.
-__global__ void k_pcg_pupdate_mixed(double* __restrict__ y, double* __restrict__ p, const float* __restrict__ z,
-                                    long long n, const double* sc, const int* fl, Act act) {
-  if (fl[FL_DONE]) return;
-  const double beta = sc[SC_BETA], lambda = sc[SC_LAMBDA];
-  const long long m = act_items(act, n);
-  const int nc = act_ncomp(act, n);
-  for (long long g = (long long)blockIdx.x * kBlock + threadIdx.x; g < m; g += (long long)gridDim.x * kBlock) {
-    const long long b = act_node(act, g);
-    if (act.list && b >= act.NN) continue;
-    for (int c = 0; c < nc; ++c) {
-      const long long i = b + c * act.NN;
-      const double pi = p[i];
-      y[i] = y[i] + lambda * pi;
-      p[i] = (double)z[i] + beta * pi;
-    }
-  }
-}
-void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const float* z, long long n, const double* sc,
+void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const float* z, long long n, const RedWs& ws, double* sc,
                         const int* fl, Act act) {
-  hipLaunchKernelGGL(k_pcg_pupdate_mixed, dim3(stream_blocks(act_items(act, n))), dim3(kBlock), 0, s, y, p, z, n, sc,
-                     fl, act);
+  pcg_pupdate(s, y, p, z, n, ws, sc, fl, act);
 }
 template <typename TD, typename TS>
 __global__ void k_convert(TD* __restrict__ dst, const TS* __restrict__ src, long long n) {
@@ -885,7 +982,8 @@ void launch_scale_diag(hipStream_t s, double* z, const double* dinv, const doubl
                        const RedWs* ws, double* sc, const int* fl) {
   const int mode = fl ? 2 : 1;
   hipLaunchKernelGGL(k_scale_diag, dim3(red1_blocks(n)), dim3(kBlock), 0, s, z, dinv, r, n, *ws, sc, fl, mode);
-  fin1(s, mode == 1 ? FIN_ZR_INIT : FIN_ZR_LOOP, red1_blocks(n), *ws, sc, (int*)fl, nullptr);
+  if (mode == 1) fin1(s, FIN_ZR_INIT, red1_blocks(n), *ws, sc, (int*)fl, nullptr);
+  else launch_fin_zr(s, red1_blocks(n), n, *ws, sc, (int*)fl);
 }
 
 __global__ void k_gather_compact(const int* __restrict__ map, int n, int ncomp, long long NN,
@@ -1040,8 +1138,13 @@ void launch_filter_apply(hipStream_t s, const Geo& g, const double* kern, const 
   if (ws) { w = *ws; step = 1; }
   int zc = 8;
   const dim3 grid = filter_grid(g, zc);
-  hipLaunchKernelGGL(k_filter_apply, grid, dim3(kFaY, kFaX), 0, s, g, zc, kern, emask, u, y, w, fl, step);
-  if (step) fin1(s, FIN_PQ, (int)(grid.x * grid.y * grid.z), w, sc, (int*)fl, nullptr);
+  const int nb = (int)(grid.x * grid.y * grid.z);
+  const bool late = step && late_fold(w, nb, g.NN);
+  RedWs at = w;
+  if (late) at.partials += kLateAt;
+  hipLaunchKernelGGL(k_filter_apply, grid, dim3(kFaY, kFaX), 0, s, g, zc, kern, emask, u, y, at, fl, step);
+  if (w.late) w.late->pq = late ? nb : 0;
+  if (step && !late) fin1(s, FIN_PQ, nb, w, sc, (int*)fl, nullptr);
 }
 
 __global__ void k_filter_n2e(Geo g, const uint8_t* __restrict__ emask, const double* __restrict__ u,

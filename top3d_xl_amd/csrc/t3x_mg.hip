@@ -524,7 +524,9 @@ void prolong_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, double 
   else
     hipLaunchKernelGGL((k_prolong_jacobi<2, TX, TR, TD, TO>), g, dim3(kBlock), 0, s, gf, gc, omega, zc, xc, rf, diag,
                        nmaskF, out, part, fl);
-  if (mode) launch_fin1(s, mode == 1 ? FIN_ZR_INIT : FIN_ZR_LOOP, (int)(g.x * g.y), *ws, sc, (int*)fl, nullptr);
+  const int nb = (int)(g.x * g.y);
+  if (mode == 1) launch_fin1(s, FIN_ZR_INIT, nb, *ws, sc, (int*)fl, nullptr);
+  if (mode == 2) launch_fin_zr(s, nb, 3 * gf.NN, *ws, sc, (int*)fl);
 }
 
 // x = omega * r / d on solid nodes (the 'Standard' cycle's pre-smoothing, 757)
