@@ -1171,8 +1171,7 @@ int filter_run(t3x_problem& P, int slot, const double* src, double* dst) {
   launch_pcg_init(s, sc, fl, P.P.tol / 10.0);          // 891
   launch_norm2(s, P.fb, NN, P.ws, &sc[SC_NORMB]);
   launch_fill(s, P.fx, 0.0, NN);
-  launch_filter_apply(s, g0, kern, P.lv[0].emask, P.fx, P.fq, nullptr, nullptr, nullptr);
-  launch_sub(s, P.fr, P.fb, P.fq, NN);
+  launch_copy(s, P.fr, P.fb, NN);  // the residual of x = 0
   launch_scale_diag(s, P.fz, dinv, P.fr, NN, &P.ws, sc, nullptr);
   launch_copy(s, P.fp, P.fz, NN);
   const int maxIT = P.P.maxIT;
