@@ -186,9 +186,13 @@ void k_apply_K_sf(Geo g, int zc, SfCoef cf, const TE* __restrict__ E,
 #pragma unroll
   for (int i = 0; i < 8; ++i) cst[i] = T(cf.k[i]);
   // staging: global loads a layer ahead into registers, LDS stores after the
-  // cell phase has released the buffer.  u is staged unmasked beside its
-  // fixation bits: the cells apply P_free when they read their nodes, and
-  // the node's own u and bits for the epilogue come from the same stage.
+  // cell phase has released the buffer.  u is staged with P_free applied, beside
+  // its fixation bits: the cells read their 12 values at once.  (Masked as they
+  // were read, each node's bits and values were a chain of LDS round trips under
+  // 12 execution masks: FP32 residual at 256x512x256 0.497 -> 0.483 ms, FP64
+  // K*p 0.613 -> 0.606, at 12x24x12 10.9 -> 10.2 us.)  A fixed node's own u is
+  // read again for the epilogue.  Loads two layers ahead, in a second register
+  // set, cost the third wave per SIMD (0.67 ms) and gave nothing on small grids.
   constexpr int NST = (CS + SF_T - 1) / SF_T;  // staged nodes per thread (2)
   T pu[NST][3], pe;
   uint8_t pf[NST];
@@ -222,9 +226,9 @@ void k_apply_K_sf(Geo g, int zc, SfCoef cf, const TE* __restrict__ E,
       const int t = tid + s2 * SF_T;
       if (t < CS) {
         const int hy = t % SF_HT, hx = t / SF_HT;
-        sU[(b * 3 + 0) * CS + hx * SF_HT + hy] = pu[s2][0];
-        sU[(b * 3 + 1) * CS + hx * SF_HT + hy] = pu[s2][1];
-        sU[(b * 3 + 2) * CS + hx * SF_HT + hy] = pu[s2][2];
+        sU[(b * 3 + 0) * CS + hx * SF_HT + hy] = (pf[s2] & 1) ? T(0) : pu[s2][0];
+        sU[(b * 3 + 1) * CS + hx * SF_HT + hy] = (pf[s2] & 2) ? T(0) : pu[s2][1];
+        sU[(b * 3 + 2) * CS + hx * SF_HT + hy] = (pf[s2] & 4) ? T(0) : pu[s2][2];
         sF[b][hx * SF_HT + hy] = pf[s2];
       }
     }
@@ -236,18 +240,16 @@ void k_apply_K_sf(Geo g, int zc, SfCoef cf, const TE* __restrict__ E,
   const bool gnode = ty < SF_NT && tx < SF_NT;
   const int yy = y0 + ty, xx = x0 + tx;
   const bool own = gnode && yy < g.NY && xx < g.NX;
-  // the 4 nodes of cell (cy, cx) in one staged layer, P_free applied as
-  // read, face-analysed
+  // the 4 nodes of cell (cy, cx) in one staged layer, face-analysed
   auto read_face = [&](int b, T F[3][4]) {
 #pragma unroll
     for (int a = 0; a < 4; ++a) {  // local nodes 0..3: the z = 0 face
       const int p = sf_pos(a);
       const int h = (cx + kLocDx[a]) * SF_HT + (cy + kLocDy[a]);
       const int o = (b * 3) * CS + h;
-      const uint8_t fa = sF[b][h];
-      F[0][p] = (fa & 1) ? T(0) : sU[o];
-      F[1][p] = (fa & 2) ? T(0) : sU[o + CS];
-      F[2][p] = (fa & 4) ? T(0) : sU[o + 2 * CS];
+      F[0][p] = sU[o];
+      F[1][p] = sU[o + CS];
+      F[2][p] = sU[o + 2 * CS];
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) face_analyse(F[c]);
@@ -297,11 +299,16 @@ void k_apply_K_sf(Geo g, int zc, SfCoef cf, const TE* __restrict__ E,
     {
       T Ft[3][4];
       read_face(bk1, Ft);
-      if (epi) {  // this node's bits and unmasked u, before its buffer is restaged
+      if (epi) {  // this node's bits and u, before its buffer is restaged
         const int h = (tx + 1) * SF_HT + (ty + 1);
         f = sF[bk][h];
 #pragma unroll
         for (int c = 0; c < 3; ++c) uo[c] = double(sU[(bk * 3 + c) * CS + h]);
+        if (f) {  // a fixed node's unmasked u
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            if ((f >> c) & 1) uo[c] = double(T(u[c * NN + n]));
+        }
       }
       T X[8], Yv[8], Z[8];
 #pragma unroll
