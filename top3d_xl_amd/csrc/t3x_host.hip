@@ -874,6 +874,11 @@ int assemble(t3x_problem& P) {
   return T3X_OK;
 }
 
+// the r.r of the update before a V-cycle, if it was left to the finest restriction
+static RrFold left_rr(t3x_problem& P, double* sc, const int* fl) {
+  return {P.ws.partials + kLateRR, fl && P.ws.late ? P.ws.late->rr : 0, sc, (int*)fl};
+}
+
 // ------------------------------------------------------------- V-cycle
 // Solving_Vcycle, 'Adapted' (747-781); fuse: z.r reduction into the last
 // prolongation (612 / 629).
@@ -883,7 +888,8 @@ void vcycle(t3x_problem& P, const double* r, double* z, double* sc, const int* f
   double* tmp = (double*)P.rtmp;
   hipEvent_t ev[2], ec[2];
   P.tbegin(TG_VCYCLE, ev);
-  launch_restrict(s, geo(P.lv[0]), geo(P.lv[1]), P.lv[1].span, r, tmp, P.lv[1].nmask, P.lv[1].r, fl, P.fineAct());
+  launch_restrict(s, geo(P.lv[0]), geo(P.lv[1]), P.lv[1].span, r, tmp, P.lv[1].nmask, P.lv[1].r, fl, P.fineAct(),
+                  left_rr(P, sc, fl));
   for (int l = 1; l < L - 1; ++l)
     launch_restrict(s, geo(P.lv[l]), geo(P.lv[l + 1]), P.lv[l + 1].span, (const double*)P.lv[l].r, tmp,
                     P.lv[l + 1].nmask, P.lv[l + 1].r, fl);
@@ -908,7 +914,8 @@ void vcycle_mixed(t3x_problem& P, const double* r, float* z, double* sc, const i
   float* tmp = (float*)P.rtmp;
   hipEvent_t ev[2], ec[2];
   P.tbegin(TG_VCYCLE, ev);
-  launch_restrict(s, geo(P.lv[0]), geo(P.lv[1]), P.lv[1].span, r, tmp, P.lv[1].nmask, P.lv[1].rf, fl, P.fineAct());
+  launch_restrict(s, geo(P.lv[0]), geo(P.lv[1]), P.lv[1].span, r, tmp, P.lv[1].nmask, P.lv[1].rf, fl, P.fineAct(),
+                  left_rr(P, sc, fl));
   for (int l = 1; l < L - 1; ++l)
     launch_restrict(s, geo(P.lv[l]), geo(P.lv[l + 1]), P.lv[l + 1].span, (const float*)P.lv[l].rf, tmp,
                     P.lv[l + 1].nmask, P.lv[l + 1].rf, fl);
@@ -1055,6 +1062,7 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
   int its = maxIT;
   bool done = false;
   const LateScope late(P.ws);
+  const int rrBlocks = P.standard() ? 0 : restrict_rr_blocks(g0, geo(P.lv[1]), P.lv[1].span);
   // one iteration: K*p (614-615), r and the residual norm (617-622), z = M r
   // (628-629), y and p (616, 630)
   auto iteration = [&]() {
@@ -1065,7 +1073,7 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
     if (mx && P.standard())  // 617-622, with the first fine Jacobi step of 628-629 fused
       launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, P.lv[0].diagf, P.x32, P.P.omega, P.fineAct());
     else
-      launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct());  // 617-622
+      launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct(), rrBlocks);  // 617-622
     if (mx) {
       if (P.standard()) vcycle_standard(P, P.r, P.z32, sc, fl, true, true);                // 628-629
       else vcycle_mixed(P, P.r, P.z32, sc, fl, true);
@@ -1180,7 +1188,8 @@ int filter_run(t3x_problem& P, int slot, const double* src, double* dst) {
   const LateScope late(P.ws);
   for (int it = 1; it <= maxIT; ++it) {
     launch_filter_apply(s, g0, kern, P.lv[0].emask, P.fp, P.fq, &P.ws, sc, fl);
-    launch_pcg_update(s, P.fx, P.fr, P.fp, P.fq, NN, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct());
+    launch_pcg_update(s, P.fx, P.fr, P.fp, P.fq, NN, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct(),
+                      scale_diag_blocks(NN));
     launch_scale_diag(s, P.fz, dinv, P.fr, NN, &P.ws, sc, fl);
     launch_pcg_pupdate(s, P.fx, P.fp, P.fz, NN, P.ws, sc, fl, P.fineAct());
     if (it % ce == 0 || it == maxIT) {

@@ -61,15 +61,23 @@ __device__ __forceinline__ long long act_node(const Act& a, long long g) {
 // late: where set (by the solver's loop), p.q and z.r of few partials are left
 // for the vector update that consumes them to fold in every block of its own;
 // late->pq, late->zr: how many there are (0: folded).  A left p.q lies at
-// partials + kLateAt: the update that folds it writes partials of its own.
-constexpr int kLateAt = 32768;
+// partials + kLateAt: the update that folds it writes partials of its own.  r.r
+// is left (at partials + kLateRR) for the kernel after the update, where that is
+// the filter's scaling or the finest restriction.
+constexpr int kLateAt = 32768, kLateRR = 49152;
 struct LateFold {
-  int pq = 0, zr = 0;
+  int pq = 0, zr = 0, rr = 0;
 };
 struct RedWs {
   double* partials;
   unsigned int* counter;
   LateFold* late = nullptr;
+};
+struct RrFold {  // a left r.r
+  const double* partials = nullptr;
+  int nb = 0;
+  double* sc = nullptr;
+  int* fl = nullptr;
 };
 
 // One-block finalisers: fold nb partials in a fixed order, then apply the
@@ -133,10 +141,14 @@ void launch_galerkin_coarse(hipStream_t s, const Geo& gf, const Geo& gc, const d
 long long restrict_tmp_len(const Geo& gf, const Geo& gc);
 // actF: the fine level's chunk flags (finest level only; the y pass reads no
 // fine value from a void chunk).
+// rr: an r.r left by the update of rf (restrict_rr_blocks tells whether it may be)
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const double* rf, double* tmp,
-                     const uint8_t* nmaskC, double* rc, const int* fl, Act actF = {});
+                     const uint8_t* nmaskC, double* rc, const int* fl, Act actF = {}, RrFold rr = {});
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const double* rf, float* tmp,
-                     const uint8_t* nmaskC, float* rc, const int* fl, Act actF = {});
+                     const uint8_t* nmaskC, float* rc, const int* fl, Act actF = {}, RrFold rr = {});
+// the blocks of an FP64 restriction that can fold a left r.r (0: it cannot)
+int restrict_rr_blocks(const Geo& gf, const Geo& gc, int span);
+int scale_diag_blocks(long long n);  // the same of launch_scale_diag
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const float* rf, float* tmp,
                      const uint8_t* nmaskC, float* rc, const int* fl, Act actF = {});
 void launch_prolong_jacobi(hipStream_t s, const Geo& gf, const Geo& gc, int span, double omega, const double* xc,
@@ -211,9 +223,10 @@ void launch_norm2(hipStream_t s, const double* v, long long n, const RedWs& ws, 
 void launch_dot(hipStream_t s, const double* a, const double* b, long long n, const RedWs& ws, double* out);
 // r -= lambda q with r.r; with xj, also xj = omega r / dj (first Jacobi step of
 // the FP32 'Standard' V-cycle).  y and p are updated later by launch_pcg_pupdate.
+// rrBlocks: blocks of the kernel after it, if that one folds a left r.r.
 void launch_pcg_update(hipStream_t s, double* y, double* r, const double* p, const double* q, long long n,
                        const RedWs& ws, double* sc, int* fl, const float* dj = nullptr, float* xj = nullptr,
-                       double omega = 0.0, Act act = {});
+                       double omega = 0.0, Act act = {}, int rrBlocks = 0);
 void launch_pcg_pupdate(hipStream_t s, double* y, double* p, const double* z, long long n, const RedWs& ws, double* sc,
                         const int* fl, Act act = {});
 void launch_pcg_finish(hipStream_t s, double* y, const double* p, long long n, const double* sc, const int* fl,

@@ -38,7 +38,6 @@ inline int grid_for(long long n) {
 // One-block finalisers: fold a reduction's partials (fixed order) and apply
 // the scalar logic of the solver step that consumes it.
 // =========================================================================
-constexpr int kFinBlock = 1024;  // the finaliser's threads (wide folds of up to kMaxPartials partials)
 __global__ __launch_bounds__(kFinBlock) void k_fin1(int op, int nb, const double* __restrict__ partials, double* sc,
                                                     int* fl, double* out) {
   if (fl && fl[FL_DONE]) return;
@@ -79,18 +78,18 @@ __global__ __launch_bounds__(kFinBlock) void k_fin1(int op, int nb, const double
 void launch_fin1(hipStream_t s, int op, int nb, const RedWs& ws, double* sc, int* fl, double* out) {
   hipLaunchKernelGGL(k_fin1, dim3(1), dim3(kFinBlock), 0, s, op, nb, ws.partials, sc, fl, out);
 }
-// Whether the nb partials of a dot product are left for the update of n elements
-// that needs it: a launch less (2.4 to 3.3 us) against a fold in each of its
-// blocks (0.4 us at 12x24x12, 1.2 at 50x100x50).  The line, in partials read by
-// all its blocks together: 32x64x32 5.61 -> 5.30 ms for a design iteration,
+// Whether the nb partials of a dot product are left for the kernel of `blocks`
+// blocks that needs it: a launch less (2.4 to 3.3 us) against a fold in each of
+// its blocks (0.4 us at 12x24x12, 1.2 at 50x100x50).  The line, in partials read
+// by all its blocks together: 32x64x32 5.61 -> 5.30 ms for a design iteration,
 // 50x100x50 (1.1 M) 8.63 -> 8.41; 64x128x64 (3.6 to 5 M) 10.57 -> 10.80.
 constexpr long long kLateReads = 1 << 21;
-static bool late_fold(const RedWs& ws, int nb, long long n) {
+static bool late_fold(const RedWs& ws, int nb, long long blocks) {
   static_assert(kLateAt + 4 * kFinBlock <= kMaxPartials, "room for a left p.q");
-  return ws.late && nb <= 4 * kFinBlock && nb * ((n + kBlock - 1) / kBlock) <= kLateReads;
+  return ws.late && nb <= 4 * kFinBlock && nb * blocks <= kLateReads;
 }
 void launch_fin_zr(hipStream_t s, int nb, long long n, const RedWs& ws, double* sc, int* fl) {
-  const bool late = late_fold(ws, nb, n);
+  const bool late = late_fold(ws, nb, stream_blocks(n));
   if (ws.late) ws.late->zr = late ? nb : 0;
   if (!late) launch_fin1(s, FIN_ZR_LOOP, nb, ws, sc, fl, nullptr);
 }
@@ -114,7 +113,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_max(int nb, const double* __rest
 void launch_apply_K(hipStream_t s, const Geo& g, const SfCoef& cf, const double* E, const uint8_t* fix,
                     const double* u, double* y, const RedWs& ws, double* sc, const int* fl, bool pcgStep) {
   const int nb = applyk_sf_blocks(g);
-  const bool late = pcgStep && late_fold(ws, nb, 3 * g.NN);
+  const bool late = pcgStep && late_fold(ws, nb, stream_blocks(3 * g.NN));
   launch_apply_K_sf(s, g, cf, E, fix, u, y, pcgStep ? ws.partials + (late ? kLateAt : 0) : nullptr, fl);
   if (ws.late) ws.late->pq = late ? nb : 0;
   if (pcgStep && !late) fin1(s, FIN_PQ, nb, ws, sc, (int*)fl, nullptr);
@@ -757,29 +756,6 @@ void launch_dot(hipStream_t s, const double* a, const double* b, long long n, co
   fin1(s, FIN_SUM, red1_blocks(n), ws, nullptr, nullptr, out);
 }
 
-// The fold of k_fin1 in a block of kBlock threads, for up to 4 kFinBlock
-// partials: its threads' sums, its waves' sums and their sum in its order; the
-// total in every thread.
-__device__ __forceinline__ double fold_here(const double* p, int nb) {
-  constexpr int V = kFinBlock / kBlock;
-  __shared__ double sh[kFinBlock / 64];
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int v = 0; v < V; ++v) {
-    double a[4] = {};
-    const int b = threadIdx.x + v * kBlock;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (b + u * kFinBlock < nb) a[u] += p[b + u * kFinBlock];
-    const double s = v * kBlock < nb ? wave_sum((a[0] + a[2]) + (a[1] + a[3])) : 0.0;
-    if ((threadIdx.x & 63) == 0) sh[w + v * (kBlock / 64)] = s;
-  }
-  __syncthreads();
-  double s = 0.0;
-#pragma unroll
-  for (int k = 0; k < kFinBlock / 64; ++k) s += sh[k];
-  return s;
-}
 // y += lambda p ; r -= lambda q ; resnorm = ||r|| / ||b|| ; convergence flag.
 // r -= lambda q (617) with the r.r reduction.  With xj given (FP32 'Standard'
 // V-cycle), also the first fine Jacobi step of the next preconditioner
@@ -787,7 +763,7 @@ __device__ __forceinline__ double fold_here(const double* p, int nb) {
 __global__ __launch_bounds__(kBlock) void k_pcg_update(double* __restrict__ r, const double* __restrict__ q,
                                                        long long n, RedWs ws, double* sc, int* fl,
                                                        const float* __restrict__ dj, float* __restrict__ xj,
-                                                       double omega, Act act) {
+                                                       double omega, Act act, double* part) {
   if (fl[FL_DONE]) return;
   // y += lambda p (616) is deferred to k_pcg_pupdate, which reads p anyway
   const double lambda = sc[SC_LAMBDA];
@@ -809,13 +785,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(double* __restrict__ r, c
     }
   }
   double v[1] = {rr};
-  write_partials<1>(v, ws.partials);
+  write_partials<1>(v, part);
 }
 // the same with p.q still to be folded
 __global__ __launch_bounds__(kBlock) void k_pcg_update_late(double* __restrict__ r, const double* __restrict__ q,
                                                        long long n, RedWs ws, double* sc, int* fl,
                                                        const float* __restrict__ dj, float* __restrict__ xj,
-                                                       double omega, Act act, int nbPQ) {
+                                                       double omega, Act act, double* part,
+                                                            int nbPQ) {
   if (fl[FL_DONE]) return;
   // y += lambda p (616) is deferred to k_pcg_pupdate, which reads p anyway
   const long long m = act_items(act, n);
@@ -846,19 +823,24 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_late(double* __restrict__
     for (int c = 1; c < nc; ++c) element(b + c * act.NN, r[b + c * act.NN], q[b + c * act.NN]);
   }
   double v[1] = {rr};
-  write_partials<1>(v, ws.partials);
+  write_partials<1>(v, part);
 }
 void launch_pcg_update(hipStream_t s, double* y, double* r, const double* p, const double* q, long long n,
-                       const RedWs& ws, double* sc, int* fl, const float* dj, float* xj, double omega, Act act) {
+                       const RedWs& ws, double* sc, int* fl, const float* dj, float* xj, double omega, Act act,
+                       int rrBlocks) {
   (void)y;
   (void)p;
   const int nb = red1_blocks(act_items(act, n));
+  const bool late = rrBlocks && late_fold(ws, nb, rrBlocks);
+  if (ws.late) ws.late->rr = late ? nb : 0;
+  double* part = ws.partials + (late ? kLateRR : 0);
   const int nbPQ = ws.late ? ws.late->pq : 0;
   if (nbPQ)
-    hipLaunchKernelGGL(k_pcg_update_late, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act, nbPQ);
+    hipLaunchKernelGGL(k_pcg_update_late, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act, part,
+                       nbPQ);
   else
-    hipLaunchKernelGGL(k_pcg_update, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act);
-  fin1(s, FIN_RR, nb, ws, sc, fl, nullptr);
+    hipLaunchKernelGGL(k_pcg_update, dim3(nb), dim3(kBlock), 0, s, r, q, n, ws, sc, fl, dj, xj, omega, act, part);
+  if (!late) fin1(s, FIN_RR, nb, ws, sc, fl, nullptr);
 }
 
 // y += lambda p (616) for the iteration just finished, then p = z + beta p (630).
@@ -963,26 +945,42 @@ void launch_pcg_init(hipStream_t s, double* sc, int* fl, double tol) {
   hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(1), 0, s, sc, fl, tol);
 }
 
-// z = dinv .* r (889) with the fused z.r reduction.
+// z = dinv .* r (889) with the fused z.r reduction; RR: the update before it left
+// r.r to be folded here (then one element per thread).
+template <bool RR>
 __global__ __launch_bounds__(kBlock) void k_scale_diag(double* __restrict__ z, const double* __restrict__ dinv,
                                                        const double* __restrict__ r, long long n, RedWs ws,
-                                                       double* sc, const int* fl, int mode) {
+                                                       const int* fl, RrFold rr) {
   if (fl && fl[FL_DONE]) return;
   double zr = 0.0;
-  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) {
-    const double zi = dinv[i] * r[i];
-    z[i] = zi;
-    zr += zi * r[i];
+  const long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (RR) {
+    const double r0 = i0 < n ? r[i0] : 0.0, d0 = i0 < n ? dinv[i0] : 0.0;  // beside the fold
+    if (rr_fold(rr)) return;
+    if (i0 < n) {
+      const double zi = d0 * r0;
+      z[i0] = zi;
+      zr += zi * r0;
+    }
+  } else {
+    for (long long i = i0; i < n; i += (long long)gridDim.x * kBlock) {
+      const double zi = dinv[i] * r[i];
+      z[i] = zi;
+      zr += zi * r[i];
+    }
   }
   double v[1] = {zr};
   write_partials<1>(v, ws.partials);
-  (void)mode;
 }
+int scale_diag_blocks(long long n) { return red1_blocks(n); }
 void launch_scale_diag(hipStream_t s, double* z, const double* dinv, const double* r, long long n,
                        const RedWs* ws, double* sc, const int* fl) {
-  const int mode = fl ? 2 : 1;
-  hipLaunchKernelGGL(k_scale_diag, dim3(red1_blocks(n)), dim3(kBlock), 0, s, z, dinv, r, n, *ws, sc, fl, mode);
-  if (mode == 1) fin1(s, FIN_ZR_INIT, red1_blocks(n), *ws, sc, (int*)fl, nullptr);
+  const RrFold rr{ws->partials + kLateRR, ws->late ? ws->late->rr : 0, sc, (int*)fl};
+  if (fl && rr.nb)
+    hipLaunchKernelGGL(k_scale_diag<true>, dim3(red1_blocks(n)), dim3(kBlock), 0, s, z, dinv, r, n, *ws, fl, rr);
+  else
+    hipLaunchKernelGGL(k_scale_diag<false>, dim3(red1_blocks(n)), dim3(kBlock), 0, s, z, dinv, r, n, *ws, fl, rr);
+  if (!fl) fin1(s, FIN_ZR_INIT, red1_blocks(n), *ws, sc, (int*)fl, nullptr);
   else launch_fin_zr(s, red1_blocks(n), n, *ws, sc, (int*)fl);
 }
 
@@ -1139,7 +1137,7 @@ void launch_filter_apply(hipStream_t s, const Geo& g, const double* kern, const 
   int zc = 8;
   const dim3 grid = filter_grid(g, zc);
   const int nb = (int)(grid.x * grid.y * grid.z);
-  const bool late = step && late_fold(w, nb, g.NN);
+  const bool late = step && late_fold(w, nb, stream_blocks(g.NN));
   RedWs at = w;
   if (late) at.partials += kLateAt;
   hipLaunchKernelGGL(k_filter_apply, grid, dim3(kFaY, kFaX), 0, s, g, zc, kern, emask, u, y, at, fl, step);

@@ -75,9 +75,9 @@ __global__ __launch_bounds__(kBlock) void k_restrict_y(Geo gf, int NYc, const TI
 // weights and summation order of k_restrict_y, so the result is the same.
 // The direct kernel's loads are stride S across lanes, each fine value read
 // by 2 S - 1 threads.
-template <int S, typename TI, typename TM>
+template <int S, typename TI, typename TM, bool RR>
 __global__ __launch_bounds__(kBlock) void k_restrict_y_lds(Geo gf, int NYc, int R, const TI* __restrict__ rf,
-                                                           TM* __restrict__ tmp, const int* fl, Act actF) {
+                                                           TM* __restrict__ tmp, const int* fl, Act actF, RrFold rr) {
   if (fl && fl[FL_DONE]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   TI* sv = (TI*)smem;  // [component][R NY]
@@ -105,6 +105,9 @@ __global__ __launch_bounds__(kBlock) void k_restrict_y_lds(Geo gf, int NYc, int 
         for (int c = 0; c < 3; ++c) sv[c * cs + i] = v[c][u];
       }
     }
+  }
+  if (RR) {
+    if (rr_fold(rr)) return;
   }
   __syncthreads();
   const long long TN = (long long)NYc * rows;
@@ -449,9 +452,18 @@ constexpr long long kOnceOut = 65536;        // coarse nodes up to which a span-
 constexpr long long kXzWideOut = 131072;     // coarse nodes up to which the x-z pass runs its planes side by side
 constexpr size_t kRestrictLds = 48 * 1024;  // LDS bytes of the y pass's rows at most
 
+// the LDS y pass: about one intermediate value per thread (R rows a block)
+// while the rows fit kRestrictLds bytes; its blocks (0: it does not apply)
+unsigned y_lds_blocks(const Geo& gf, const Geo& gc, size_t elem, int* R, size_t* lds) {
+  *R = std::max(1, (kBlock + gc.NY / 2) / gc.NY);
+  *lds = (size_t)*R * gf.NY * 3 * elem;
+  const long long n = ((long long)gf.NX * gf.NZ + *R - 1) / *R;
+  return *lds <= kRestrictLds && n <= 0x7fffffffLL ? (unsigned)n : 0;
+}
+
 template <typename TI, typename TM, typename TO>
 void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const TI* rf, TM* tmp,
-                   const uint8_t* nmaskC, TO* rc, const int* fl, Act actF) {
+                   const uint8_t* nmaskC, TO* rc, const int* fl, Act actF, RrFold rr = {}) {
   const int plane = gc.NY * gf.NX;
   // span 2: both passes in one launch while the launch saved is worth the values
   // read 3.4 times over.  637 outputs 4.6 us against 7.1, 9,537 5.2 / 9.6, 31,213
@@ -463,21 +475,23 @@ void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const 
     return;
   }
   const dim3 g1((plane + kBlock - 1) / kBlock, gf.NZ);
-  // the LDS y pass: about one intermediate value per thread (R rows a block)
-  // while the rows fit kRestrictLds bytes
-  const int R = std::max(1, (kBlock + gc.NY / 2) / gc.NY);
-  const size_t lds = (size_t)R * gf.NY * 3 * sizeof(TI);
-  const long long rows = (long long)gf.NX * gf.NZ;
-  const bool viaLds = lds <= kRestrictLds && (rows + R - 1) / R <= 0x7fffffffLL;
-  const dim3 gl((unsigned)((rows + R - 1) / R));
+  int R = 0;
+  size_t lds = 0;
+  const unsigned viaLds = y_lds_blocks(gf, gc, sizeof(TI), &R, &lds);
+  const dim3 gl(viaLds);
   if (span == 4) {
-    if (viaLds)
-      hipLaunchKernelGGL((k_restrict_y_lds<4, TI, TM>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl, actF);
+    if (viaLds && rr.nb)
+      hipLaunchKernelGGL((k_restrict_y_lds<4, TI, TM, true>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl, actF,
+                         rr);
+    else if (viaLds)
+      hipLaunchKernelGGL((k_restrict_y_lds<4, TI, TM, false>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl,
+                         actF, rr);
     else
       hipLaunchKernelGGL((k_restrict_y<4, TI, TM>), g1, dim3(kBlock), 0, s, gf, gc.NY, rf, tmp, fl, actF);
   } else {
     if (viaLds)
-      hipLaunchKernelGGL((k_restrict_y_lds<2, TI, TM>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl, actF);
+      hipLaunchKernelGGL((k_restrict_y_lds<2, TI, TM, false>), gl, dim3(kBlock), lds, s, gf, gc.NY, R, rf, tmp, fl,
+                         actF, rr);
     else
       hipLaunchKernelGGL((k_restrict_y<2, TI, TM>), g1, dim3(kBlock), 0, s, gf, gc.NY, rf, tmp, fl, actF);
   }
@@ -553,12 +567,17 @@ __global__ __launch_bounds__(kBlock) void k_jacobi0(const TR* __restrict__ r, co
 long long restrict_tmp_len(const Geo& gf, const Geo& gc) { return 3LL * gc.NY * gf.NX * gf.NZ; }
 
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const double* rf, double* tmp,
-                     const uint8_t* nmaskC, double* rc, const int* fl, Act actF) {
-  restrict_impl<double, double, double>(s, gf, gc, span, rf, tmp, nmaskC, rc, fl, actF);
+                     const uint8_t* nmaskC, double* rc, const int* fl, Act actF, RrFold rr) {
+  restrict_impl<double, double, double>(s, gf, gc, span, rf, tmp, nmaskC, rc, fl, actF, rr);
 }
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const double* rf, float* tmp,
-                     const uint8_t* nmaskC, float* rc, const int* fl, Act actF) {
-  restrict_impl<double, float, float>(s, gf, gc, span, rf, tmp, nmaskC, rc, fl, actF);
+                     const uint8_t* nmaskC, float* rc, const int* fl, Act actF, RrFold rr) {
+  restrict_impl<double, float, float>(s, gf, gc, span, rf, tmp, nmaskC, rc, fl, actF, rr);
+}
+int restrict_rr_blocks(const Geo& gf, const Geo& gc, int span) {
+  int R = 0;
+  size_t lds = 0;
+  return span == 4 ? (int)y_lds_blocks(gf, gc, sizeof(double), &R, &lds) : 0;
 }
 void launch_restrict(hipStream_t s, const Geo& gf, const Geo& gc, int span, const float* rf, float* tmp,
                      const uint8_t* nmaskC, float* rc, const int* fl, Act actF) {

@@ -10,6 +10,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "t3x_kernels.h"
+
 namespace t3x {
 
 constexpr int kBlock = 256;
@@ -151,6 +153,48 @@ __device__ __forceinline__ void fold_partials(const double* partials, int nb, do
     out[i] = a[0];
   }
   block_sum<NV, NT>(out);
+}
+
+constexpr int kFinBlock = 1024;  // the finaliser's threads (wide folds of up to kMaxPartials partials)
+// The fold of k_fin1 in a block of kBlock threads, for up to 4 kFinBlock
+// partials: its threads' sums, its waves' sums and their sum in its order; the
+// total in every thread.
+__device__ __forceinline__ double fold_here(const double* p, int nb) {
+  constexpr int V = kFinBlock / kBlock;
+  __shared__ double sh[kFinBlock / 64];
+  const int w = threadIdx.x >> 6;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    double a[4] = {};
+    const int b = threadIdx.x + v * kBlock;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (b + u * kFinBlock < nb) a[u] += p[b + u * kFinBlock];
+    const double s = v * kBlock < nb ? wave_sum((a[0] + a[2]) + (a[1] + a[3])) : 0.0;
+    if ((threadIdx.x & 63) == 0) sh[w + v * (kBlock / 64)] = s;
+  }
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < kFinBlock / 64; ++k) s += sh[k];
+  return s;
+}
+// FIN_RR in every block of the kernel after the residual's update; true: the
+// solve has converged
+__device__ __forceinline__ bool rr_fold(const RrFold& f) {
+  const double t = fold_here(f.partials, f.nb), res = sqrt(t) / f.sc[SC_NORMB];
+  const bool done = res < f.sc[SC_TOL];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // (the flag may reach blocks that start later: they would return here)
+    f.sc[SC_RR] = t;
+    f.sc[SC_RES] = res;
+    const int it = f.fl[FL_ITER] + 1;
+    f.fl[FL_ITER] = it;
+    if (done) {
+      f.fl[FL_DONE] = 1;
+      f.fl[FL_ITS] = it;
+    }
+  }
+  return done;
 }
 
 __device__ __forceinline__ double fold_max(const double* partials, int nb) {
