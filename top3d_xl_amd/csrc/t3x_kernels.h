@@ -198,18 +198,8 @@ void launch_coarse_resid64(hipStream_t s, const Geo& g, const double* Ks, const 
 void launch_coarse_smooth64(hipStream_t s, const Geo& g, const double* Ks, const double* x, const double* r,
                             const double* diag, double omega, double* out, double* tmp, const int* fl,
                             const uint8_t* emask, const uint8_t* nmask);
-void launch_coarse_gather(hipStream_t s, int n, const long long* map, const double* r, double* v, const int* fl);
-void launch_coarse_gather(hipStream_t s, int n, const long long* map, const float* r, double* v, const int* fl);
-void launch_coarse_scatter(hipStream_t s, int n, const long long* map, const double* v, double* x, long long NN3,
-                           const int* fl);
-void launch_coarse_scatter(hipStream_t s, int n, const long long* map, const double* v, float* x, long long NN3,
-                           const int* fl);
 void launch_band_assemble(hipStream_t s, const Geo& g, const double* Ks, const uint8_t* emask, const int* nodePos,
                           int bw, double* band, long long nBand);
-int launch_band_factor(hipStream_t s, int n, int bw, double* band, int* status);
-void launch_band_post(hipStream_t s, int n, int bw, int nb, const double* band, double* bandT, double* dinv);
-void launch_band_solve(hipStream_t s, int n, int bw, int nb, const double* band, const double* bandT,
-                       const double* dinv, double* v, const int* fl);
 
 // ---------------------------------------------------------------- vectors
 void launch_fill(hipStream_t s, double* p, double v, long long n);

@@ -479,38 +479,9 @@ void launch_galerkin_coarse(hipStream_t s, const Geo& gf, const Geo& gc, const d
 // Multigrid transfers (783-814) live in t3x_mg.hip.
 
 // =========================================================================
-// Coarsest level: banded Cholesky (1052-1065) and solves (767).
+// Coarsest level: assembly of its band (1052-1065; factored and solved in t3x_coarse.hip).
 // Band storage: row i holds L(i, i-k) at band[i*W + k], W = bw+1.
 // =========================================================================
-template <typename TR>
-__global__ void k_coarse_gather(int n, const long long* __restrict__ map, const TR* __restrict__ r,
-                                double* __restrict__ v, const int* fl) {
-  if (fl && fl[FL_DONE]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) v[i] = (double)r[map[i]];
-}
-void launch_coarse_gather(hipStream_t s, int n, const long long* map, const double* r, double* v, const int* fl) {
-  hipLaunchKernelGGL(k_coarse_gather<double>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, map, r, v, fl);
-}
-void launch_coarse_gather(hipStream_t s, int n, const long long* map, const float* r, double* v, const int* fl) {
-  hipLaunchKernelGGL(k_coarse_gather<float>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, map, r, v, fl);
-}
-template <typename TX>
-__global__ void k_coarse_scatter(int n, const long long* __restrict__ map, const double* __restrict__ v,
-                                 TX* __restrict__ x, const int* fl) {
-  if (fl && fl[FL_DONE]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) x[map[i]] = (TX)v[i];
-}
-void launch_coarse_scatter(hipStream_t s, int n, const long long* map, const double* v, double* x, long long,
-                           const int* fl) {
-  hipLaunchKernelGGL(k_coarse_scatter<double>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, map, v, x, fl);
-}
-void launch_coarse_scatter(hipStream_t s, int n, const long long* map, const double* v, float* x, long long,
-                           const int* fl) {
-  hipLaunchKernelGGL(k_coarse_scatter<float>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, map, v, x, fl);
-}
-
 // Assembly of the lower band: one thread per (coarsest node a, node b of its
 // 3x3x3 neighbourhood) sums the 3x3 entries of rows a, columns b over the
 // cells that hold both, in the cells' order, and writes them once.  Bound: one
@@ -564,141 +535,6 @@ void launch_band_assemble(hipStream_t s, const Geo& g, const double* Ks, const u
                           int bw, double* band, long long nBand) {
   launch_fill(s, band, 0.0, nBand);
   hipLaunchKernelGGL(k_band_assemble, dim3(grid_for(27 * g.NN)), dim3(kBlock), 0, s, g, Ks, emask, nodePos, bw, band);
-}
-
-// Right-looking banded Cholesky in one work-group.
-constexpr int kFactBlock = 1024;
-__global__ __launch_bounds__(kFactBlock) void k_band_factor(int n, int bw, double* __restrict__ B, int* status) {
-  const int W = bw + 1;
-  __shared__ double shd;
-  __shared__ int bad;
-  if (threadIdx.x == 0) bad = 0;
-  __syncthreads();
-  for (int j = 0; j < n; ++j) {
-    if (threadIdx.x == 0) {
-      const double a = B[(size_t)j * W];
-      if (!(a > 0.0)) bad = 1;
-      shd = sqrt(a);
-      B[(size_t)j * W] = shd;
-    }
-    __syncthreads();
-    if (bad) break;
-    const int iend = min(n - 1, j + bw);
-    const int m = iend - j;
-    const double d = shd;
-    for (int i = j + 1 + threadIdx.x; i <= iend; i += kFactBlock) B[(size_t)i * W + (i - j)] /= d;
-    __syncthreads();
-    const long long tot = (long long)m * (m + 1) / 2;
-    for (long long t = threadIdx.x; t < tot; t += kFactBlock) {
-      int ii = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-      while ((long long)(ii + 1) * (ii + 2) / 2 <= t) ++ii;
-      while ((long long)ii * (ii + 1) / 2 > t) --ii;
-      const int kk = (int)(t - (long long)ii * (ii + 1) / 2);
-      const int i = j + 1 + ii, k = j + 1 + kk;  // k <= i
-      B[(size_t)i * W + (i - k)] -= B[(size_t)i * W + (i - j)] * B[(size_t)k * W + (k - j)];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *status = bad;
-}
-int launch_band_factor(hipStream_t s, int n, int bw, double* band, int* status) {
-  hipLaunchKernelGGL(k_band_factor, dim3(1), dim3(kFactBlock), 0, s, n, bw, band, status);
-  return 0;
-}
-
-// Transposed band (bandT[i*W+k] = L(i+k, i)) and inverses of the nb x nb
-// diagonal blocks (row-major lower triangles), one block per work-group.
-__global__ void k_band_transpose(int n, int bw, const double* __restrict__ B, double* __restrict__ BT) {
-  const int W = bw + 1;
-  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= (long long)n * W) return;
-  const int i = (int)(t / W), k = (int)(t % W);
-  BT[t] = (i + k < n) ? B[(size_t)(i + k) * W + k] : 0.0;
-}
-__global__ void k_band_dinv(int n, int bw, int nb, const double* __restrict__ B, double* __restrict__ Dinv) {
-  const int W = bw + 1;
-  const int r0 = blockIdx.x * nb;
-  const int m = min(nb, n - r0);
-  double* D = Dinv + (size_t)blockIdx.x * nb * nb;
-  const int c = threadIdx.x;  // column of the inverse
-  if (c >= nb) return;
-  for (int i = 0; i < nb; ++i) D[(size_t)i * nb + c] = 0.0;
-  if (c >= m) return;
-  auto L = [&](int i, int k) { return (i - k <= bw) ? B[(size_t)(r0 + i) * W + (i - k)] : 0.0; };
-  D[(size_t)c * nb + c] = 1.0 / L(c, c);
-  for (int i = c + 1; i < m; ++i) {
-    double s = 0.0;
-    for (int k = c; k < i; ++k) s += L(i, k) * D[(size_t)k * nb + c];
-    D[(size_t)i * nb + c] = -s / L(i, i);
-  }
-}
-void launch_band_post(hipStream_t s, int n, int bw, int nb, const double* band, double* bandT, double* dinv) {
-  const long long tot = (long long)n * (bw + 1);
-  hipLaunchKernelGGL(k_band_transpose, dim3(grid_for(tot)), dim3(kBlock), 0, s, n, bw, band, bandT);
-  const int nblk = (n + nb - 1) / nb;
-  hipLaunchKernelGGL(k_band_dinv, dim3(nblk), dim3(nb), 0, s, n, bw, nb, band, dinv);
-}
-
-// Forward and backward substitution in one work-group, nb = 64 rows per step:
-// the off-block part is a GEMV over the band, the block part a GEMV with the
-// precomputed diagonal-block inverse.
-constexpr int kSolveNb = 64;
-__global__ __launch_bounds__(kBlock) void k_band_solve(int n, int bw, const double* __restrict__ B,
-                                                       const double* __restrict__ BT,
-                                                       const double* __restrict__ Dinv, double* __restrict__ v,
-                                                       const int* fl) {
-  if (fl && fl[FL_DONE]) return;
-  const int W = bw + 1, nb = kSolveNb;
-  __shared__ double sh[kSolveNb];
-  const int nblk = (n + nb - 1) / nb;
-  const int row = threadIdx.x >> 2, lane = threadIdx.x & 3;
-  // forward: L y = v
-  for (int b = 0; b < nblk; ++b) {
-    const int r0 = b * nb, m = min(nb, n - r0);
-    if (row < m) {
-      const int i = r0 + row;
-      const int k0 = max(0, i - bw);
-      double s = 0.0;
-      for (int k = k0 + lane; k < r0; k += 4) s += B[(size_t)i * W + (i - k)] * v[k];
-      s += __shfl_xor(s, 1, 64);
-      s += __shfl_xor(s, 2, 64);
-      if (lane == 0) sh[row] = v[i] - s;
-    }
-    __syncthreads();
-    if (threadIdx.x < m) {
-      const double* D = Dinv + (size_t)b * nb * nb + (size_t)threadIdx.x * nb;
-      double y = 0.0;
-      for (int j = 0; j <= (int)threadIdx.x; ++j) y += D[j] * sh[j];
-      v[r0 + threadIdx.x] = y;
-    }
-    __syncthreads();
-  }
-  // backward: L^T x = y
-  for (int b = nblk - 1; b >= 0; --b) {
-    const int r0 = b * nb, m = min(nb, n - r0), r1 = r0 + m;
-    if (row < m) {
-      const int i = r0 + row;
-      const int k1 = min(n - 1, i + bw);
-      double s = 0.0;
-      for (int k = r1 + lane; k <= k1; k += 4) s += BT[(size_t)i * W + (k - i)] * v[k];
-      s += __shfl_xor(s, 1, 64);
-      s += __shfl_xor(s, 2, 64);
-      if (lane == 0) sh[row] = v[i] - s;
-    }
-    __syncthreads();
-    if (threadIdx.x < m) {
-      const double* D = Dinv + (size_t)b * nb * nb;
-      double x = 0.0;
-      for (int j = threadIdx.x; j < m; ++j) x += D[(size_t)j * nb + threadIdx.x] * sh[j];
-      v[r0 + threadIdx.x] = x;
-    }
-    __syncthreads();
-  }
-}
-void launch_band_solve(hipStream_t s, int n, int bw, int nb, const double* band, const double* bandT,
-                       const double* dinv, double* v, const int* fl) {
-  (void)nb;
-  hipLaunchKernelGGL(k_band_solve, dim3(1), dim3(kBlock), 0, s, n, bw, band, bandT, dinv, v, fl);
 }
 
 // =========================================================================
