@@ -32,15 +32,18 @@ class HostStage {
   HostStage& operator=(const HostStage&) = delete;
 
  private:
-  static constexpr size_t kMinRing = 2 << 20, kMaxRing = 16 << 20;  // pinned bytes: by the largest copy so far
+  static constexpr size_t kMinRing = 256 << 10, kMaxRing = 16 << 20;  // pinned bytes: by the largest copy so far
   static constexpr int kMaxSlots = 32, kMaxThreads = 8;
   // A chunk costs the link 6 us beside its bytes (a kernel's start and end) and
   // the copy one chunk's memcpy; a thread 20 us to start.  15 MB down with 4
   // threads: 570, 450, 400 us in chunks of 256, 512, 1024 KB; 5 MB with one
   // thread 207, 167, 207.
-  static size_t chunk_of(size_t bytes) { return bytes < (8u << 20) ? 512 << 10 : bytes < (32u << 20) ? 1 << 20 : 2 << 20; }
+  static size_t chunk_of(size_t bytes) {
+    return bytes <= kMinRing ? kMinRing : bytes < (8u << 20) ? 512 << 10 : bytes < (32u << 20) ? 1 << 20 : 2 << 20;
+  }
   static int threads_of(size_t bytes) { return bytes < (8u << 20) ? 1 : bytes < (64u << 20) ? 4 : kMaxThreads; }
   bool reserve(size_t bytes);
+  hipError_t record(int slot, hipStream_t s);  // the slot's event, made when first used
   hipError_t move(char* dev, char* host, size_t bytes, bool up, hipStream_t s);
   hipError_t issue(struct StageJob& job, size_t c);
   hipError_t part(struct StageJob& job);

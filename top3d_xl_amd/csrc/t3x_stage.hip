@@ -51,12 +51,8 @@ bool HostStage::reserve(size_t bytes) {
   if (busy_ && hipEventSynchronize(ev_[last_]) != hipSuccess) return false;
   busy_ = false;
   char* ring = nullptr;
-  bool ok = hipHostMalloc((void**)&ring, want, hipHostMallocCoherent) == hipSuccess;
-  for (hipEvent_t& e : ev_)
-    if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-  if (!ok) {  // the ring that is there, if any, serves on
-    (void)hipGetLastError();
-    if (ring) (void)hipHostFree(ring);
+  if (hipHostMalloc((void**)&ring, want, hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();  // the ring that is there, if any, serves on
     failed_ = true;
     return ringBytes_ > 0;
   }
@@ -64,6 +60,14 @@ bool HostStage::reserve(size_t bytes) {
   ring_ = ring;
   ringBytes_ = want;
   return true;
+}
+
+hipError_t HostStage::record(int slot, hipStream_t s) {
+  if (!ev_[slot]) {
+    const hipError_t e = hipEventCreateWithFlags(&ev_[slot], hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+  }
+  return hipEventRecord(ev_[slot], s);
 }
 
 // Chunk c between its slot and the device, and the slot's event behind it
@@ -81,7 +85,7 @@ hipError_t HostStage::issue(StageJob& job, size_t c) {
     e = hipMemcpyAsync(job.up ? dev : pin, job.up ? pin : dev, n, job.up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost,
                        job.s);
   }
-  if (e == hipSuccess && (!job.up || c + job.slots < job.chunks)) e = hipEventRecord(ev_[slot], job.s);
+  if (e == hipSuccess && (!job.up || c + job.slots < job.chunks)) e = record(slot, job.s);
   job.issued[slot].store(c / job.slots + 1, std::memory_order_release);
   return e;
 }
@@ -116,7 +120,7 @@ hipError_t HostStage::part(StageJob& job) {
 }
 
 hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStream_t s) {
-  const size_t chunk = chunk_of(bytes);
+  const size_t chunk = std::min(chunk_of(bytes), ringBytes_);  // (a ring that could not grow)
   StageJob job{dev, host, bytes, chunk, (bytes + chunk - 1) / chunk, (int)std::min<size_t>(ringBytes_ / chunk, kMaxSlots),
                up, s};
   static_assert(sizeof(job.issued) / sizeof(job.issued[0]) == kMaxSlots, "a count per slot");
@@ -150,7 +154,7 @@ hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStre
   }
   if (up) {
     last_ = (int)((job.chunks - 1) % job.slots);
-    e = hipEventRecord(ev_[last_], s);
+    e = record(last_, s);
     busy_ = e == hipSuccess;
   } else {
     busy_ = false;
