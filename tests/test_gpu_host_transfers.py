@@ -67,3 +67,14 @@ def test_zero_start_is_the_zero_vector():
     a, c = p.pcg(b), p.pcg(b, x0=np.zeros(3 * p.nN))
     assert a[1] == c[1] and a[2] == c[2] and np.array_equal(a[0], c[0])
     p.close()
+
+
+def test_an_earlier_error_of_the_thread_is_not_the_transfer_s():
+    import top3d_xl_amd.t3x as t3x
+    p = t3x.Problem(np.ones((6, 8, 6), bool))
+    p.set_modulus(np.ones(p.nE))
+    u = np.random.default_rng(2).standard_normal(3 * p.nN)
+    y = p.apply_K(u)
+    assert p.L.hipSetDevice(4096) != 0  # refused by the runtime, and remembered as the thread's last error
+    assert np.array_equal(p.apply_K(u), y)
+    p.close()

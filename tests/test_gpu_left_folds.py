@@ -49,3 +49,27 @@ def test_pcg(shape):
     # the precision form stops at the same tolerance, which its recursive residual meets to rounding
     assert res < 1e-3 and np.linalg.norm(b - o.apply_K(xm)) < 1.01e-3 * np.linalg.norm(b)
     g.close(), m.close()
+
+
+def test_filter_of_a_few_cells_at_the_end_of_a_large_grid():
+    """20 M nodes, 64 solid cells: few partials, more elements than a block per
+    element's 256 threads can take; the same filter on those cells alone."""
+    import top3d_xl_amd as t3x
+    vox = np.zeros((2000, 4, 2000), bool)
+    vox[-4:, :, -4:] = True
+    ny, nx, nz = vox.shape
+    node = lambda y, x, z: y + (ny + 1) * (x + (nx + 1) * z)  # noqa: E731
+    fix = np.array([node(y, 0, z) for z in range(nz - 4, nz + 1) for y in range(ny - 4, ny + 1)])
+    load = np.array([node(ny - 2, 4, nz - 2)])
+    big = t3x.Problem(vox, (fix, np.ones((fix.size, 3), np.uint8)), (load, np.array([[0.0, 0.0, -1.0]])))
+    small = t3x.Problem(np.ones((4, 4, 4), bool))
+    try:
+        assert big.nE == small.nE == 64
+        src = np.random.default_rng(8).random(64)
+        out = []
+        for m in (big, small):
+            m.filter_setup(0, 2.5)
+            out.append(m.filter(0, src))
+        assert out[0][1] == out[1][1] and _rel(out[0][0], out[1][0]) < 1e-10
+    finally:
+        big.close(), small.close()

@@ -86,7 +86,8 @@ void launch_fin1(hipStream_t s, int op, int nb, const RedWs& ws, double* sc, int
 constexpr long long kLateReads = 1 << 21;
 static bool late_fold(const RedWs& ws, int nb, long long blocks) {
   static_assert(kLateAt + 4 * kFinBlock <= kMaxPartials, "room for a left p.q");
-  return ws.late && nb <= 4 * kFinBlock && nb * blocks <= kLateReads;
+  // (at most kMaxPartials blocks: the kernels that fold take one element per thread)
+  return ws.late && nb <= 4 * kFinBlock && blocks <= kMaxPartials && nb * blocks <= kLateReads;
 }
 void launch_fin_zr(hipStream_t s, int nb, long long n, const RedWs& ws, double* sc, int* fl) {
   const bool late = late_fold(ws, nb, stream_blocks(n));
@@ -808,7 +809,7 @@ __global__ __launch_bounds__(kBlock) void k_scale_diag(double* __restrict__ z, c
   double v[1] = {zr};
   write_partials<1>(v, ws.partials);
 }
-int scale_diag_blocks(long long n) { return red1_blocks(n); }
+int scale_diag_blocks(long long n) { return stream_blocks(n); }
 void launch_scale_diag(hipStream_t s, double* z, const double* dinv, const double* r, long long n,
                        const RedWs* ws, double* sc, const int* fl) {
   const RrFold rr{ws->partials + kLateRR, ws->late ? ws->late->rr : 0, sc, (int*)fl};

@@ -78,9 +78,11 @@ hipError_t HostStage::issue(StageJob& job, size_t c) {
   const size_t n = std::min(job.chunk, job.bytes - c * job.chunk);
   hipError_t e = hipSuccess;
   if ((uintptr_t)dev % 16 == 0) {
-    hipLaunchKernelGGL(k_stage_copy, dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0, job.s, job.up ? pin : dev,
-                       job.up ? dev : pin, (unsigned)n);
-    e = hipGetLastError();
+    const char* src = job.up ? pin : dev;
+    char* dst = job.up ? dev : pin;
+    unsigned len = (unsigned)n;
+    void* args[] = {&src, &dst, &len};  // (its own status: the thread's last error may be another call's)
+    e = hipLaunchKernel((const void*)k_stage_copy, dim3((len + 4095) / 4096), dim3(256), args, 0, job.s);
   } else {
     e = hipMemcpyAsync(job.up ? dev : pin, job.up ? pin : dev, n, job.up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost,
                        job.s);
