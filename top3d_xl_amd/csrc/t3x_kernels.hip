@@ -788,7 +788,7 @@ template <bool RR>
 __global__ __launch_bounds__(kBlock) void k_scale_diag(double* __restrict__ z, const double* __restrict__ dinv,
                                                        const double* __restrict__ r, long long n, RedWs ws,
                                                        const int* fl, RrFold rr) {
-  if (fl && fl[FL_DONE]) return;
+  if (!RR && fl && fl[FL_DONE]) return;  // RR: rr_fold looks
   double zr = 0.0;
   const long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (RR) {

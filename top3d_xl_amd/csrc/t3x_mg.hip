@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_y(Geo gf, int NYc, const TI
 template <int S, typename TI, typename TM, bool RR>
 __global__ __launch_bounds__(kBlock) void k_restrict_y_lds(Geo gf, int NYc, int R, const TI* __restrict__ rf,
                                                            TM* __restrict__ tmp, const int* fl, Act actF, RrFold rr) {
-  if (fl && fl[FL_DONE]) return;
+  if (!RR && fl && fl[FL_DONE]) return;  // RR: rr_fold looks
   extern __shared__ __align__(16) unsigned char smem[];
   TI* sv = (TI*)smem;  // [component][R NY]
   const long long rows = (long long)gf.NX * gf.NZ;

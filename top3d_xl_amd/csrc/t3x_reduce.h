@@ -180,11 +180,17 @@ __device__ __forceinline__ double fold_here(const double* p, int nb) {
   return s;
 }
 // FIN_RR in every block of the kernel after the residual's update; true: the
-// solve has converged
+// solve has converged, here or in an earlier iteration.  Block 0 sets the flag
+// while other blocks of its kernel start, so a kernel that folds does not test
+// it wave by wave: a block's first thread reads it for all of them, and whatever
+// it reads the block folds the same sum and leaves together.
 __device__ __forceinline__ bool rr_fold(const RrFold& f) {
-  const double t = fold_here(f.partials, f.nb), res = sqrt(t) / f.sc[SC_NORMB];
+  __shared__ int was;
+  if (threadIdx.x == 0) was = f.fl[FL_DONE];
+  const double t = fold_here(f.partials, f.nb), res = sqrt(t) / f.sc[SC_NORMB];  // (its barrier: was is there)
+  if (was) return true;
   const bool done = res < f.sc[SC_TOL];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {  // (the flag may reach blocks that start later: they would return here)
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     f.sc[SC_RR] = t;
     f.sc[SC_RES] = res;
     const int it = f.fl[FL_ITER] + 1;
