@@ -107,3 +107,149 @@ enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorUnknown = 999
 inline const char* hipGetErrorString(hipError_t) { return "model"; }
 struct ModelStream;
 using hipStream_t = ModelStream*;
+
+// ---- the runtime: streams, events, pinned memory
+namespace model {
+inline thread_local int newsLeft = -1;  // C++ allocations of this thread until one fails (-1: none does)
+struct Spare {                          // the model's own allocations do not fail
+  int keep = newsLeft;
+  Spare() { newsLeft = -1; }
+  ~Spare() { newsLeft = keep; }
+};
+inline std::atomic<int> pinnedNow{0}, pinnedCalls{0}, eventsNow{0};
+inline std::atomic<size_t> pinnedLimit{~size_t(0)};  // bytes of the largest pinned allocation that succeeds
+inline std::atomic<int> launchesUntilError{-1};
+}  // namespace model
+
+struct ModelStream {
+  std::mutex m;
+  std::condition_variable cv;
+  std::deque<std::function<void()>> todo;
+  unsigned long long asked = 0, ran = 0;
+  bool end = false;
+  std::thread t{[this] {
+    unsigned seed = 1;
+    for (;;) {
+      std::function<void()> f;
+      {
+        std::unique_lock<std::mutex> l(m);
+        cv.wait(l, [&] { return end || !todo.empty(); });
+        if (todo.empty()) return;
+        f = std::move(todo.front());
+        todo.pop_front();
+      }
+      if ((seed = seed * 1664525u + 1013904223u) >> 30 == 0) std::this_thread::sleep_for(std::chrono::microseconds(200));
+      f();
+      {
+        std::lock_guard<std::mutex> l(m);
+        ++ran;
+      }
+      cv.notify_all();
+    }
+  }};
+  ~ModelStream() {
+    {
+      std::lock_guard<std::mutex> l(m);
+      end = true;
+    }
+    cv.notify_all();
+    t.join();
+  }
+  unsigned long long push(std::function<void()> f) {
+    std::lock_guard<std::mutex> l(m);
+    todo.push_back(std::move(f));
+    cv.notify_all();
+    return ++asked;
+  }
+  void wait(unsigned long long upTo) {
+    std::unique_lock<std::mutex> l(m);
+    cv.wait(l, [&] { return ran >= upTo; });
+  }
+};
+struct ModelEvent {
+  ModelStream* s = nullptr;
+  unsigned long long at = 0;
+};
+using hipEvent_t = ModelEvent*;
+enum { hipEventDisableTiming = 2, hipHostMallocCoherent = 0x40000000 };
+enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t {
+  hipMemoryType type;
+};
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+  a->type = hipMemoryTypeUnregistered;
+  return hipSuccess;
+}
+inline hipError_t hipGetLastError() { return hipSuccess; }
+inline thread_local int modelDevice = 0;
+inline hipError_t hipGetDevice(int* d) {
+  *d = modelDevice;
+  return hipSuccess;
+}
+inline hipError_t hipSetDevice(int d) {
+  modelDevice = d;
+  return hipSuccess;
+}
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++model::pinnedCalls;
+  if (n > model::pinnedLimit) return hipErrorOutOfMemory;
+  *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+  ++model::pinnedNow;
+  return hipSuccess;
+}
+inline hipError_t hipHostFree(void* p) {
+  std::memset(p, 0xCD, 4096);  // whoever still reads or fills it shows
+  std::free(p);
+  --model::pinnedNow;
+  return hipSuccess;
+}
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  model::Spare s;
+  *e = new ModelEvent;
+  ++model::eventsNow;
+  return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) {
+  delete e;
+  --model::eventsNow;
+  return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
+  model::Spare s;
+  e->s = st;
+  e->at = st->push([] {});
+  return hipSuccess;
+}
+inline hipError_t hipEventSynchronize(hipEvent_t e) {
+  if (e->s) e->s->wait(e->at);
+  return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t st) {
+  model::Spare s;
+  st->wait(st->push([] {}));
+  return hipSuccess;
+}
+inline hipError_t hipMemcpyAsync(void* d, const void* h, size_t n, hipMemcpyKind, hipStream_t st) {
+  model::Spare s;
+  st->push([=] { std::memcpy(d, h, n); });
+  return hipSuccess;
+}
+// kernels of the form (const char*, char*, unsigned)
+inline hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 threads, void** args, size_t, hipStream_t st) {
+  if (model::launchesUntilError >= 0 && model::launchesUntilError-- == 0) return hipErrorUnknown;
+  model::Spare s;
+  auto* k = (void (*)(const char*, char*, unsigned))f;
+  const char* a = *(const char**)args[0];
+  char* b = *(char**)args[1];
+  const unsigned n = *(unsigned*)args[2];
+  st->push([=] {
+    for (unsigned g = 0; g < grid.x; ++g)
+      for (unsigned t = 0; t < threads.x; ++t) {
+        blockIdx = dim3(g, 0, 0);
+        threadIdx = dim3(t, 0, 0);
+        k(a, b, n);
+      }
+  });
+  return hipSuccess;
+}

@@ -1,0 +1,60 @@
+// HostStage (t3x_stage.hip) on the CPU: exit status 0 if every check holds.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <new>
+
+#include "../top3d_xl_amd/csrc/t3x_stage.hip"
+
+void* operator new(size_t n) {
+  if (model::newsLeft >= 0 && model::newsLeft-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+using namespace t3x;
+
+static int bad = 0;
+static void check(bool ok, const char* what, size_t n) {
+  if (!ok) std::printf("wrong: %s, %zu\n", what, n), ++bad;
+}
+static std::vector<char> pattern(size_t n, unsigned seed) {
+  std::vector<char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (char)((i * 2654435761u + seed) >> 13);
+  return v;
+}
+// n bytes up and back, the source overwritten as soon as the call returns
+static bool round_trip(HostStage& S, hipStream_t s, size_t n, unsigned seed) {
+  std::vector<char> src = pattern(n, seed), dev(n + 16), out(n, 1);
+  char* d = dev.data() + (16 - (uintptr_t)dev.data() % 16) % 16;
+  if (S.to_device(d, src.data(), n, s) != hipSuccess) return false;
+  std::fill(src.begin(), src.end(), 7);
+  if (S.to_host(out.data(), d, n, s) != hipSuccess) return false;
+  return out == pattern(n, seed);
+}
+
+// memory for a thread's start runs out: the threads that run take all chunks
+static void no_more_threads() {
+  ModelStream s;
+  for (int left : {0, 1, 2, 5}) {
+    HostStage S;
+    for (size_t n : {(size_t)9 << 20, ((size_t)65 << 20) + 40}) {
+      std::vector<char> src = pattern(n, 3), dev(n), out(n);
+      char* d = dev.data();  // (malloc'ed: 16-byte aligned)
+      model::newsLeft = left;
+      const hipError_t a = S.to_device(d, src.data(), n, &s);
+      model::newsLeft = left;
+      const hipError_t b = S.to_host(out.data(), d, n, &s);
+      model::newsLeft = -1;
+      check(a == hipSuccess && b == hipSuccess && out == src, "a copy without its threads", n);
+    }
+  }
+}
+
+int main() {
+  no_more_threads();
+  check(model::pinnedNow == 0 && model::eventsNow == 0, "all given back", model::pinnedNow);
+  return bad != 0;
+}

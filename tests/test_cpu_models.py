@@ -19,3 +19,8 @@ def test_residual_fold_is_the_same_for_a_whole_block(tmp_path):
     whenever its waves start beside the block that ends the solve, and nothing
     counted once the solve has ended."""
     _run(tmp_path, "rr_fold_model.cpp")
+
+
+def test_host_transfers(tmp_path):
+    """Host arrays through the ring of pinned chunks (t3x_stage.hip)."""
+    _run(tmp_path, "stage_model.cpp")

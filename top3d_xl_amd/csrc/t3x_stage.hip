@@ -5,7 +5,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace t3x {
@@ -142,7 +142,7 @@ hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStre
   if (e == hipSuccess) {
     try {
       for (int t = 1; t < nt; ++t) th[t] = std::thread(run, t);
-    } catch (const std::system_error&) {  // no more threads: those that run take all chunks
+    } catch (const std::exception&) {  // no thread or no memory for one: those that run take all chunks
     }
   }
   run(0);
