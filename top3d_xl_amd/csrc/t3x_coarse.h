@@ -27,8 +27,6 @@ struct CoarseSolver {
   int np = 0;    // padded order (multiple of SB)
   int nblk = 0;  // np / SB
   ChainState* chain = nullptr;  // device words of the one-launch recurrences (null: a launch per block)
-  int sets = 1;  // of work-groups that take the blocks of a recurrence in turn (k_solve_chain)
-  bool sets_apply() const { return SB > kFusedMaxSB && SB <= kChainMaxSB / 2; }
   bool one_launch() const { return chain && SB <= kChainMaxSB; }
   // parts per million of the current device's work-group slots (its
   // occupancy for the recurrences' registers and LDS) that one launch of the

@@ -841,10 +841,11 @@ __global__ void k_solve_scatter(int n, const long long* __restrict__ map, const 
 // sets one set's rows arrive while the other one's block is formed: 62.9 ->
 // 48.3 us forward, 58.2 -> 49.5 us backward at 128x256x128 (18 blocks), 53 ->
 // 46 us at 96x192x96.  480 groups of one row per wave: 49 us and twice the
-// share of the device; 3 or 4 sets 53 to 72 us.
+// share of the device; 3 or 4 sets 53 to 72 us.  Above SB 1024 two rows of a
+// wave do not fit its registers: one set.
 // All groups must be resident together: 4 waves and SB doubles of LDS each, far
-// below the device's capacity; two sets keep to 128 registers for that (a
-// share of 23.4% of the device at SB 960, one set 18.8%).  Each wait is bounded:
+// below the device's capacity; two sets keep to 128 registers for that (see
+// chain_share; 23.4% of the device at SB 960).  Each wait is bounded:
 // after kChainSpin polls the launch sets fail, every group stops waiting (the
 // solve is then garbage) and the caller reports the error; fail stays set.
 // Measured alternatives (same operators): one launch for everything with a
@@ -992,15 +993,19 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(SETS == 2 ? 
 // back's (DT y) when the block before arrives.  Against k_solve_f0, two
 // k_solve_chain and k_solve_b0 that is three launches and two passes over the
 // vectors less, with the same sums in the same order.  Words and polls as in
-// k_solve_chain.  Rows: one per wave; NW waves per group, few, so that a
-// block's loads spread over many CUs.
-// Bound: the hand-over, 1.4 us a step.  50x100x50 (SB 256, 11 blocks): 36.3 us,
-// 39 with words of half a value, against 51 us and three launches; 2 waves per
-// group against 4: 42.4 / 42.9 us (words of half a value), at SB 384 70 / 76 us.
-// Two sets of groups in turn: 34.9 us and twice the share of the device.  Groups
-// with waves that only poll, beside the row waves, were slower (62 us; at SB
-// 960 163 against 92 us a direction: polls that do not wait for the operator
-// rows compete with them for memory).
+// k_solve_chain.  Rows: one per wave, few per group, so that a block's loads
+// spread over many CUs.
+// Four waves a group and four groups a CU, as the other forms (chain_share): 128
+// registers, for which the wave's row is in scalars and a DT row is summed before
+// the next own terms are asked for (154 registers otherwise, three groups).
+// Bound: the hand-over, 1.4 us a step.  50x100x50 (SB 256, 11 blocks): 38 us,
+// against 54 us in four launches; at SB 384 (12 blocks) 68 against 77, at SB 512
+// 108 to 113 against 122 and three launches.  Groups of two waves 39, 65 and 108
+// us: two of them need not leave a slot on each SIMD for a group of four.  Two sets
+// of groups in turn: 4% less and twice the share of the device.  Groups with waves
+// that only poll, beside the row waves, were slower (62 us; at SB 960 163 against
+// 92 us a direction: polls that do not wait for the operator rows compete with
+// them for memory).
 struct FusedArgs {
   int n, SB, nblk;
   const long long* map;
@@ -1010,15 +1015,16 @@ struct FusedArgs {
   ChainState* st;
 };
 // NCH: 64-column chunks of a row (SB <= 64 NCH), PT = NCH / NW entries polled per thread
-template <typename TV, int NW, int NCH>
-__global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* __restrict__ rdense,
-                                                         TV* __restrict__ xdense, const int* fl) {
+template <typename TV, int NCH>
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(4)))
+void k_solve_fused(FusedArgs A, const TV* __restrict__ rdense, TV* __restrict__ xdense, const int* fl) {
   if (fl && fl[FL_DONE]) return;
-  constexpr int PT = NCH / NW, NT = 64 * NW;
+  constexpr int NW = CT / 64, PT = NCH / NW, NT = CT;
   extern __shared__ double chainNbr[];  // two neighbour blocks, in turn
   const int SB = A.SB, nblk = A.nblk;
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * NW + (threadIdx.x >> 6);  // SB is a multiple of NW: row < SB
+  // SB is a multiple of NW: row < SB
+  const int row = blockIdx.x * NW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned turn = A.st->turn[blockIdx.x];
   const size_t wn = (size_t)(turn & 1) * nblk * SB, wo = (size_t)(~turn & 1) * nblk * SB;
   int step = 0;
@@ -1118,14 +1124,12 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
       chain_put(A.W + wn + b * SB + row, y);
       chain_clear(A.W + wo + b * SB + row);
     }
-    if (b + 1 < nblk) {
-      load(op_row(A.Gm, b + 1), SB, rg);
-      load_own(b + 1);
-    }
+    if (b + 1 < nblk) load(op_row(A.Gm, b + 1), SB, rg);
     if (b > 0) {
       const double t = dot(rt, sY + row, SB - row);
       if (lane == 0) A.vb[(size_t)(b - 1) * SB + row] = t;
     }
+    if (b + 1 < nblk) load_own(b + 1);
     load(op_row(A.DT, b) + row, SB - row, rt);
   }
   {  // x of the last block is its own term
@@ -1146,45 +1150,43 @@ __global__ __launch_bounds__(64 * NW) void k_solve_fused(FusedArgs A, const TV* 
 
 // ---- host side -----------------------------------------------------------
 template <typename TV>
-struct FusedForm {
-  int waves;  // per group
-  void (*fn)(FusedArgs, const TV*, TV*, const int*);
-};
-template <typename TV>
-static FusedForm<TV> fused_form(int SB) {
-  if (SB <= 256) return {2, k_solve_fused<TV, 2, 4>};
-  return {2, k_solve_fused<TV, 2, 8>};
+static auto fused_form(int SB) {
+  return SB <= 256 ? k_solve_fused<TV, 4> : k_solve_fused<TV, 8>;
 }
 static size_t fused_lds(int SB) { return 2 * (size_t)SB * sizeof(double); }
 
 template <typename TV, bool FWD>
-static auto chain_form(int SB, int sets) {
-  if (SB > 4 * CT) return k_solve_chain<TV, kChainMaxSB / CT, 1, FWD>;
-  return sets == 2 ? k_solve_chain<TV, 4, 2, FWD> : k_solve_chain<TV, 4, 1, FWD>;
+static auto chain_form(int SB) {
+  return SB > 4 * CT ? k_solve_chain<TV, kChainMaxSB / CT, 1, FWD> : k_solve_chain<TV, 4, 2, FWD>;
 }
 
+// Every form's groups have four waves, one per SIMD, and up to SB 1024 at most
+// 128 registers: they count as a quarter of a CU each, whatever else is resident
+// on it, also where a form alone would fit six times (77 registers up to SB
+// 256).  So while the shares add up to the device, some CU has room for every
+// such group that is not resident yet.  (Counted by their own occupancy, groups of
+// 96 and of 128 registers could keep each other out, both launches incomplete: two
+// of the one and two of the other leave 64 registers on a SIMD.)
 long long CoarseSolver::chain_share() const {
   constexpr long long kNever = 2000000;
+  constexpr int kGroupsPerCU = 4;
   if (SB > kChainMaxSB) return kNever;
   int dev = 0, cus = 0, perCU = 0, perCU2 = 0;
   if (hipGetDevice(&dev) != hipSuccess) return kNever;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return kNever;
-  int G = (SB + 3) / 4;
+  const int G = (SB + 3) / 4;
   if (SB <= kFusedMaxSB) {
-    const FusedForm<double> fd = fused_form<double>(SB);
-    const FusedForm<float> ff = fused_form<float>(SB);
-    G = SB / fd.waves;
     const size_t lds = fused_lds(SB);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fd.fn, 64 * fd.waves, lds) != hipSuccess) return kNever;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, ff.fn, 64 * ff.waves, lds) != hipSuccess) return kNever;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fused_form<double>(SB), CT, lds) != hipSuccess) return kNever;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, fused_form<float>(SB), CT, lds) != hipSuccess) return kNever;
   } else {
     const size_t lds = (size_t)SB * sizeof(double);
-    auto fwd = chain_form<double, true>(SB, sets);
-    auto bwd = chain_form<float, false>(SB, sets);
+    auto fwd = chain_form<double, true>(SB);
+    auto bwd = chain_form<float, false>(SB);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fwd, CT, lds) != hipSuccess) return kNever;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, bwd, CT, lds) != hipSuccess) return kNever;
   }
-  const long long slots = (long long)std::min(perCU, perCU2) * cus;
+  const long long slots = (long long)std::min({perCU, perCU2, kGroupsPerCU}) * cus;
   if (slots <= 0) return kNever;
   return (1000000LL * G + slots - 1) / slots;
 }
@@ -1234,16 +1236,15 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
   const int wpb = CT / 64;
   const int n = C.n, np = C.np, SB = C.SB, nblk = C.nblk;
   if (C.one_launch() && SB <= kFusedMaxSB) {
-    const FusedForm<TV> f = fused_form<TV>(SB);
     const FusedArgs A{n, SB, nblk, map, Dinv, DT, Gm, H, vb, (unsigned long long*)(va + np),
                       (unsigned long long*)(vb + np), C.chain};
-    hipLaunchKernelGGL(f.fn, dim3(SB / f.waves), dim3(64 * f.waves), fused_lds(SB), s, A, rdense, xdense, fl);
+    hipLaunchKernelGGL(fused_form<TV>(SB), dim3(SB / wpb), dim3(CT), fused_lds(SB), s, A, rdense, xdense, fl);
     return;
   }
   const dim3 ownGrid(np / kOwnRows);
   if (C.one_launch()) {  // va, vb: np plain doubles, then 2 np words each
-    auto fwd = chain_form<TV, true>(SB, C.sets);
-    auto bwd = chain_form<TV, false>(SB, C.sets);
+    auto fwd = chain_form<TV, true>(SB);
+    auto bwd = chain_form<TV, false>(SB);
     const dim3 grid((SB + wpb - 1) / wpb);
     hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
                        fl);

@@ -159,7 +159,6 @@ struct GroupTimer {
 // parts per million of the device's work-group slots held by this process's
 // handles for the one-launch coarsest recurrences
 static std::atomic<long long> gChainShare{0};
-constexpr long long kTwoSetShare = 250000;  // parts per million of the device, with the handles there are
 
 struct t3x_problem {
   // Caller-provided resources (the serving engine's pooled slot): device
@@ -792,14 +791,8 @@ int setup(t3x_problem& P, const uint8_t* vox, int nFix, const int* fixNodes, con
     // need at most all of the device's work-group slots, so recurrences
     // running at the same time can always all be resident
     if (P.oneLaunchCoarse) {
-      long long need = 0, held = gChainShare.load();
-      // two sets of work-groups (15 to 23% less time per recurrence; a share of
-      // 23% against 19% at SB 960) for a handle within the first quarter of the
-      // device: room is left for as many handles as with one set each
-      for (P.cs.sets = P.cs.sets_apply() ? 2 : 1;; P.cs.sets = 1) {
-        need = P.cs.chain_share();
-        if (P.cs.sets == 1 || held + need <= kTwoSetShare) break;
-      }
+      const long long need = P.cs.chain_share();
+      long long held = gChainShare.load();
       while (held + need <= 1000000 && !gChainShare.compare_exchange_weak(held, held + need)) {
       }
       if (held + need <= 1000000) {
