@@ -47,8 +47,9 @@ class HostStage {
   hipError_t move(char* dev, char* host, size_t bytes, bool up, hipStream_t s);
   hipError_t issue(struct StageJob& job, size_t c);
   hipError_t part(struct StageJob& job);
-  char* ring_ = nullptr;
+  char* ring_ = nullptr;  // lent by the process's pool of rings
   size_t ringBytes_ = 0;
+  int device_ = 0;  // where it was made
   hipEvent_t ev_[kMaxSlots] = {};
   bool busy_ = false;    // the last upload may still be reading the ring; ev_[last_] ends it
   int last_ = 0;
