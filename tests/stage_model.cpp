@@ -94,8 +94,44 @@ static void rings_serve_on() {
   check(model::pinnedNow <= 4, "rings kept", model::pinnedNow);
 }
 
+// every number of threads, below, at and above each line, and the ring's slots
+// used again: with all of it, and with a ring that could not grow
+static void every_form() {
+  for (size_t limit : {(size_t)256 << 10, (size_t)1 << 20, ~(size_t)0}) {
+    model::pinnedLimit = limit;
+    const int made = model::pinnedNow;
+    ModelStream s;
+    HostStage S;
+    const size_t first = min(limit, (size_t)16 << 20);  // the ring is as large as it will be from the start
+    check(round_trip(S, &s, first, 1) && model::pinnedNow == made + 1, "a ring of this size", first);
+    check(round_trip(S, &s, 1, 1), "one byte", 1);
+    for (size_t mb : {5, 8, 32, 64})
+      for (size_t n : {(mb << 20) - 8, mb << 20, (mb << 20) + 4099}) check(round_trip(S, &s, n, (unsigned)n), "a copy", n);
+    for (size_t n : {(size_t)262144, (size_t)262152, (size_t)3000001}) check(round_trip(S, &s, n, (unsigned)n), "a copy", n);
+  }
+  model::pinnedLimit = ~(size_t)0;
+}
+// a launch that fails ends the copy with its error, and the next one is whole
+static void errors() {
+  ModelStream s;
+  HostStage S;
+  for (size_t n : {(size_t)1000, (size_t)3 << 20, (size_t)20 << 20})
+    for (int k : {0, 1, 5}) {
+      std::vector<char> src = pattern(n, 2), dev(n);
+      model::launchesUntilError = k;
+      const hipError_t a = S.to_device(dev.data(), src.data(), n, &s);
+      const hipError_t b = a == hipSuccess ? S.to_host(src.data(), dev.data(), n, &s) : hipSuccess;
+      const bool hit = model::launchesUntilError < 0;
+      model::launchesUntilError = -1;
+      check(!hit || a != hipSuccess || b != hipSuccess, "an error reported", n);
+      check(round_trip(S, &s, n, 4), "a copy after an error", n);
+    }
+}
+
 int main() {
+  every_form();  // first: no larger ring is there to be lent
   rings_serve_on();
+  errors();
   no_more_threads();
   check(model::pinnedNow <= 4 && model::eventsNow == 0, "all given back", model::pinnedNow);
   return bad != 0;
