@@ -118,7 +118,9 @@ struct Spare {                          // the model's own allocations do not fa
 };
 inline std::atomic<int> pinnedNow{0}, pinnedCalls{0}, eventsNow{0};
 inline std::atomic<size_t> pinnedLimit{~size_t(0)};  // bytes of the largest pinned allocation that succeeds
-inline std::atomic<int> launchesUntilError{-1};
+inline std::atomic<int> launchesUntilError{-1}, eventsRecorded{0};
+inline std::mutex streamsMutex;
+inline std::vector<ModelStream*> streams;
 }  // namespace model
 
 struct ModelStream {
@@ -147,7 +149,15 @@ struct ModelStream {
       cv.notify_all();
     }
   }};
+  ModelStream() {
+    std::lock_guard<std::mutex> l(model::streamsMutex);
+    model::streams.push_back(this);
+  }
   ~ModelStream() {
+    {
+      std::lock_guard<std::mutex> l(model::streamsMutex);
+      model::streams.erase(std::find(model::streams.begin(), model::streams.end(), this));
+    }
     {
       std::lock_guard<std::mutex> l(m);
       end = true;
@@ -217,6 +227,7 @@ inline hipError_t hipEventDestroy(hipEvent_t e) {
 }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
   model::Spare s;
+  ++model::eventsRecorded;
   e->s = st;
   e->at = st->push([] {});
   return hipSuccess;
@@ -228,6 +239,12 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) {
 inline hipError_t hipStreamSynchronize(hipStream_t st) {
   model::Spare s;
   st->wait(st->push([] {}));
+  return hipSuccess;
+}
+inline hipError_t hipDeviceSynchronize() {
+  model::Spare s;
+  std::lock_guard<std::mutex> l(model::streamsMutex);
+  for (ModelStream* st : model::streams) st->wait(st->push([] {}));
   return hipSuccess;
 }
 inline hipError_t hipMemcpyAsync(void* d, const void* h, size_t n, hipMemcpyKind, hipStream_t st) {

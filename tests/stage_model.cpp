@@ -128,10 +128,34 @@ static void errors() {
     }
 }
 
+// small copies follow each other through the ring, each source overwritten at
+// once, with no event of their own; larger ones between them
+static void small_copies() {
+  ModelStream s;
+  HostStage S;
+  const size_t n = 4100, many = 200;
+  std::vector<std::vector<char>> dev(many, std::vector<char>(n));
+  const int before = model::eventsRecorded;
+  int events = 0;
+  for (size_t i = 0; i < many; ++i) {
+    std::vector<char> src = pattern(n, (unsigned)i), back(n);
+    check(S.to_device(dev[i].data(), src.data(), n, &s) == hipSuccess, "a small upload", i);
+    std::fill(src.begin(), src.end(), 5);
+    if (i % 70 == 30)
+      check(S.to_host(back.data(), dev[i - 9].data(), n, &s) == hipSuccess && back == pattern(n, i - 9), "a small result", i);
+    if (i == 90) events = model::eventsRecorded;
+    if (i == 149) check(round_trip(S, &s, 3 << 20, 1), "a large copy among small ones", i);
+  }
+  check(events == before, "events behind small copies", events - before);
+  (void)hipStreamSynchronize(&s);
+  for (size_t i = 0; i < many; ++i) check(dev[i] == pattern(n, (unsigned)i), "a small upload's bytes", i);
+}
+
 int main() {
   every_form();  // first: no larger ring is there to be lent
   rings_serve_on();
   errors();
+  small_copies();
   no_more_threads();
   check(model::pinnedNow <= 4 && model::eventsNow == 0, "all given back", model::pinnedNow);
   return bad != 0;

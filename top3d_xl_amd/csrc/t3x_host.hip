@@ -322,7 +322,7 @@ struct t3x_problem {
       for (auto& pr : T.pending) { (void)hipEventDestroy(pr.first); (void)hipEventDestroy(pr.second); }
       for (auto e : T.pool) (void)hipEventDestroy(e);
     }
-    if (stream) (void)hipStreamSynchronize(stream);
+    if (stream && hipStreamSynchronize(stream) == hipSuccess) stage->drained();
     for (void* p : allocs) (void)hipFree(p);
     if (hbuf && ownHostBuf) (void)hipHostFree(hbuf);
     if (stream && ownStream) (void)hipStreamDestroy(stream);
@@ -335,7 +335,10 @@ struct t3x_problem {
   bool f16() const { return P.precision == 2; }    // ... with FP16 coarse Galerkin copies
   const uint8_t* design_mask() const { return active ? active : lv[0].emask; }
   bool standard() const { return P.vcycle == 1; }  // 'Standard' V-cycle (FP64 or, mixed, FP32)
-  void sync() { T3X_HIP(hipStreamSynchronize(stream)); }
+  void sync() {
+    T3X_HIP(hipStreamSynchronize(stream));
+    stage->drained();
+  }
   // Host-to-device upload ordered on the problem stream; the host buffer may be
   // released on return.
   void upload(void* dst, const void* src, size_t bytes) { T3X_HIP(stage->to_device(dst, src, bytes, stream)); }

@@ -26,6 +26,11 @@ class HostStage {
   // still be on the link), to_host when `dst` is written.
   hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t s);
   hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
+  // The caller has waited for the stream (as the last thing before it goes).
+  void drained() {
+    busy_ = false;
+    used_ = 0;
+  }
   ~HostStage();
   HostStage() = default;
   HostStage(const HostStage&) = delete;
@@ -46,8 +51,11 @@ class HostStage {
   static int threads_of(size_t bytes) {
     return bytes < (5u << 20) ? 1 : bytes < (8u << 20) ? 2 : bytes < (64u << 20) ? 4 : kMaxThreads;
   }
-  bool reserve(size_t bytes);
+  bool reserve(size_t bytes, hipStream_t s);
   hipError_t record(int slot, hipStream_t s);  // the slot's event, made when first used
+  hipError_t drain(hipStream_t s);
+  hipError_t put(char* dev, const char* host, size_t bytes, hipStream_t s);
+  hipError_t get(char* dev, char* host, size_t bytes, hipStream_t s);
   hipError_t move(char* dev, char* host, size_t bytes, bool up, hipStream_t s);
   hipError_t issue(struct StageJob& job, size_t c);
   hipError_t part(struct StageJob& job);
@@ -55,8 +63,11 @@ class HostStage {
   size_t ringBytes_ = 0;
   int device_ = 0;  // where it was made
   hipEvent_t ev_[kMaxSlots] = {};
-  bool busy_ = false;    // the last upload may still be reading the ring; ev_[last_] ends it
+  // What may still be reading the ring: an upload of several chunks, ended by
+  // ev_[last_], or small ones in its first used_ bytes.
+  bool busy_ = false;
   int last_ = 0;
+  size_t used_ = 0;
   bool failed_ = false;  // no pinned memory: the runtime's own path
 };
 

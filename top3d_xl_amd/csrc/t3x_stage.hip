@@ -101,7 +101,8 @@ class RingPool {
 static RingPool gRings;
 
 HostStage::~HostStage() {
-  const bool idle = !busy_ || hipEventSynchronize(ev_[last_]) == hipSuccess;
+  const bool idle = (!used_ || hipDeviceSynchronize() == hipSuccess) &&  // (drained() is the owner's way)
+                    (!busy_ || hipEventSynchronize(ev_[last_]) == hipSuccess);
   for (hipEvent_t e : ev_)
     if (e) (void)hipEventDestroy(e);
   if (!ring_) return;
@@ -110,13 +111,12 @@ HostStage::~HostStage() {
 }
 
 // a ring for a copy of this size
-bool HostStage::reserve(size_t bytes) {
+bool HostStage::reserve(size_t bytes, hipStream_t s) {
   size_t want = kMinRing;
   while (want < kMaxRing && want < bytes) want *= 2;
   if (ringBytes_ >= want) return true;
   if (failed_) return ringBytes_ > 0;
-  if (busy_ && hipEventSynchronize(ev_[last_]) != hipSuccess) return false;
-  busy_ = false;
+  if (drain(s) != hipSuccess) return false;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return false;
   char* ring = gRings.take(&want, device);
@@ -140,23 +140,52 @@ hipError_t HostStage::record(int slot, hipStream_t s) {
   return hipEventRecord(ev_[slot], s);
 }
 
+// no upload reads the ring any more
+hipError_t HostStage::drain(hipStream_t s) {
+  const hipError_t e = used_ ? hipStreamSynchronize(s) : busy_ ? hipEventSynchronize(ev_[last_]) : hipSuccess;
+  if (e == hipSuccess) drained();
+  return e;
+}
+
+// n bytes between pinned and device memory
+static hipError_t copy_pinned(char* dev, char* pin, size_t n, bool up, hipStream_t s) {
+  if ((uintptr_t)dev % 16 != 0)
+    return hipMemcpyAsync(up ? dev : pin, up ? pin : dev, n, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
+  const char* src = up ? pin : dev;
+  char* dst = up ? dev : pin;
+  unsigned len = (unsigned)n;
+  void* args[] = {&src, &dst, &len};  // (its own status: the thread's last error may be another call's)
+  return hipLaunchKernel((const void*)k_stage_copy, dim3((len + 4095) / 4096), dim3(256), args, 0, s);
+}
+
+// Copies of up to kMinRing bytes: one chunk, and no event, which would cost the
+// stream 5 us and, waited for instead of the stream, the next call 10.  An upload
+// goes behind those before it in the ring.
+hipError_t HostStage::put(char* dev, const char* host, size_t bytes, hipStream_t s) {
+  if (busy_ || used_ + bytes > ringBytes_) {
+    const hipError_t e = drain(s);
+    if (e != hipSuccess) return e;
+  }
+  char* pin = ring_ + used_;
+  std::memcpy(pin, host, bytes);
+  used_ += (bytes + 15) & ~(size_t)15;
+  return copy_pinned(dev, pin, bytes, true, s);
+}
+hipError_t HostStage::get(char* dev, char* host, size_t bytes, hipStream_t s) {
+  hipError_t e = copy_pinned(dev, ring_, bytes, false, s);  // (on the stream behind the uploads)
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return e;
+  drained();
+  std::memcpy(host, ring_, bytes);
+  return e;
+}
+
 // Chunk c between its slot and the device, and the slot's event behind it
 // where somebody waits for it.
 hipError_t HostStage::issue(StageJob& job, size_t c) {
   const int slot = (int)(c % job.slots);
-  char *dev = job.dev + c * job.chunk, *pin = ring_ + slot * job.chunk;
   const size_t n = std::min(job.chunk, job.bytes - c * job.chunk);
-  hipError_t e = hipSuccess;
-  if ((uintptr_t)dev % 16 == 0) {
-    const char* src = job.up ? pin : dev;
-    char* dst = job.up ? dev : pin;
-    unsigned len = (unsigned)n;
-    void* args[] = {&src, &dst, &len};  // (its own status: the thread's last error may be another call's)
-    e = hipLaunchKernel((const void*)k_stage_copy, dim3((len + 4095) / 4096), dim3(256), args, 0, job.s);
-  } else {
-    e = hipMemcpyAsync(job.up ? dev : pin, job.up ? pin : dev, n, job.up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost,
-                       job.s);
-  }
+  hipError_t e = copy_pinned(job.dev + c * job.chunk, ring_ + slot * job.chunk, n, job.up, job.s);
   if (e == hipSuccess && (!job.up || c + job.slots < job.chunks)) e = record(slot, job.s);
   job.issued[slot].store(c / job.slots + 1, std::memory_order_release);
   return e;
@@ -197,7 +226,7 @@ hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStre
                up, s};
   static_assert(sizeof(job.issued) / sizeof(job.issued[0]) == kMaxSlots, "a count per slot");
   hipError_t e = hipSuccess;
-  if (up && busy_) e = hipEventSynchronize(ev_[last_]);  // (a download follows it on the stream)
+  if (up) e = drain(s);  // (a download follows the uploads on the stream)
   if (e != hipSuccess) return e;
   if (!up)
     for (size_t c = 0; e == hipSuccess && c < std::min<size_t>(job.chunks, job.slots); ++c) e = issue(job, c);
@@ -220,16 +249,17 @@ hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStre
     if (t.joinable()) t.join();
   e = (hipError_t)job.err.load();
   if (e != hipSuccess) {
-    (void)hipStreamSynchronize(s);  // no slot is left to a chunk in flight
-    busy_ = false;
+    used_ = ringBytes_;  // no slot is left to a chunk in flight
+    if (hipStreamSynchronize(s) == hipSuccess) drained();
     return e;
   }
   if (up) {
     last_ = (int)((job.chunks - 1) % job.slots);
     e = record(last_, s);
     busy_ = e == hipSuccess;
+    if (!busy_) used_ = ringBytes_;
   } else {
-    busy_ = false;
+    drained();
   }
   return e;
 }
@@ -247,14 +277,16 @@ static bool plain_memory(const void* p) {
 
 hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStream_t s) {
   if (bytes == 0) return hipSuccess;
-  if (plain_memory(src) && reserve(bytes)) return move((char*)dst, (char*)src, bytes, true, s);
+  if (plain_memory(src) && reserve(bytes, s))
+    return bytes <= kMinRing ? put((char*)dst, (const char*)src, bytes, s) : move((char*)dst, (char*)src, bytes, true, s);
   const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
   return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
 
 hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
   if (bytes == 0) return hipSuccess;
-  if (plain_memory(dst) && reserve(bytes)) return move((char*)src, (char*)dst, bytes, false, s);
+  if (plain_memory(dst) && reserve(bytes, s))
+    return bytes <= kMinRing ? get((char*)src, (char*)dst, bytes, s) : move((char*)src, (char*)dst, bytes, false, s);
   const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
   return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
