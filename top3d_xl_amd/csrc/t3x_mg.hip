@@ -175,9 +175,10 @@ __global__ __launch_bounds__(kBlock) void k_restrict_xz(Geo gf, Geo gc, const TM
   rc[2 * gc.NN + n] = (TO)a2;
 }
 
-// The x-z pass with the (2S - 1) fine planes side by side: a block takes 64 outputs of one coarse plane; wave dz + S - 1 forms the x sums
-// of its fine plane (3 (2S - 1) independent loads per thread), which one wave
-// per component then adds up over z in order (the sums above, term by term).
+// The x-z pass with the (2S - 1) fine planes side by side: a block takes 64
+// outputs of one coarse plane; wave dz + S - 1 forms the x sums of its fine plane
+// (3 (2S - 1) independent loads per thread), which one wave per component then
+// adds up over z in order (the sums above, term by term).
 // Bound: load latency, a coarse grid has few outputs.
 constexpr int kXzOut = 64;
 template <int S, typename TM, typename TO>
@@ -448,8 +449,10 @@ void k_prolong_add(Geo gf, Geo gc, int zc, const TX* __restrict__ xc,
   }
 }
 
-constexpr long long kOnceOut = 65536;        // coarse nodes up to which a span-2 restriction is one launch
-constexpr long long kXzWideOut = 131072;     // coarse nodes up to which the x-z pass runs its planes side by side
+constexpr long long kOnceOut = 65536;  // coarse nodes up to which a span-2 restriction is one launch
+// coarse nodes up to which the x-z pass runs its planes side by side, by the intermediate's type
+template <typename TM>
+constexpr long long kXzWideOut = sizeof(TM) == 8 ? 92160 : 131072;
 constexpr size_t kRestrictLds = 48 * 1024;  // LDS bytes of the y pass's rows at most
 
 // the LDS y pass: about one intermediate value per thread (R rows a block)
@@ -466,9 +469,11 @@ void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const 
                    const uint8_t* nmaskC, TO* rc, const int* fl, Act actF, RrFold rr = {}) {
   const int plane = gc.NY * gf.NX;
   // span 2: both passes in one launch while the launch saved is worth the values
-  // read 3.4 times over.  637 outputs 4.6 us against 7.1, 9,537 5.2 / 9.6, 31,213
-  // 6.7 / 9.9, 70,785 11.4 / 11.9, 217,800 18.0 / 16.7.  (Span 4 reads 5.4 times
-  // over: 112 outputs 16.5 us against 9.1, 70,785 109 / 39.)
+  // read 3.4 times over.  637 outputs 3.3 us against 6.3, 9,537 3.6 / 6.6, 30,625 4.3
+  // / 8.4, 47,937 5.0 / 10.3 (FP64, the same data over and over).  The line is on the
+  // safe side: 70,785 8.1 / 12.6 and 136,161 14.3 / 15.4 there, but 11.4 / 11.9 at
+  // 70,785 and 18.0 / 16.7 at 217,800 inside a solve.  (Span 4 reads 5.4 times over:
+  // 112 outputs 16.5 us against 9.1, 70,785 109 / 39.)
   if (span == 2 && gc.NN <= kOnceOut) {
     const dim3 g((gc.NY * gc.NX + kXzOut - 1) / kXzOut, gc.NZ, 3);
     hipLaunchKernelGGL((k_restrict_once<2, TI, TM, TO>), g, dim3(kXzOut * 3), 0, s, gf, gc, rf, nmaskC, rc, fl, actF);
@@ -496,9 +501,11 @@ void restrict_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, const 
       hipLaunchKernelGGL((k_restrict_y<2, TI, TM>), g1, dim3(kBlock), 0, s, gf, gc.NY, rf, tmp, fl, actF);
   }
   // the x-z pass: planes side by side while one thread per output would leave
-  // the chip idle.  FP64, span 4: 18.4 -> 5.2 us at 6,075 outputs, 19.4 -> 17.3
-  // at 70,785; FP32 at 545,025 outputs 55 -> 62 us
-  if (gc.NN <= kXzWideOut) {
+  // the chip idle.  Both passes of span 4, one thread per output / side by side:
+  // FP64 6,525 outputs 22.4 / 9.9 us, 47,937 33.6 / 27.0, 84,525 43.1 / 42.0, 99,937
+  // 47.1 / 48.4, 117,117 52.9 / 54.1; to FP32 117,117 48.6 / 42.8, 136,161 51.1 /
+  // 49.7, 180,225 69.2 / 69.4; in FP32 117,117 41.7 / 35.9, 205,437 49.8 / 53.4
+  if (gc.NN <= kXzWideOut<TM>) {
     const dim3 g2((gc.NY * gc.NX + kXzOut - 1) / kXzOut, gc.NZ), b2(kXzOut * (2 * span - 1));
     if (span == 4) hipLaunchKernelGGL((k_restrict_xz_w<4, TM, TO>), g2, b2, 0, s, gf, gc, tmp, nmaskC, rc, fl);
     else hipLaunchKernelGGL((k_restrict_xz_w<2, TM, TO>), g2, b2, 0, s, gf, gc, tmp, nmaskC, rc, fl);
@@ -527,8 +534,12 @@ void prolong_impl(hipStream_t s, const Geo& gf, const Geo& gc, int span, double 
   if (ws) mode = (fl && sc) ? 2 : 1;
   int zc = 0;
   dim3 g = prolong_grid(gf, &zc);
-  if (!mode && (long long)g.x * g.y <= 512) {  // no partials to keep: a coarse grid's planes all side by side
-    zc = 1;                                    // (span 2, 14x26x14 cells: 7.5 -> 5.9 us)
+  // No partials to keep: a coarse grid's planes all side by side.  Span 2 onto 2, 13,
+  // 33 and 42 tiles of a plane (8, 143, 561 and 798 blocks at kPZ planes each), FP64:
+  // 6.1 -> 3.5, 6.7 -> 5.8, 13.0 -> 12.5 and 13.6 -> 15.7 us; FP32 5.5 -> 3.3, 5.7 ->
+  // 4.4, 9.8 -> 9.1, 10.5 -> 12.0
+  if (!mode && (long long)g.x * g.y <= 512) {
+    zc = 1;
     g.y = gf.NZ;
   }
   double* part = mode ? ws->partials : nullptr;
