@@ -1100,8 +1100,6 @@ void k_solve_fused(FusedArgs A, const TV* __restrict__ rdense, TV* __restrict__ 
     }
     load(op_row(A.Dinv, b), SB, rd);
   };
-  long long to = 0;  // where the row's entry of x goes (read ahead: the store must not wait for it)
-  auto load_to = [&](int b) { to = A.map[min(b * SB + row, A.n - 1)]; };
   auto emit_x = [&](int b, double v) {
     const int g = b * SB + row;
     chain_put(A.X + wn + g, v);

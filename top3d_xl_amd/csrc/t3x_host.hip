@@ -510,7 +510,7 @@ long long footprint_estimate(int nely, int nelx, int nelz, long long nv, const t
   add(8 * np * 64);                                  // tile inverses
   add(8 * 2 * ((bw + 63) / 64 + 1) * 64 * 64);       // factorization panels
   add(8 * (np / SB) * SB * SB, 4);                   // Dinv, DT, G, H
-  add(8 * 3 * np, 2);                                // solve vectors (with the tagged words)
+  add(8 * 3 * np, 2);                                // solve vectors and their exchanged words
   add((long long)sizeof(ChainState));                 // one-launch recurrences' words
   add(8LL * std::max(kMaxRedBlocks * 8, kMaxPartials) + 4096 * 4);  // reductions, scalars, flags
   add(4LL * kMaxPartials);                           // K*u tile list (irregular domains)
