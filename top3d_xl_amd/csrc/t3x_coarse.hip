@@ -24,8 +24,9 @@
 //     blocks on entry by entry, or as a chain of 2*nblk+1 small launches,
 //     instead of one dependent step per 64 rows.
 //
-// Everything else synchronises at kernel boundaries: on MI355X a device-wide barrier inside a kernel (cooperative grid sync, or fences that
-// write back the per-XCD L2) costs more than a dependent launch (~3 us).
+// Everything else synchronises at kernel boundaries: on MI355X a device-wide
+// barrier inside a kernel (cooperative grid sync, or fences that write back the
+// per-XCD L2) costs more than a dependent launch (~3 us).
 //
 // All arithmetic is FP64.  Rows beyond the true size are identity rows.
 #include <hip/hip_runtime.h>
@@ -148,7 +149,8 @@ __device__ __forceinline__ void tile16_syrk(double (*sC)[TB + 1], const double (
 template <class Side>
 __device__ __forceinline__ void tile_potrf(double (*sA)[TB + 1], double (*sD)[16][17], int* status, Side side) {
   constexpr int PB = 16;
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kq = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, kq = lane >> 4;
   // the rank-16 update of panel b on 16x16 tile (I, J)
   auto update = [&](int b, int I, int J) {
     cd4 acc;
@@ -643,9 +645,9 @@ __device__ __forceinline__ void trsm_strip(BandView V, int SB, int b, int col0, 
     else if (K1 > I && I + 1 < st) load_diag(I + 1);
   }
 }
-__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void k_trsm_blocks(BandView V, int SB, const double* __restrict__ tinv,
-                                                    double* __restrict__ Dinv, double* __restrict__ DT,
-                                                    double* __restrict__ Gm) {
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_trsm_blocks(BandView V, int SB, const double* __restrict__ tinv, double* __restrict__ Dinv,
+                   double* __restrict__ DT, double* __restrict__ Gm) {
   // two tiles of LDS (66.6 KB: two work-groups per CU); the right-hand side
   // minus the accumulated products is formed in sX once the products are done
   __shared__ double sL[TB][TB + 1];
@@ -658,15 +660,16 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const int wg = g ? blockIdx.x : blockIdx.x - nG;
   const int b = wg / st, p = wg % st + (g ? st : 0);
   if (p < st) trsm_strip<true>(V, SB, b, p * TB, tinv, Dinv + (size_t)b * SB * SB, DT, sL, sX);
-  else if (b > 0) trsm_strip<false>(V, SB, b, (p - st) * TB, tinv, Gm + (size_t)b * SB * SB, DT, sL, sX);  // G_0 is unused
+  else if (b > 0)  // G_0 is unused
+    trsm_strip<false>(V, SB, b, (p - st) * TB, tinv, Gm + (size_t)b * SB * SB, DT, sL, sX);
 }
 
 // H_b = Dinv_b^T L_{b+1,b}^T, i.e. H_b(i,j) = sum_k DT_b(i,k) L((b+1)SB + j, b SB + k).
 // One work-group per (b, output tile I, J); the next step's tiles are loaded
 // beside a step's product (0.75 -> 0.48 ms at 256x512x256, 25 -> 16.5 us at
 // 50x100x50).
-__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void k_h_blocks(BandView V, int SB, int nblk, const double* __restrict__ DT,
-                                                 double* __restrict__ H) {
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_h_blocks(BandView V, int SB, int nblk, const double* __restrict__ DT, double* __restrict__ H) {
   __shared__ double sA[TB][TB + 1];
   __shared__ double sB[TB][TB + 1];
   const int st = SB / TB;
@@ -867,17 +870,19 @@ __device__ __forceinline__ void chain_clear(unsigned long long* w) {
 __device__ __forceinline__ unsigned long long chain_get(const unsigned long long* w) {
   return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ double chain_value(unsigned long long w) { return __longlong_as_double((long long)(w ^ kUnset)); }
+__device__ __forceinline__ double chain_value(unsigned long long w) {
+  return __longlong_as_double((long long)(w ^ kUnset));
+}
 
 // FWD: y_b = a_b - G_b y_{b-1} (a = Dinv_b v_b from k_solve_f0, overwritten
 // by y for k_solve_b0); backward: x_b = a_b - H_b x_{b+1} (a = Dinv_b^T y_b
 // from k_solve_b0), scattered to xdense as formed.  PT: block entries per
 // thread (SB <= PT * CT).
 template <typename TV, int PT, int SETS, bool FWD>
-__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(SETS == 2 ? 4 : 1))) void k_solve_chain(int n, int SB, int nblk, const long long* __restrict__ map,
-                                                    TV* __restrict__ xdense, const double* __restrict__ M,
-                                                    double* __restrict__ a, unsigned long long* W, ChainState* st,
-                                                    const int* fl) {
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(SETS == 2 ? 4 : 1)))
+void k_solve_chain(int n, int SB, int nblk, const long long* __restrict__ map, TV* __restrict__ xdense,
+                   const double* __restrict__ M, double* __restrict__ a, unsigned long long* W, ChainState* st,
+                   const int* fl) {
   if (fl && fl[FL_DONE]) return;
   constexpr int NCH = PT * CT / 64;  // 64-column chunks of a row
   constexpr int RPW = SETS;          // rows per wave: the grid is as large in either form
@@ -1090,7 +1095,8 @@ void k_solve_fused(FusedArgs A, const TV* __restrict__ rdense, TV* __restrict__ 
     return wave_sum((s0 + s1) + (s2 + s3));
   };
   auto op_row = [&](const double* M, int b) { return M + ((size_t)b * SB + row) * SB; };
-  double rg[NCH], rt[NCH], rd[NCH], rv[NCH];  // rows of G or H, of DT from the diagonal on, of Dinv; the right-hand side
+  // rows of G or H, of DT from the diagonal on, of Dinv; the right-hand side
+  double rg[NCH], rt[NCH], rd[NCH], rv[NCH];
   auto load_own = [&](int b) {
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -1175,8 +1181,10 @@ long long CoarseSolver::chain_share() const {
   const int G = (SB + 3) / 4;
   if (SB <= kFusedMaxSB) {
     const size_t lds = fused_lds(SB);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fused_form<double>(SB), CT, lds) != hipSuccess) return kNever;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, fused_form<float>(SB), CT, lds) != hipSuccess) return kNever;
+    auto f64 = fused_form<double>(SB);
+    auto f32 = fused_form<float>(SB);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, f64, CT, lds) != hipSuccess) return kNever;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU2, f32, CT, lds) != hipSuccess) return kNever;
   } else {
     const size_t lds = (size_t)SB * sizeof(double);
     auto fwd = chain_form<double, true>(SB);
@@ -1244,8 +1252,7 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
     auto fwd = chain_form<TV, true>(SB);
     auto bwd = chain_form<TV, false>(SB);
     const dim3 grid((SB + wpb - 1) / wpb);
-    hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
-                       fl);
+    hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va, fl);
     hipLaunchKernelGGL(fwd, grid, dim3(CT), SB * sizeof(double), s, n, SB, nblk, map, xdense, Gm, va,
                        (unsigned long long*)(va + np), C.chain, fl);
     hipLaunchKernelGGL(k_solve_b0, dim3((np + wpb - 1) / wpb), dim3(CT), 0, s, np, SB, DT, va, vb, fl);
@@ -1253,8 +1260,7 @@ static void solve_impl(const CoarseSolver& C, hipStream_t s, const long long* ma
                        (unsigned long long*)(vb + np), C.chain, fl);
     return;
   }
-  hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va,
-                     fl);
+  hipLaunchKernelGGL(k_solve_f0<TV>, ownGrid, dim3(CT), 0, s, n, np, SB, map, rdense, Dinv, va, fl);
   for (int b = 1; b < nblk; ++b)
     hipLaunchKernelGGL(k_solve_step, dim3((SB + wpb - 1) / wpb), dim3(CT), 0, s, SB, b, -1, Gm, va, fl);
   hipLaunchKernelGGL(k_solve_b0, dim3((np + wpb - 1) / wpb), dim3(CT), 0, s, np, SB, DT, va, vb, fl);

@@ -1069,11 +1069,12 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
     if (mx && P.standard())  // 617-622, with the first fine Jacobi step of 628-629 fused
       launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, P.lv[0].diagf, P.x32, P.P.omega, P.fineAct());
     else
-      launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct(), rrBlocks);  // 617-622
+      launch_pcg_update(s, y, P.r, P.p, P.q, n3, P.ws, sc, fl, nullptr, nullptr, 0.0, P.fineAct(),
+                        rrBlocks);  // 617-622
     if (mx) {
       if (P.standard()) vcycle_standard(P, P.r, P.z32, sc, fl, true, true);                // 628-629
       else vcycle_mixed(P, P.r, P.z32, sc, fl, true);
-      launch_pcg_pupdate(s, y, P.p, P.z32, n3, P.ws, sc, fl, P.fineAct());                        // 616, 630
+      launch_pcg_pupdate(s, y, P.p, P.z32, n3, P.ws, sc, fl, P.fineAct());                    // 616, 630
     } else {
       if (P.standard()) vcycle_standard64(P, P.r, P.z, sc, fl, true);                         // 628-629
       else vcycle(P, P.r, P.z, sc, fl, true);

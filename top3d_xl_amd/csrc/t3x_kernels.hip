@@ -314,7 +314,8 @@ __global__ __launch_bounds__(kBcThreads) void k_galerkin_l2_bc(Geo gf, Geo gc, i
 #pragma unroll
   for (int b = 0; b < 8; ++b) ke[b] = Ke[row * 24 + 3 * b + cp];
   if (tid < s3) {
-    const long long fe = nidx(gf, span * cy + tid % span, span * cx + (tid / span) % span, span * cz + tid / (span * span));
+    const long long fe =
+        nidx(gf, span * cy + tid % span, span * cx + (tid / span) % span, span * cz + tid / (span * span));
     shE[tid] = E[fe];
     shM[tid] = emaskF[fe];
   }
@@ -396,7 +397,8 @@ void launch_galerkin_l2_bc(hipStream_t s, const Geo& gf, const Geo& gc, int span
                            const double* Ke, const double* E, const uint8_t* emaskF, const uint8_t* fix,
                            double* Ks) {
   if (nBc <= 0) return;
-  hipLaunchKernelGGL(k_galerkin_l2_bc, dim3(nBc), dim3(kBcThreads), 0, s, gf, gc, span, bcCells, Ke, E, emaskF, fix, Ks);
+  hipLaunchKernelGGL(k_galerkin_l2_bc, dim3(nBc), dim3(kBcThreads), 0, s, gf, gc, span, bcCells, Ke, E, emaskF, fix,
+                     Ks);
 }
 
 // Level >= 3 (span 2): Ks_c = sum over 8 children of Q^T Ks_child Q (980-995).
@@ -626,10 +628,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(double* __restrict__ r, c
 }
 // the same with p.q still to be folded
 __global__ __launch_bounds__(kBlock) void k_pcg_update_late(double* __restrict__ r, const double* __restrict__ q,
-                                                       long long n, RedWs ws, double* sc, int* fl,
-                                                       const float* __restrict__ dj, float* __restrict__ xj,
-                                                       double omega, Act act, double* part,
-                                                            int nbPQ) {
+                                                            long long n, RedWs ws, double* sc, int* fl,
+                                                            const float* __restrict__ dj, float* __restrict__ xj,
+                                                            double omega, Act act, double* part, int nbPQ) {
   if (fl[FL_DONE]) return;
   // y += lambda p (616) is deferred to k_pcg_pupdate, which reads p anyway
   const long long m = act_items(act, n);

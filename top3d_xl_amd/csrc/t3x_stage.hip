@@ -222,8 +222,8 @@ hipError_t HostStage::part(StageJob& job) {
 
 hipError_t HostStage::move(char* dev, char* host, size_t bytes, bool up, hipStream_t s) {
   const size_t chunk = std::min(chunk_of(bytes), ringBytes_);  // (a ring that could not grow)
-  StageJob job{dev, host, bytes, chunk, (bytes + chunk - 1) / chunk, (int)std::min<size_t>(ringBytes_ / chunk, kMaxSlots),
-               up, s};
+  const int slots = (int)std::min<size_t>(ringBytes_ / chunk, kMaxSlots);
+  StageJob job{dev, host, bytes, chunk, (bytes + chunk - 1) / chunk, slots, up, s};
   static_assert(sizeof(job.issued) / sizeof(job.issued[0]) == kMaxSlots, "a count per slot");
   hipError_t e = hipSuccess;
   if (up) e = drain(s);  // (a download follows the uploads on the stream)
@@ -278,7 +278,8 @@ static bool plain_memory(const void* p) {
 hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStream_t s) {
   if (bytes == 0) return hipSuccess;
   if (plain_memory(src) && reserve(bytes, s))
-    return bytes <= kMinRing ? put((char*)dst, (const char*)src, bytes, s) : move((char*)dst, (char*)src, bytes, true, s);
+    return bytes <= kMinRing ? put((char*)dst, (const char*)src, bytes, s)
+                             : move((char*)dst, (char*)src, bytes, true, s);
   const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
   return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
@@ -286,7 +287,8 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStr
 hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
   if (bytes == 0) return hipSuccess;
   if (plain_memory(dst) && reserve(bytes, s))
-    return bytes <= kMinRing ? get((char*)src, (char*)dst, bytes, s) : move((char*)src, (char*)dst, bytes, false, s);
+    return bytes <= kMinRing ? get((char*)src, (char*)dst, bytes, s)
+                             : move((char*)src, (char*)dst, bytes, false, s);
   const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
   return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }

@@ -97,7 +97,8 @@ def load_library():
     L.t3x_assemble.argtypes = [vp]
     L.t3x_apply_K.argtypes = [vp, _dp, _dp]
     L.t3x_vcycle.argtypes = [vp, _dp, _dp]
-    L.t3x_pcg.argtypes = L.t3x_pcg_zero.argtypes = [vp, _dp, _dp, C.c_double, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]
+    L.t3x_pcg.argtypes = [vp, _dp, _dp, C.c_double, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]
+    L.t3x_pcg_zero.argtypes = L.t3x_pcg.argtypes
     L.t3x_compliance.argtypes = [vp, _dp, _dp]
     L.t3x_get_nodal.argtypes = [vp, C.c_int, C.c_int, _dp]
     L.t3x_filter_setup.argtypes = [vp, C.c_int, C.c_double]
@@ -126,13 +127,13 @@ def load_library():
     return L
 
 
-EXPORTED = ["t3x_default_params", "t3x_create", "t3x_create_multi", "t3x_num_load_cases", "t3x_destroy", "t3x_last_error", "t3x_info", "t3x_run",
-            "t3x_opt_begin", "t3x_opt_step", "t3x_opt_result", "t3x_kernel_time", "t3x_kernel_time_reset",
-            "t3x_set_modulus", "t3x_assemble", "t3x_apply_K", "t3x_vcycle", "t3x_pcg", "t3x_pcg_zero", "t3x_compliance", "t3x_get_nodal",
-            "t3x_filter_setup", "t3x_filter", "t3x_oc", "t3x_oc_to", "t3x_mma", "t3x_footprint", "t3x_memory", "t3x_stream_copy", "t3x_set_passive",
-            "t3x_set_passive_layers", "t3x_get_passive",
-            "t3x_server_create", "t3x_server_submit", "t3x_server_poll", "t3x_server_release",
-            "t3x_server_stats", "t3x_server_destroy", "t3x_oc_noalloc"]
+EXPORTED = ["t3x_default_params", "t3x_create", "t3x_create_multi", "t3x_num_load_cases", "t3x_destroy",
+            "t3x_last_error", "t3x_info", "t3x_run", "t3x_opt_begin", "t3x_opt_step", "t3x_opt_result",
+            "t3x_kernel_time", "t3x_kernel_time_reset", "t3x_set_modulus", "t3x_assemble", "t3x_apply_K", "t3x_vcycle",
+            "t3x_pcg", "t3x_pcg_zero", "t3x_compliance", "t3x_get_nodal", "t3x_filter_setup", "t3x_filter", "t3x_oc",
+            "t3x_oc_to", "t3x_mma", "t3x_footprint", "t3x_memory", "t3x_stream_copy", "t3x_set_passive",
+            "t3x_set_passive_layers", "t3x_get_passive", "t3x_server_create", "t3x_server_submit", "t3x_server_poll",
+            "t3x_server_release", "t3x_server_stats", "t3x_server_destroy", "t3x_oc_noalloc"]
 
 
 def default_params(**kw) -> Params:
