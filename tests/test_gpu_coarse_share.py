@@ -2,10 +2,14 @@
 work-groups of four rows count as a quarter of a CU each (t3x_coarse.hip,
 chain_share), so SB / 4 groups of 4 x CUs a handle; the next handle gets a launch
 per block, with the same bits."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+
+MULTIPROCESSOR_COUNT = 63  # hipDeviceAttributeMultiprocessorCount
 
 # shape: solve block
 SHAPES = {(20, 17, 60): 128, (50, 100, 50): 256, (72, 144, 72): 384, (88, 176, 88): 512, (96, 192, 96): 576,
@@ -14,9 +18,10 @@ SHAPES = {(20, 17, 60): 128, (50, 100, 50): 256, (72, 144, 72): 384, (88, 176, 8
 
 @pytest.mark.parametrize("shape", list(SHAPES), ids=str)
 def test_handles_that_fit(shape):
-    import torch
     import top3d_xl_amd as t3x
-    slots = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    cus = C.c_int()
+    assert t3x.load_library().hipDeviceGetAttribute(C.byref(cus), MULTIPROCESSOR_COUNT, 0) == 0
+    slots = 4 * cus.value
     groups = SHAPES[shape] // 4
     fit = 1_000_000 // -(-1_000_000 * groups // slots)  # shares are whole parts per million
     print(f"\n[gpu-coarse-share] {shape}: {fit} handles", flush=True)
