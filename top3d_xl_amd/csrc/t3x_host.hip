@@ -1084,10 +1084,12 @@ int pcg_elastic(t3x_problem& P, const double* b, double* y, double tol, int maxI
   // With params.graphs (and no kernel-group timing) the iteration is captured
   // once per solution vector and replayed: every kernel reads its scalars and
   // the convergence flag from device memory, so the same graph serves every
-  // iteration.  Measured on MI355X it neither gains nor loses (0.27 ms per
-  // PCG iteration at 32x64x32, 1.44 ms at 128x256x128, either way): the
-  // kernels' own dispatch latency, not host launch cost, bounds small
-  // problems, so it is off by default.
+  // iteration.  Off by default: it gains next to nothing and costs each handle
+  // 130 to 700 us of capture and instantiation.  us per PCG iteration, launched
+  // / replayed: FP64 12x24x12 58.6 / 57.9, 32x64x32 76.9 / 77.7, 50x100x50 113 /
+  // 119, 96x192x96 366 / 370; precision form 122 / 113, 134 / 131, 184 / 189, 538
+  // / 542.  The kernels' own dispatch latency, not the host's launches, bounds
+  // small problems.
   hipGraphExec_t graph = nullptr;
   if (P.P.graphs && !P.P.timing) {
     for (auto& g : P.pcgGraphs)
