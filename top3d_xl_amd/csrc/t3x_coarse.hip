@@ -1171,6 +1171,9 @@ static auto chain_form(int SB) {
 // such group that is not resident yet.  (Counted by their own occupancy, groups of
 // 96 and of 128 registers could keep each other out, both launches incomplete: two
 // of the one and two of the other leave 64 registers on a SIMD.)
+// Above SB 1024 a group has 176 registers and counts as half a CU: it may have to
+// wait for the others' launches to end, but no mix of a CU whose shares are below
+// one refuses a quarter, so those do end.
 long long CoarseSolver::chain_share() const {
   constexpr long long kNever = 2000000;
   constexpr int kGroupsPerCU = 4;
