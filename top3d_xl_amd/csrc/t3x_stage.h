@@ -7,10 +7,12 @@
 // through the ring, a chunk's memcpy beside the chunks on the link.  A chunk is
 // moved by a kernel that reads or writes the pinned memory itself: the copy
 // engine with an event per chunk leaves the link idle between chunks (15 MB
-// down 716 us against 517, up 724 against 444, one thread).  Large copies are shared by
-// threads: the memcpy out of memory that the device has written runs at
-// 26 GB/s per thread, and result arrays are often fresh pages, whose faults
-// (0.28 ms per MB in 4 KB pages, 0.1 in huge ones) are the memcpy's.
+// down 716 us against 517, up 724 against 444, one thread).  Large copies are
+// shared by threads: the memcpy out of memory that the device has written runs
+// at 26 GB/s per thread, and result arrays are often fresh pages, whose faults
+// (0.28 ms per MB in 4 KB pages, 0.1 in huge ones) are the memcpy's.  What the
+// ring gains least in is 6 to 20 MB up with nothing else between (11.7 MB 413 us,
+// 372 by the runtime; 422 and 518 with an operator application between).
 #pragma once
 
 #include <hip/hip_runtime.h>

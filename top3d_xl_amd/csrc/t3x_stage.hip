@@ -36,10 +36,11 @@ __global__ __launch_bounds__(256) void k_stage_copy(const char* __restrict__ src
     for (unsigned j = i; j < n; ++j) dst[j] = src[j];
 }
 
-// Rings that no object holds, for the next one that asks.  A ring is worth more
-// than most copies gain by it (0.1 ms to make, 0.28 a megabyte for the first touch
-// of its pages, 0.3 to free): made per handle, they brought creating a 36x60x36
-// model from 3.98 to 5.09 ms and closing it from 4.35 to 4.97; lent, 3.84 and 4.35.
+// Rings that no object holds, for the next one that asks.  A ring costs more than
+// a handle's first copies gain by it (0.1 ms to make, 0.28 a megabyte for the first
+// touch of its pages, 0.3 to free): made per handle, they brought creating a
+// 36x60x36 model from 3.98 to 5.09 ms and closing it from 4.35 to 4.97; lent, 3.84
+// and 4.35.
 // The rings kept are the largest given back, at most kRings of them and kBytes in
 // all, until the process ends.
 class RingPool {
